@@ -1,5 +1,6 @@
 // jk_kernels.hip -- gfx950 kernels of The Joker's likelihood + rejection path.
 //
+//  k_lnl_split             the same for few rows, a row's epochs over many lanes.
 //  k_lnl<L, PHYS, MIXED>   fused per-sample marginal lnL: phase, Kepler solve,
 //                          design column, moments, L x L Cholesky, lnL.  One
 //                          lane per prior sample; the star's epoch arrays are
@@ -12,6 +13,7 @@
 //  k_uniform               the raw uniforms (tests / callers).
 //  k_linear_posterior      a = G^-1 rhs and G^-1 for accepted rows (one wave
 //                          per row for diagonal-covariance stars).
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -48,10 +50,11 @@ __device__ double2 g_sincos_tab[JK_TAB_N + 1];
 __device__ float2 g_sincos_tab32[JK_TAB_N + 1];
 // (R_i, -ln R_i) of jk_log_tab.
 __device__ double2 g_log_tab[JK_LOG_TAB_N];
-// LDS image: the FP64 table, then the FP32 table packed two per double2 slot,
-// then the log table.
-#define JK_TAB_LOG_OFF (JK_TAB_N + 1 + (JK_TAB_N + 2) / 2)
-#define JK_TAB_LDS (JK_TAB_LOG_OFF + JK_LOG_TAB_N)
+// LDS image: the FP64 table, the log table, then (kernels with mixed-precision
+// rows only) the FP32 table packed two per double2 slot.
+#define JK_TAB_LOG_OFF (JK_TAB_N + 1)
+#define JK_TAB_LDS64 (JK_TAB_LOG_OFF + JK_LOG_TAB_N)
+#define JK_TAB_LDS (JK_TAB_LDS64 + (JK_TAB_N + 2) / 2)
 
 // Minimum waves per SIMD asked of the row kernels that evaluate many stars
 // or scattered rows: 4 (at most 128 VGPRs) for L <= 3, where the allocator
@@ -59,12 +62,14 @@ __device__ double2 g_log_tab[JK_LOG_TAB_N];
 // spilling at 128; none for larger L, which would spill.
 #define JK_ROW_WAVES(L) ((L) <= 3 ? 4 : 1)
 
+// F32: with the FP32 grid of the mixed-precision row.
+template <bool F32>
 __device__ __forceinline__ void jk_stage_tab(double2 *s_tab)
 {
-    float2 *t32 = reinterpret_cast<float2 *>(s_tab + JK_TAB_N + 1);
+    float2 *t32 = reinterpret_cast<float2 *>(s_tab + JK_TAB_LDS64);
     for (int i = threadIdx.x; i <= JK_TAB_N; i += blockDim.x) {
         s_tab[i] = g_sincos_tab[i];
-        t32[i] = g_sincos_tab32[i];
+        if constexpr (F32) t32[i] = g_sincos_tab32[i];
     }
     for (int i = threadIdx.x; i < JK_LOG_TAB_N; i += blockDim.x)
         s_tab[JK_TAB_LOG_OFF + i] = g_log_tab[i];
@@ -119,7 +124,7 @@ __device__ __forceinline__ void jk_sincos_tab(float Ef, const double2 *__restric
 __device__ __forceinline__ void jk_sincos_tab_f32(float E, const double2 *__restrict__ tab,
                                                   float &s, float &c)
 {
-    const float2 *__restrict__ t32 = reinterpret_cast<const float2 *>(tab + JK_TAB_N + 1);
+    const float2 *__restrict__ t32 = reinterpret_cast<const float2 *>(tab + JK_TAB_LDS64);
     int idx = (int)(E * JK_TAB_INV_H_F);
     idx = min(max(idx, 0), JK_TAB_N);
     const float2 t = t32[idx];
@@ -311,24 +316,29 @@ __device__ __forceinline__ void jk_kepler_markley_f32(float x, float e, float om
 // value, a positive bound a mixed-precision value.
 #define JK_BOUND_UPPER (-1.0f)
 
-// With ONE the first trend column is the constant 1 (StarDev::t0_one): its
-// products fold away, with the same roundings (w * 1 = w exactly).
-template <int L, bool PHYS, bool MIXED, bool SAFE = false, bool BOUND = false, bool ONE = false>
-__device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
+// One prior row's orbit: what every epoch of it shares.
+struct RowOrbit {
+    double e, invP, nP, M0, M0t, s2, lam0, cw, ecw, swsq, dmax;
+    // FP32 copies for the Kepler starter (e capped below 1 in FP32; 1 - e
+    // rounded from its FP64 value, so it keeps its relative accuracy) and for
+    // the mixed row's design value, which is combined in FP32.
+    float ef, omef, a1f, cwf, swsqf, ecwf;
+};
+
+// Reads row r's columns and derives its orbit; false for an invalid row
+// (its lnL is NaN).  Both precisions read the FP64 columns: the kernels are
+// bound by arithmetic, not by the prior stream, and an FP32 copy of e would
+// carry a relative error of up to 2^-24 / (1 - e) into sqrt(1 - e^2), the
+// scale of the whole design column as e -> 1.
+template <bool PHYS>
+__device__ __forceinline__ bool jk_row_orbit(const StarDev &st, int64_t r,
                                              const double *__restrict__ P,
                                              const void *__restrict__ e_,
                                              const void *__restrict__ om_,
                                              const void *__restrict__ M0_,
                                              const void *__restrict__ s_,
-                                             const double2 *__restrict__ tab,
-                                             float *bnd = nullptr)
+                                             const double2 *__restrict__ tab, RowOrbit &o)
 {
-    static_assert(!BOUND || MIXED, "the error bound belongs to the mixed-precision row");
-    if constexpr (BOUND) *bnd = INFINITY;
-    // Both precisions read the FP64 columns: the kernels are bound by
-    // arithmetic, not by the prior stream, and an FP32 copy of e would carry
-    // a relative error of up to 2^-24 / (1 - e) into sqrt(1 - e^2), the scale
-    // of the whole design column as e -> 1.
     const double *__restrict__ ecol = static_cast<const double *>(e_);
     const double *__restrict__ omcol = static_cast<const double *>(om_);
     const double *__restrict__ M0col = static_cast<const double *>(M0_);
@@ -343,35 +353,178 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
     bool valid = isfinite(Pv) && Pv != 0.0 && ev >= 0.0 && ev < 1.0 && isfinite(omv) &&
                  isfinite(M0v);
     if (PHYS) valid = valid && isfinite(sv);
-    if (!valid) return __builtin_nan("");
+    if (!valid) return false;
 
-    double lam0;
     if (st.k_prior_mode == JK_KPRIOR_FIXED_COMPANION_MASS)
-        lam0 = jk_k_variance(&st, Pv, ev, true);
+        o.lam0 = jk_k_variance(&st, Pv, ev, true);
     else
-        lam0 = st.lam0;
+        o.lam0 = st.lam0;
 
-    const double invP = jk_rcp2(Pv);
-    const double nP = JK_TWO_PI * invP;
-    const double M0t = M0v * JK_INV_TWO_PI;
-    const double s2 = sv * sv;
-
-    // Per-sample orbit constants.
-    double cw, ecw, swsq;
-    // FP32 copies for the Kepler starter (e capped below 1 in FP32; 1 - e
-    // rounded from its FP64 value, so it keeps its relative accuracy).
-    const float ef = fminf((float)ev, 0.99999994f);
-    const float omef = fmaxf((float)(1.0 - ev), 5.9604645e-08f);
-    const float a1f = JK_MARKLEY_A1N * __builtin_amdgcn_rcpf(1.0f + ef);
+    o.e = ev;
+    o.invP = jk_rcp2(Pv);
+    o.nP = JK_TWO_PI * o.invP;
+    o.M0 = M0v;
+    o.M0t = M0v * JK_INV_TWO_PI;
+    o.s2 = sv * sv;
+    o.ef = fminf((float)ev, 0.99999994f);
+    o.omef = fmaxf((float)(1.0 - ev), 5.9604645e-08f);
+    o.a1f = JK_MARKLEY_A1N * __builtin_amdgcn_rcpf(1.0f + o.ef);
     double sw;
-    jk_sincos_tab_f64(omv, tab, sw, cw);
-    ecw = ev * cw;
-    swsq = sw * sqrt((1.0 - ev) * (1.0 + ev));
-    // FP32 copies for the mixed row's design value, which is combined in FP32
-    const float cwf = (float)cw, swsqf = (float)swsq, ecwf = (float)ecw;
+    jk_sincos_tab_f64(omv, tab, sw, o.cw);
+    o.ecw = ev * o.cw;
+    o.swsq = sw * sqrt((1.0 - ev) * (1.0 + ev));
+    o.cwf = (float)o.cw;
+    o.swsqf = (float)o.swsq;
+    o.ecwf = (float)o.ecw;
     // The FP32 starter sees e rounded to FP32; within 1e-7 of 1 that can put
     // it outside the correction's reach, so such samples take the fallback.
-    const double dmax = ev > 0.9999999 ? -1.0 : 1e-3;
+    o.dmax = ev > 0.9999999 ? -1.0 : 1e-3;
+    return true;
+}
+
+// The design value of an epoch at dt and, with PHYS, its weight from the
+// epoch's variance vk = sigma^2 + s^2.  MIXED: denb = 1 / (1 - e cos E) for
+// the error bound.  FP64 (not SAFE): bad is set where the row needs the
+// bracketed Newton iteration.
+template <bool PHYS, bool MIXED, bool SAFE>
+__device__ __forceinline__ double jk_row_epoch(const RowOrbit &o, double dtk, double vk,
+                                               const double2 *__restrict__ tab, double &w,
+                                               float &denb, bool &bad)
+{
+    double x;
+    if constexpr (MIXED) {
+        // the FP32 Kepler step reads x rounded to FP32: the low part of
+        // 2 pi (k * 2.4e-16 rad) is far below that rounding
+        const double ph = fma(o.nP, dtk, -o.M0);
+        x = fma(-rint(ph * JK_INV_TWO_PI), JK_TWO_PI_HI, ph);
+    } else {
+        // the phase in turns, dt / P - M0 / (2 pi), one rounding; its
+        // fractional part is exact (Sterbenz) and scales to radians with
+        // one more
+        const double pt = fma(o.invP, dtk, -o.M0t);
+        x = (pt - rint(pt)) * JK_TWO_PI;
+    }
+    double m;
+    if constexpr (MIXED) {
+        float sE, cE;
+        jk_kepler_markley_f32((float)x, o.ef, o.omef, o.a1f, tab, sE, cE);
+        const float den = __builtin_amdgcn_rcpf(fmaf(-o.ef, cE, 1.0f));
+        // the design value combined in FP32 too (an FP32 instruction
+        // issues in half the cycles of an FP64 one): its rounding stays
+        // inside the per-epoch error model of the bound
+        m = (double)fmaf(fmaf(o.cwf, cE - o.ef, -o.swsqf * sE), den, o.ecwf);
+        denb = den;
+        // the FP32 reciprocal (relative error below 2^-22, which the bound
+        // covers)
+        if constexpr (PHYS) w = (double)__builtin_amdgcn_rcpf((float)vk);
+    } else {
+        double sE, cE;
+        if constexpr (SAFE) {
+            jk_kepler_poly_f64(x, o.e, tab, sE, cE);
+            if constexpr (PHYS) w = jk_rcp1(vk);
+        } else if constexpr (PHYS) {
+            // w = 1 / (sigma^2 + s^2) to a relative 2.5e-15 (one Newton step
+            // on the hardware reciprocal, shared with the Kepler step's)
+            bad |= !jk_kepler_markley_f64<true>(x, o.e, o.ef, o.omef, o.a1f, o.dmax, tab, sE, cE,
+                                                vk, &w);
+        } else {
+            bad |= !jk_kepler_markley_f64(x, o.e, o.ef, o.omef, o.a1f, o.dmax, tab, sE, cE);
+        }
+        // m = [cos w (cos E - e) - sin w sqrt(1-e^2) sin E] / (1 - e cos E) + e cos w
+        // (one Newton step on the hardware reciprocal: relative 2e-15)
+        const double den = jk_rcp1(fma(-o.e, cE, 1.0));
+        m = fma(fma(o.cw, cE - o.e, -o.swsq * sE), den, o.ecw);
+    }
+    return m;
+}
+
+// The row's lnL from its sums over the epochs (PHYS: those of the trend
+// columns too, and the product prod 2^pexp of the variances; otherwise they
+// are star constants).  BOUND: with its error bound, from sum w and the
+// largest 1 / (1 - e cos E).
+template <int L, bool PHYS, bool BOUND>
+__device__ __forceinline__ double jk_row_finish(const StarDev &st, double lam0,
+                                                double Smm, double Smr, double Srr,
+                                                const double *Smt, const double *Str,
+                                                const double *Stt, double prod, int pexp,
+                                                double Sw, float dmx,
+                                                const double2 *__restrict__ tab, float *bnd)
+{
+    constexpr int LT = L > 1 ? L - 1 : 1;
+    // Assemble G (lower triangle used), u, chi0, log-constant.
+    double G[L * L], u[L];
+    const double mu0 = st.mu0;
+    const bool fcm = st.k_prior_mode == JK_KPRIOR_FIXED_COMPANION_MASS;
+    G[0] = (fcm ? jk_rcp2(lam0) : st.lam_inv[0]) + Smm;
+    u[0] = fma(-mu0, Smm, Smr);
+    // log-constant: st.ln_c / ln_c_phys hold everything but the sample's
+    // product prod(sigma_n^2 + s^2) = prod * 2^pexp and, for FixedCompanionMass,
+    // ln lam0
+    double chi0, lnc, scale = 1.0;
+    if constexpr (PHYS) {
+        chi0 = Srr;
+        lnc = st.ln_c_phys + (double)pexp * JK_LN2;
+        scale = prod;
+    } else {
+        chi0 = st.S_rr;
+        lnc = st.ln_c;
+    }
+    if (fcm) scale *= lam0;
+    chi0 = fma(mu0 * mu0, Smm, fma(-2.0 * mu0, Smr, chi0));
+    if constexpr (L > 1) {
+#pragma unroll
+        for (int j = 1; j < L; ++j) {
+            G[j * L] = Smt[j - 1];
+            G[j] = Smt[j - 1];
+            const double trj = PHYS ? Str[j - 1] : st.S_tr[j - 1];
+            u[j] = fma(-mu0, Smt[j - 1], trj);
+#pragma unroll
+            for (int q = 1; q <= j; ++q) {
+                const double tt =
+                    PHYS ? Stt[(j - 1) * LT + (q - 1)] : st.S_tt[(j - 1) * JK_LMAX + (q - 1)];
+                const double g = (q == j ? st.lam_inv[j] : 0.0) + tt;
+                G[j * L + q] = g;
+                G[q * L + j] = g;
+            }
+        }
+    }
+    if constexpr (BOUND) {
+        double post[3];
+        const double ll = jk_finish_lnl<L, true>(G, u, chi0, lnc, scale, tab + JK_TAB_LOG_OFF, post);
+        const double aK = fabs(mu0 + post[1]);
+        const double t1 = 1.0 + (double)dmx;
+        const double ek = t1 * t1 * fma(1e-3, (double)dmx, 1.0);
+        double b = 2.0 * JK_BOUND_EPS * ek * sqrt(Sw) *
+                   fma(aK, sqrt(fmax(post[2], 0.0)), sqrt(fmax(post[0], 0.0)));
+        // the weights' relative error e_w moves lnL by at most
+        // e_w (chi2_min + L) / 2 (envelope theorem on chi2_min; the log-det
+        // term is tr(G^-1 X^T W X) e_w <= L e_w); e_w < 2^-22 for the FP32
+        // reciprocal of the physical jitter mode, 2.4e-15 otherwise
+        b += (PHYS ? JK_BOUND_EPS : 2e-15) * (fmax(post[2], 0.0) + (double)L);
+        b = fma(1e-9, 1.0 + fabs(ll), b) * 1.000001;
+        *bnd = (isfinite(b) && isfinite(ll)) ? (float)b : INFINITY;
+        return ll;
+    } else {
+        return jk_finish_lnl<L>(G, u, chi0, lnc, scale, tab + JK_TAB_LOG_OFF);
+    }
+}
+
+// With ONE the first trend column is the constant 1 (StarDev::t0_one): its
+// products fold away, with the same roundings (w * 1 = w exactly).
+template <int L, bool PHYS, bool MIXED, bool SAFE = false, bool BOUND = false, bool ONE = false>
+__device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
+                                             const double *__restrict__ P,
+                                             const void *__restrict__ e_,
+                                             const void *__restrict__ om_,
+                                             const void *__restrict__ M0_,
+                                             const void *__restrict__ s_,
+                                             const double2 *__restrict__ tab,
+                                             float *bnd = nullptr)
+{
+    static_assert(!BOUND || MIXED, "the error bound belongs to the mixed-precision row");
+    if constexpr (BOUND) *bnd = INFINITY;
+    RowOrbit o;
+    if (!jk_row_orbit<PHYS>(st, r, P, e_, om_, M0_, s_, tab, o)) return __builtin_nan("");
 
     constexpr int LT = L > 1 ? L - 1 : 1;
     double Smm = 0.0, Smr = 0.0;
@@ -393,60 +546,17 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
     float dmx = 0.0f;      // largest 1 / (1 - e cos E) (BOUND only)
 #pragma unroll 2
     for (int k = 0; k < N; ++k) {
-        const double dtk = st.dt[k];
-        double x;
-        if constexpr (MIXED) {
-            // the FP32 Kepler step reads x rounded to FP32: the low part of
-            // 2 pi (k * 2.4e-16 rad) is far below that rounding
-            const double ph = fma(nP, dtk, -M0v);
-            x = fma(-rint(ph * JK_INV_TWO_PI), JK_TWO_PI_HI, ph);
-        } else {
-            // the phase in turns, dt / P - M0 / (2 pi), one rounding; its
-            // fractional part is exact (Sterbenz) and scales to radians with
-            // one more
-            const double pt = fma(invP, dtk, -M0t);
-            x = (pt - rint(pt)) * JK_TWO_PI;
-        }
+        const double vk = PHYS ? st.sig2[k] + o.s2 : 0.0;
         double w = 0.0;
-        const double vk = PHYS ? st.sig2[k] + s2 : 0.0;
-        double m;
         float denb = 0.0f;
-        if constexpr (MIXED) {
-            float sE, cE;
-            jk_kepler_markley_f32((float)x, ef, omef, a1f, tab, sE, cE);
-            const float den = __builtin_amdgcn_rcpf(fmaf(-ef, cE, 1.0f));
-            // the design value combined in FP32 too (an FP32 instruction
-            // issues in half the cycles of an FP64 one): its rounding stays
-            // inside the per-epoch error model of the bound
-            m = (double)fmaf(fmaf(cwf, cE - ef, -swsqf * sE), den, ecwf);
-            denb = den;
-        } else {
-            double sE, cE;
-            if constexpr (SAFE) {
-                jk_kepler_poly_f64(x, ev, tab, sE, cE);
-                if constexpr (PHYS) w = jk_rcp1(vk);
-            } else if constexpr (PHYS) {
-                bad |= !jk_kepler_markley_f64<true>(x, ev, ef, omef, a1f, dmax, tab, sE, cE,
-                                                    vk, &w);
-            } else {
-                bad |= !jk_kepler_markley_f64(x, ev, ef, omef, a1f, dmax, tab, sE, cE);
-            }
-            // m = [cos w (cos E - e) - sin w sqrt(1-e^2) sin E] / (1 - e cos E) + e cos w
-            // (one Newton step on the hardware reciprocal: relative 2e-15)
-            const double den = jk_rcp1(fma(-ev, cE, 1.0));
-            m = fma(fma(cw, cE - ev, -swsq * sE), den, ecw);
-        }
+        const double m = jk_row_epoch<PHYS, MIXED, SAFE>(o, st.dt[k], vk, tab, w, denb, bad);
         const double rp = st.rp[k];
         if constexpr (PHYS) {
-            // w = 1 / (sigma^2 + s^2): FP64 to a relative 2.5e-15 (one Newton
-            // step on the hardware reciprocal, shared with the Kepler step's),
-            // or in the mixed row the FP32 reciprocal (relative error below
-            // 2^-22, which the bound covers); sum ln w = -ln of the running
-            // product of the FP64 variances, renormalised every fourth epoch
-            // (frexp scales by a power of two, exactly, so the product's
-            // rounding is that of renormalising every epoch; four factors
-            // stay far inside the exponent range)
-            if constexpr (MIXED) w = (double)__builtin_amdgcn_rcpf((float)vk);
+            // sum ln w = -ln of the running product of the FP64 variances,
+            // renormalised every fourth epoch (frexp scales by a power of
+            // two, exactly, so the product's rounding is that of
+            // renormalising every epoch; four factors stay far inside the
+            // exponent range)
             prod *= vk;
             if ((k & 3) == 3) {
                 int ex;
@@ -484,62 +594,232 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
     if constexpr (!MIXED && !SAFE) {
         if (bad) return jk_lnl_row<L, PHYS, false, true>(st, r, P, e_, om_, M0_, s_, tab);
     }
+    return jk_row_finish<L, PHYS, BOUND>(st, o.lam0, Smm, Smr, Srr, Smt, Str, Stt, prod, pexp,
+                                         Sw, dmx, tab, bnd);
+}
 
-    // Assemble G (lower triangle used), u, chi0, log-constant.
-    double G[L * L], u[L];
-    const double mu0 = st.mu0;
-    const bool fcm = st.k_prior_mode == JK_KPRIOR_FIXED_COMPANION_MASS;
-    G[0] = (fcm ? jk_rcp2(lam0) : st.lam_inv[0]) + Smm;
-    u[0] = fma(-mu0, Smm, Smr);
-    // log-constant: st.ln_c / ln_c_phys hold everything but the sample's
-    // product prod(sigma_n^2 + s^2) = prod * 2^pexp and, for FixedCompanionMass,
-    // ln lam0
-    double chi0, lnc, scale = 1.0;
-    if constexpr (PHYS) {
-        chi0 = Srr;
-        lnc = st.ln_c_phys + (double)pexp * JK_LN2;
-        scale = prod;
-    } else {
-        chi0 = st.S_rr;
-        lnc = st.ln_c;
+// ---------------------------------------------------------------------------
+// Few rows: a workgroup of 4 waves takes R <= 64 rows.  With one lane per row,
+// n rows are n / 64 waves, and below 4096 of them (4 per SIMD) the device
+// idles while each lane walks its epochs alone; its Kepler solves, which do
+// not depend on one another, are nearly all of that work.  So three waves
+// evaluate (row, epoch) pairs, G = 192 / R lanes to a row, and leave each
+// pair's design value m and weight w in LDS, a chunk of epochs at a time; the
+// fourth, one lane per row, adds the chunk before to the rows' sums, epoch
+// after epoch, meanwhile (two buffers, one barrier per chunk).  Each sum
+// therefore rounds exactly as in jk_lnl_row, and the row's lnL (and bound) is
+// the same bits however it is evaluated.  A row that needs the bracketed
+// Newton iteration is evaluated again by jk_lnl_row's own fallback.
+// Tried first: one lane per (row, sum) adding up (three LDS reads per sum and
+// epoch made LDS the bound), and every wave evaluating with a barrier around
+// one wave's adding (the other three idle meanwhile).
+// ---------------------------------------------------------------------------
+#define JK_SPLIT_PAIRS 512
+
+template <int L, bool PHYS, bool MIXED>
+struct SplitLds {
+    // an epoch's record: r', sigma^2 or ivar, T, dt; the epochs of a chunk at
+    // most (one value of the next chunk per evaluating lane)
+    static constexpr int NEP = L + 2, CMAX = 192 / NEP;
+    struct Chunk {
+        double m[JK_SPLIT_PAIRS];
+        double w[PHYS ? JK_SPLIT_PAIRS : 1];
+    } chunk[2];
+    double ep[3][CMAX * NEP];      // the chunk added up, the one evaluated, the next
+    float dmx[MIXED ? 192 : 1];
+    int bad[64];
+};
+
+// A lane's number in the split: the workgroup's lanes counted from wave sw,
+// the one that adds up (another wave in each workgroup, so that the SIMDs of
+// a compute unit share that work).  Lanes 0 .. 63 add up, lane l row l; lane
+// 64 + q evaluates epochs of row q mod R.
+__device__ __forceinline__ int jk_split_lane(int sw)
+{
+    return ((int)threadIdx.x - 64 * sw) & 255;
+}
+
+// The adding wave of workgroup b.  Workgroups go round the 8 XCDs, and within
+// one round its 32 compute units: those that share a compute unit differ in
+// b / 256.
+__device__ __forceinline__ int jk_split_wave(unsigned b)
+{
+    return (int)((b >> 3) + (b >> 8)) & 3;
+}
+
+__device__ __forceinline__ int jk_split_row(int lane, int R)
+{
+    return lane < 64 ? lane : (lane - 64) % R;
+}
+
+// Every lane of the workgroup calls this with the same star, R and sw; r: the
+// cache row of the lane's row (jk_split_row), -1 for none.  The result is
+// that of the lanes whose number is below R.
+template <int L, bool PHYS, bool MIXED>
+__device__ __forceinline__ double jk_rows_split(const StarDev &st, int R, int sw, int64_t r,
+                                                const double *__restrict__ P,
+                                                const void *__restrict__ e_,
+                                                const void *__restrict__ om_,
+                                                const void *__restrict__ M0_,
+                                                const void *__restrict__ s_,
+                                                const double2 *__restrict__ tab,
+                                                SplitLds<L, PHYS, MIXED> &sh, float *bnd)
+{
+    typedef SplitLds<L, PHYS, MIXED> Sh;
+    const int lane = jk_split_lane(sw), G = 192 / R, N = st.n;
+    int C = min(JK_SPLIT_PAIRS / R, Sh::CMAX);      // whole rounds of the lanes, if any fit
+    C = C >= 2 * G ? C / (2 * G) * (2 * G) : (C >= G ? G : C);
+    const int row = jk_split_row(lane, R), g = (lane - 64) / R;
+    RowOrbit o;
+    const bool valid = r >= 0 && jk_row_orbit<PHYS>(st, r, P, e_, om_, M0_, s_, tab, o);
+    const bool sums = lane < 64;      // wave-uniform
+    constexpr int LT = L > 1 ? L - 1 : 1;
+    double Smm = 0.0, Smr = 0.0, Srr = 0.0, Sw = 0.0, prod = 1.0;
+    double Smt[LT], Str[LT], Stt[LT * LT];
+    int pexp = 0;
+#pragma unroll
+    for (int j = 0; j < LT; ++j) {
+        Smt[j] = 0.0;
+        Str[j] = 0.0;
+#pragma unroll
+        for (int k = 0; k < LT; ++k) Stt[j * LT + k] = 0.0;
     }
-    if (fcm) scale *= lam0;
-    chi0 = fma(mu0 * mu0, Smm, fma(-2.0 * mu0, Smr, chi0));
-    if constexpr (L > 1) {
-#pragma unroll
-        for (int j = 1; j < L; ++j) {
-            G[j * L] = Smt[j - 1];
-            G[j] = Smt[j - 1];
-            const double trj = PHYS ? Str[j - 1] : st.S_tr[j - 1];
-            u[j] = fma(-mu0, Smt[j - 1], trj);
-#pragma unroll
-            for (int q = 1; q <= j; ++q) {
-                const double tt = PHYS ? Stt[(j - 1) * LT + (q - 1)] : st.S_tt[(j - 1) * JK_LMAX + (q - 1)];
-                const double g = (q == j ? st.lam_inv[j] : 0.0) + tt;
-                G[j * L + q] = g;
-                G[q * L + j] = g;
+    __syncthreads();   // the workgroup's previous rows are done with sh
+    if (sums) sh.bad[lane] = 0;
+    bool bad = false;
+    float dmx = 0.0f;
+    const int nch = (N + C - 1) / C;
+    // evaluating lane 64 + q brings in value q of each chunk's records, a chunk
+    // ahead of its use
+    const int ev = (lane - 64) / C, ek = lane - 64 - ev * C;
+    const double *esrc = nullptr;
+    if (!sums && ev < Sh::NEP)
+        esrc = (ev == 0 ? st.rp
+                        : (ev == 1 ? (PHYS ? st.sig2 : st.ivar)
+                                   : (ev == L + 1 ? st.dt : st.T + (size_t)(ev - 2) * N))) + ek;
+    double enext = esrc && ek < N ? *esrc : 0.0;
+    if (esrc) sh.ep[0][ek * Sh::NEP + ev] = enext;
+    __syncthreads();
+    for (int c = 0; c <= nch; ++c) {
+        if (!sums && c < nch) {
+            typename Sh::Chunk &ck = sh.chunk[c & 1];
+            const int c0 = c * C, cnt = min(C, N - c0);
+            if (esrc && c0 + C + ek < N) enext = esrc[c0 + C];
+            if (valid && g < G) {
+                const double *rec = sh.ep[c % 3];
+                // two epochs at a time, both solved before either is stored:
+                // the LDS stores would keep the second solve behind the first
+                for (int kk = g; kk < cnt; kk += 2 * G) {
+                    const bool two = kk + G < cnt;
+                    const int k2 = two ? kk + G : kk;
+                    const double d1 = rec[kk * Sh::NEP + L + 1], d2 = rec[k2 * Sh::NEP + L + 1];
+                    const double v1 = PHYS ? rec[kk * Sh::NEP + 1] + o.s2 : 0.0;
+                    const double v2 = PHYS ? rec[k2 * Sh::NEP + 1] + o.s2 : 0.0;
+                    double w1 = 0.0, w2 = 0.0, m1, m2 = 0.0;
+                    float b1 = 0.0f, b2 = 0.0f;
+                    if (__any(two)) {
+                        m1 = jk_row_epoch<PHYS, MIXED, false>(o, d1, v1, tab, w1, b1, bad);
+                        m2 = jk_row_epoch<PHYS, MIXED, false>(o, d2, v2, tab, w2, b2, bad);
+                    } else {
+                        m1 = jk_row_epoch<PHYS, MIXED, false>(o, d1, v1, tab, w1, b1, bad);
+                    }
+                    ck.m[kk * R + row] = m1;
+                    if constexpr (PHYS) ck.w[kk * R + row] = w1;
+                    if (two) {
+                        ck.m[k2 * R + row] = m2;
+                        if constexpr (PHYS) ck.w[k2 * R + row] = w2;
+                    }
+                    if constexpr (MIXED) dmx = fmaxf(dmx, fmaxf(b1, b2));
+                }
             }
         }
+        if (sums && c > 0 && lane < R) {
+            const typename Sh::Chunk &ck = sh.chunk[(c - 1) & 1];
+            const double *rec = sh.ep[(c - 1) % 3];
+            const int c0 = (c - 1) * C, cnt = min(C, N - c0);
+            // the LDS reads of U epochs in flight together
+            constexpr int U = L <= 4 ? 4 : 2;
+            for (int k0 = 0; k0 < cnt; k0 += U) {
+                double em[U], ew[U], er[U][Sh::NEP];
+#pragma unroll
+                for (int j = 0; j < U; ++j) {
+                    const int kk = min(k0 + j, cnt - 1);
+                    em[j] = ck.m[kk * R + row];
+                    ew[j] = PHYS ? ck.w[kk * R + row] : rec[kk * Sh::NEP + 1];
+#pragma unroll
+                    for (int q = 0; q < L + 1; ++q) er[j][q] = rec[kk * Sh::NEP + q];
+                }
+#pragma unroll
+                for (int j = 0; j < U; ++j) {
+                    if (k0 + j >= cnt) break;
+                    const double m = em[j], w = ew[j], rp = er[j][0];
+                    const double *ep = er[j];
+                    if constexpr (PHYS) {
+                        prod *= ep[1] + o.s2;
+                        if (((c0 + k0 + j) & 3) == 3) {
+                            int ex;
+                            prod = frexp(prod, &ex);
+                            pexp += ex;
+                        }
+                    }
+                    if constexpr (MIXED) Sw += w;
+                    const double wm = w * m;
+                    Smm = fma(wm, m, Smm);
+                    Smr = fma(wm, rp, Smr);
+                    if constexpr (L > 1) {
+#pragma unroll
+                        for (int i = 0; i < L - 1; ++i) {
+                            Smt[i] = fma(wm, ep[2 + i], Smt[i]);
+                            if constexpr (PHYS) {
+                                const double wT = w * ep[2 + i];
+                                Str[i] = fma(wT, rp, Str[i]);
+#pragma unroll
+                                for (int q = 0; q <= i; ++q)
+                                    Stt[i * LT + q] = fma(wT, ep[2 + q], Stt[i * LT + q]);
+                            }
+                        }
+                    }
+                    if constexpr (PHYS) Srr = fma(w * rp, rp, Srr);
+                }
+            }
+        }
+        if (esrc && c + 1 < nch) sh.ep[(c + 1) % 3][ek * Sh::NEP + ev] = enext;
+        if (c == nch - 1) {
+            // after the last chunk's pairs: what the adding lanes need of them
+            if (bad) sh.bad[row] = 1;
+            if constexpr (MIXED)
+                if (!sums) sh.dmx[lane - 64] = dmx;
+        }
+        __syncthreads();
     }
-    if constexpr (BOUND) {
-        double post[3];
-        const double ll = jk_finish_lnl<L, true>(G, u, chi0, lnc, scale, tab + JK_TAB_LOG_OFF, post);
-        const double aK = fabs(mu0 + post[1]);
-        const double t1 = 1.0 + (double)dmx;
-        const double ek = t1 * t1 * fma(1e-3, (double)dmx, 1.0);
-        double b = 2.0 * JK_BOUND_EPS * ek * sqrt(Sw) *
-                   fma(aK, sqrt(fmax(post[2], 0.0)), sqrt(fmax(post[0], 0.0)));
-        // the weights' relative error e_w moves lnL by at most
-        // e_w (chi2_min + L) / 2 (envelope theorem on chi2_min; the log-det
-        // term is tr(G^-1 X^T W X) e_w <= L e_w); e_w < 2^-22 for the FP32
-        // reciprocal of the physical jitter mode, 2.4e-15 otherwise
-        b += (PHYS ? JK_BOUND_EPS : 2e-15) * (fmax(post[2], 0.0) + (double)L);
-        b = fma(1e-9, 1.0 + fabs(ll), b) * 1.000001;
-        *bnd = (isfinite(b) && isfinite(ll)) ? (float)b : INFINITY;
-        return ll;
+    if constexpr (MIXED) *bnd = INFINITY;
+    if (!valid || lane >= R) return __builtin_nan("");
+    if constexpr (!MIXED) {
+        if (sh.bad[row]) return jk_lnl_row<L, PHYS, false, true>(st, r, P, e_, om_, M0_, s_, tab);
     } else {
-        return jk_finish_lnl<L>(G, u, chi0, lnc, scale, tab + JK_TAB_LOG_OFF);
+        for (int q = 0; q < G; ++q) dmx = fmaxf(dmx, sh.dmx[q * R + row]);
     }
+    return jk_row_finish<L, PHYS, MIXED>(st, o.lam0, Smm, Smr, Srr, Smt, Str, Stt, prod, pexp, Sw,
+                                         dmx, tab, bnd);
+}
+
+// Rows per workgroup of the split evaluation of n rows of N epochs, or 0 for
+// the launch with one row per lane: R = n / 512 up to 40, then n / 768 up to
+// 64.  Measured on one MI355X, N = 149, L = 3, against one row per lane
+// (about 50 us up to 65536 rows, the time of one wave per SIMD): 22 us at 2048
+// rows, 26 at 8192, 28 at 16384, 37 at 33001 (R = 64 there: 42; n / 1024:
+// 41); at 65536 rows the two are equal, so the line lies below.  Below
+// JK_SPLIT_MIN_EPOCHS there is little to spread (N = 6: no gain).
+#define JK_SPLIT_MAX_ROWS 49152
+#define JK_SPLIT_MIN_EPOCHS 10
+#define JK_SPLIT_RMIN 8
+
+static int jk_split_rows(int64_t n, int N)
+{
+    if (n > JK_SPLIT_MAX_ROWS || N < JK_SPLIT_MIN_EPOCHS) return 0;
+    int R = (int)((n + 511) / 512);
+    if (R > 40) R = (int)((n + 767) / 768);
+    return std::min(std::max(std::max(R, 192 / N), JK_SPLIT_RMIN), 64);
 }
 
 // ---------------------------------------------------------------------------
@@ -733,8 +1013,8 @@ __global__ __launch_bounds__(256) void k_lnl(const StarDev st, int64_t n,
                                              double *__restrict__ blockmax,
                                              float *__restrict__ bound)
 {
-    __shared__ double2 s_tab[JK_TAB_LDS];
-    jk_stage_tab(s_tab);
+    __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
+    jk_stage_tab<MIXED>(s_tab);
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     double vmax = -INFINITY;
@@ -758,6 +1038,42 @@ __global__ __launch_bounds__(256) void k_lnl(const StarDev st, int64_t n,
     }
 }
 
+// The dense launch for few rows (jk_split_rows): blockmax[block] receives the
+// workgroup's maximum.
+template <int L, bool PHYS, bool MIXED>
+__global__ __launch_bounds__(256) void k_lnl_split(const StarDev st, int64_t n, int R,
+                                                   const double *__restrict__ P,
+                                                   const void *__restrict__ e_,
+                                                   const void *__restrict__ om_,
+                                                   const void *__restrict__ M0_,
+                                                   const void *__restrict__ s_,
+                                                   const int64_t *__restrict__ rows,
+                                                   double *__restrict__ ll,
+                                                   double *__restrict__ blockmax,
+                                                   float *__restrict__ bound)
+{
+    __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
+    __shared__ SplitLds<L, PHYS, MIXED> sh;
+    jk_stage_tab<MIXED>(s_tab);
+    const int sw = jk_split_wave(blockIdx.x), lane = jk_split_lane(sw);
+    const int row = jk_split_row(lane, R);
+    const int64_t i = (int64_t)blockIdx.x * R + row;
+    const int64_t r = row < R && i < n ? (rows ? rows[i] : i) : -1;
+    float b = 0.0f;
+    const double v =
+        jk_rows_split<L, PHYS, MIXED>(st, R, sw, r, P, e_, om_, M0_, s_, s_tab, sh, &b);
+    if (lane >= 64) return;
+    const bool mine = lane < R && i < n;
+    if (mine) {
+        ll[i] = v;
+        if (MIXED && bound) bound[i] = b;
+    }
+    if (blockmax) {
+        const double vmax = wave_nanmax(mine ? v : -INFINITY);
+        if ((threadIdx.x & 63) == 0) blockmax[blockIdx.x] = vmax;
+    }
+}
+
 // Full-covariance stars, FP64: one lane per row, 64 lanes per workgroup, the
 // design columns in dynamic LDS (N x 64 doubles).
 template <int L, bool PHYS>
@@ -770,9 +1086,9 @@ __global__ __launch_bounds__(JK_COV_LANES) void k_lnl_cov(const StarDev st, int6
                                                           const int64_t *__restrict__ rows,
                                                           double *__restrict__ ll)
 {
-    __shared__ double2 s_tab[JK_TAB_LDS];
+    __shared__ double2 s_tab[JK_TAB_LDS64];
     extern __shared__ double s_m[];
-    jk_stage_tab(s_tab);
+    jk_stage_tab<false>(s_tab);
     const int64_t i = (int64_t)blockIdx.x * JK_COV_LANES + threadIdx.x;
     if (i < n) {
         const int64_t r = rows ? rows[i] : i;
@@ -833,8 +1149,8 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_scatter_f64(const 
                                                          const int64_t *__restrict__ rows,
                                                          double *__restrict__ ll)
 {
-    __shared__ double2 s_tab[JK_TAB_LDS];
-    jk_stage_tab(s_tab);
+    __shared__ double2 s_tab[JK_TAB_LDS64];
+    jk_stage_tab<false>(s_tab);
     const int64_t cnt = *count;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < cnt; j += stride) {
@@ -844,12 +1160,19 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_scatter_f64(const 
     }
 }
 
-// Workgroups of a dense launch over n rows: one row per lane up to 16384
+// Workgroups of a dense launch over n rows, one row per lane: up to 16384
 // workgroups (2^22 rows), then a stride.
 static int64_t jk_dense_blocks(int64_t n)
 {
     const int64_t b = (n + 255) / 256;
     return b < 16384 ? (b < 1 ? 1 : b) : 16384;
+}
+
+// Entries of blockmax the launch over n rows of an N-epoch star writes.
+static int64_t jk_lnl_partials(int64_t n, int N)
+{
+    const int R = jk_split_rows(n, N);
+    return R ? (n + R - 1) / R : 4 * jk_dense_blocks(n);
 }
 
 template <int L, bool PHYS, bool MIXED>
@@ -858,6 +1181,12 @@ static hipError_t launch_lnl_t(const jk_star *st, int64_t n, const double *P, co
                                const int64_t *rows, double *ll, double *blockmax, float *bound,
                                hipStream_t stream)
 {
+    if (const int R = jk_split_rows(n, st->dev.n)) {
+        hipLaunchKernelGGL((k_lnl_split<L, PHYS, MIXED>), dim3((unsigned)((n + R - 1) / R)),
+                           dim3(256), 0, stream, st->dev, n, R, P, e, om, M0, s, rows, ll,
+                           blockmax, bound);
+        return hipGetLastError();
+    }
     const int64_t blocks = jk_dense_blocks(n);
     if constexpr (MIXED) {
         if (bound) {
@@ -1380,8 +1709,10 @@ hipError_t jk_launch_reject(const double *ll, int64_t n, const double *llmax, u1
 // inside the likelihood launch (one partial per wave).
 int64_t jk_lnl_reject_scratch_bytes(int64_t n)
 {
-    const int64_t waves = 4 * jk_dense_blocks(n);
-    return (int64_t)sizeof(double) * (waves + 1024) +
+    // the most partials a launch over n rows writes, whatever its epochs
+    int64_t parts = 4 * jk_dense_blocks(n);
+    if (n <= JK_SPLIT_MAX_ROWS) parts = std::max(parts, n / JK_SPLIT_RMIN + 1);
+    return (int64_t)sizeof(double) * (parts + 1024) +
            (int64_t)sizeof(uint64_t) * jk_reject_mask_words(n) +
            (int64_t)sizeof(int64_t) * jk_reject_bsum_count(n);
 }
@@ -1393,9 +1724,9 @@ hipError_t jk_launch_lnl_reject_f64(const jk_star *st, int64_t n, const double *
                                     int64_t *n_pass_out, double *llmax_out, void *scratch,
                                     hipStream_t stream)
 {
-    const int64_t waves = 4 * jk_dense_blocks(n);
-    double *partials = (double *)scratch;       // one per likelihood wave
-    double *partials2 = partials + waves;       // second level, at most 1024
+    const int64_t parts = jk_lnl_partials(n, st->dev.n);
+    double *partials = (double *)scratch;       // one per likelihood wave or workgroup
+    double *partials2 = partials + parts;       // second level, at most 1024
     uint64_t *mask = (uint64_t *)(partials2 + 1024);
     int64_t *bsum = (int64_t *)(mask + jk_reject_mask_words(n));
     hipError_t err;
@@ -1408,8 +1739,8 @@ hipError_t jk_launch_lnl_reject_f64(const jk_star *st, int64_t n, const double *
         err = launch_lnl_dispatch<false>(st, n, P, e, om, M0, s, rows, ll, partials, nullptr,
                                          stream);
         if (err != hipSuccess) return err;
-        // the per-wave maxima reduced like any array (two parallel levels)
-        err = jk_launch_max(partials, waves, partials2, jk_max_partials_count(waves), llmax_out,
+        // the partial maxima reduced like any array (two parallel levels)
+        err = jk_launch_max(partials, parts, partials2, jk_max_partials_count(parts), llmax_out,
                             stream);
     }
     if (err != hipSuccess) return err;
@@ -1532,8 +1863,8 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_batch(const StarDe
                                                    float *__restrict__ bound)
 {
     __shared__ unsigned s_item;
-    __shared__ double2 s_tab[JK_TAB_LDS];
-    jk_stage_tab(s_tab);
+    __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
+    jk_stage_tab<MIXED>(s_tab);
     for (;;) {
         if (threadIdx.x == 0) s_item = atomicAdd(counter, 1u);
         __syncthreads();
@@ -1670,8 +2001,8 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const 
     __shared__ unsigned s_item;
     __shared__ int s_n;
     __shared__ int s_list[JK_PRUNE_LIST];
-    __shared__ double2 s_tab[JK_TAB_LDS];
-    jk_stage_tab(s_tab);
+    __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
+    jk_stage_tab<MIXED>(s_tab);
     for (;;) {
         if (threadIdx.x == 0) s_item = atomicAdd(counter, 1u);
         __syncthreads();
@@ -2052,6 +2383,25 @@ __global__ __launch_bounds__(256) void k_seg_count_scan(const int64_t *__restric
     if (threadIdx.x == 255) cum[n_seg] = run;
 }
 
+// The segment of padded position j0: the last one that starts at or before it.
+__device__ __forceinline__ int jk_seg_of(const int64_t *__restrict__ cum, int n_seg, int64_t j0)
+{
+    int lo = 0, hi = n_seg;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (cum[mid] <= j0) lo = mid; else hi = mid;
+    }
+    return lo;
+}
+
+// Scatters of at most this many padded waves (49152 positions, as the dense
+// launch's line) take the split evaluation, 16 rows to a workgroup or as many
+// more as it takes to fill the grid once.  The FP64 re-evaluations around a
+// maximum are a few hundred rows: 100 epochs 36 -> 18 us, 16 epochs 10.6 ->
+// 8.6 us (8 or 32 rows to a workgroup: the same within 1 us).
+#define JK_SPLIT_SCATTER_WAVES 768
+#define JK_SPLIT_SCATTER_LGR 4
+
 // FP64 re-evaluation of every segment's selected entries as one flat list
 // spread over the whole grid: wavefront w takes padded positions
 // [64 w, 64 w + 64), all in one segment (found by binary search in cum and
@@ -2072,20 +2422,43 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_seg_scatter_f64(const 
                                                          double *__restrict__ ll,
                                                          float *__restrict__ bound)
 {
-    __shared__ double2 s_tab[JK_TAB_LDS];
-    jk_stage_tab(s_tab);
+    __shared__ double2 s_tab[JK_TAB_LDS64];
+    __shared__ SplitLds<L, PHYS, false> sh;
     const int lane = threadIdx.x & 63;
     const int64_t total_waves = cum[n_seg] >> 6;
+    if (total_waves <= JK_SPLIT_SCATTER_WAVES) {
+        // Few rows: each 64 positions over 64 / R workgroups, a row's epochs
+        // over many lanes (jk_rows_split; the same bits).
+        int lgR = JK_SPLIT_SCATTER_LGR;
+        while (lgR < 6 && (total_waves << (6 - lgR)) > gridDim.x) ++lgR;
+        const int R = 1 << lgR, sw = jk_split_wave(blockIdx.x), sl = jk_split_lane(sw),
+                  row = jk_split_row(sl, R);
+        const int64_t units = total_waves << (6 - lgR);
+        if ((int64_t)blockIdx.x >= units) return;
+        jk_stage_tab<false>(s_tab);
+        for (int64_t w = blockIdx.x; w < units; w += gridDim.x) {
+            const int64_t j0 = w << lgR;
+            const int sidx = __builtin_amdgcn_readfirstlane(jk_seg_of(cum, n_seg, j0));
+            const SegDev &sg = segs[sidx];
+            const int64_t local = j0 - cum[sidx] + row;
+            const bool some = row < R && local < count[sidx];
+            const int64_t p = some ? idx[sg.idx_off + local] : 0, q = sg.row0 + p;
+            const double v = jk_rows_split<L, PHYS, false>(
+                stars[sg.star], R, sw, some ? (rows ? rows[q] : q) : -1, P, e_, om_, M0_, s_, s_tab,
+                sh, nullptr);
+            if (some && sl < R) {
+                ll[sg.off + p] = v;
+                if (bound) bound[sg.off + p] = 0.0f;
+            }
+        }
+        return;
+    }
+    jk_stage_tab<false>(s_tab);
     const int64_t wstride = (int64_t)gridDim.x * (blockDim.x >> 6);
     for (int64_t w = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
          w < total_waves; w += wstride) {
         const int64_t j0 = w << 6;
-        int lo = 0, hi = n_seg;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (cum[mid] <= j0) lo = mid; else hi = mid;
-        }
-        const int sidx = __builtin_amdgcn_readfirstlane(lo);
+        const int sidx = __builtin_amdgcn_readfirstlane(jk_seg_of(cum, n_seg, j0));
         const SegDev &sg = segs[sidx];
         const int64_t local = j0 - cum[sidx] + lane;
         if (local < count[sidx]) {
