@@ -286,12 +286,14 @@ static int star_build(int n, const double *t, const double *rv, const double *iv
         d.ln_lam_trend += log(lambda_diag[i]);
     }
 
-    // Host epoch arrays: dt, r' = y - T mu_trend, y, ivar, T (L-1 rows of n).
+    // Host epoch arrays: dt, r' = y - T mu_trend, y, ivar, 1/ivar, T (L-1 rows of
+    // n), then the epochs' records.
     const int LT = L - 1;
     const size_t n_q = Qt ? (size_t)n * n : 0;
-    std::vector<double> h((size_t)n * (5 + LT) + n_q);
+    const size_t n_ep = JK_EPOCH_DOUBLES(n, LT);
+    std::vector<double> h(n_ep + n_q);
     double *h_dt = h.data(), *h_rp = h_dt + n, *h_y = h_rp + n, *h_iv = h_y + n, *h_s2 = h_iv + n,
-           *h_T = h_s2 + n;
+           *h_T = h_s2 + n, *h_ep = h_T + (size_t)LT * n;
     d.sum_ln_ivar = 0.0;
     d.S_rr = 0.0;
     for (int k = 0; k < n; ++k) {
@@ -310,6 +312,13 @@ static int star_build(int n, const double *t, const double *rv, const double *iv
         h_y[k] = rv[k];
         h_iv[k] = ivar[k];
         h_s2[k] = 1.0 / ivar[k];
+        double *rec = h_ep + (size_t)k * (JK_EP_T + LT);
+        rec[JK_EP_RP2] = rp * rp;
+        rec[JK_EP_SIG2] = h_s2[k];
+        rec[JK_EP_DT] = h_dt[k];
+        rec[JK_EP_RP] = rp;
+        rec[JK_EP_IVAR] = ivar[k];
+        for (int j = 0; j < LT; ++j) rec[JK_EP_T + j] = h_T[(size_t)j * n + k];
         d.sum_ln_ivar += log(ivar[k]);
         d.S_rr += ivar[k] * rp * rp;
         for (int j = 0; j < LT; ++j) {
@@ -328,7 +337,7 @@ static int star_build(int n, const double *t, const double *rv, const double *iv
     d.ln_c = d.ln_c_phys - d.sum_ln_ivar;
     for (int j = 0; j < LT; ++j)
         for (int q = 0; q < j; ++q) d.S_tt[q * JK_LMAX + j] = d.S_tt[j * JK_LMAX + q];
-    if (Qt) std::copy(Qt, Qt + n_q, h.begin() + (size_t)n * (5 + LT));
+    if (Qt) std::copy(Qt, Qt + n_q, h.begin() + n_ep);
 
     void *dmem = nullptr;
     if (hipMalloc(&dmem, h.size() * sizeof(double)) != hipSuccess) {
@@ -352,8 +361,9 @@ static int star_build(int n, const double *t, const double *rv, const double *iv
     d.y = base + 2 * n;
     d.ivar = base + 3 * n;
     d.sig2 = base + 4 * n;
-    d.T = base + 5 * n;
-    d.Qt = Qt ? base + (size_t)n * (5 + LT) : nullptr;
+    d.T = base + JK_EPOCH_ARRAYS * n;
+    d.ep = d.T + (size_t)LT * n;
+    d.Qt = Qt ? base + n_ep : nullptr;
     *out = st;
     return JK_OK;
 }
@@ -702,7 +712,7 @@ int jk_batch_create(const jk_star *const *stars, int n_stars, jk_batch **out)
     for (int i = 0; i < n_stars; ++i) {
         if (!stars[i] || stars[i]->dev.L != L || stars[i]->dev.jitter_mode != jm) return JK_EINVAL;
         if (stars[i]->dev.Qt) return JK_EINVAL;   // full covariance: single-star calls only
-        n_epoch_doubles += (size_t)stars[i]->dev.n * (5 + L - 1);
+        n_epoch_doubles += JK_EPOCH_DOUBLES(stars[i]->dev.n, L - 1);
     }
     jk_batch *b = new (std::nothrow) jk_batch;
     if (!b) return JK_ENOMEM;
@@ -722,7 +732,7 @@ int jk_batch_create(const jk_star *const *stars, int n_stars, jk_batch **out)
     size_t off = 0;
     for (int i = 0; i < n_stars; ++i) {
         h[i] = stars[i]->dev;
-        const size_t cnt = (size_t)h[i].n * (5 + L - 1);
+        const size_t cnt = JK_EPOCH_DOUBLES(h[i].n, L - 1);
         if (hipMemcpy(base + off, stars[i]->d_epochs, sizeof(double) * cnt,
                       hipMemcpyDeviceToDevice) != hipSuccess) {
             (void)hipFree(b->d_stars);
@@ -737,7 +747,8 @@ int jk_batch_create(const jk_star *const *stars, int n_stars, jk_batch **out)
         h[i].y = p + 2 * n;
         h[i].ivar = p + 3 * n;
         h[i].sig2 = p + 4 * n;
-        h[i].T = p + 5 * n;
+        h[i].T = p + JK_EPOCH_ARRAYS * n;
+        h[i].ep = h[i].T + (size_t)(L - 1) * n;
         off += cnt;
     }
     if (hipMemcpy(b->d_stars, h.data(), sizeof(StarDev) * n_stars, hipMemcpyHostToDevice) !=

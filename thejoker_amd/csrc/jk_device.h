@@ -28,6 +28,15 @@
 #define JK_KEPLER_MAXITER 128
 #define JK_KEPLER_TOL 1e-10
 
+// An epoch's record in StarDev::ep: the values the likelihood rows read per
+// epoch, side by side, so that a wave fetches them with one run of scalar
+// loads from one base address.  The physical jitter mode reads the first four
+// (and T), the reference mode dt, r', ivar and T.
+enum { JK_EP_RP2 = 0, JK_EP_SIG2, JK_EP_DT, JK_EP_RP, JK_EP_IVAR, JK_EP_T };
+#define JK_EPOCH_ARRAYS 5   // arrays of StarDev before T
+// FP64 values of a star's epoch block: the arrays, T and the records.
+#define JK_EPOCH_DOUBLES(n, LT) ((size_t)(n) * (JK_EPOCH_ARRAYS + (LT) + JK_EP_T + (LT)))
+
 // Per-star constants, device resident, read through scalar loads (every lane
 // of a wavefront evaluates the same epoch at the same time).
 struct StarDev {
@@ -63,13 +72,15 @@ struct StarDev {
     // Posterior right-hand side pieces: sum ivar T_j y (j >= 1).
     double S_ty[JK_LMAX];
     // Epoch arrays (device): dt = t - t_ref, rp = r', y, ivar, sig2 = 1/ivar,
-    // T (L-1 rows of n).
+    // T (L-1 rows of n); then ep, the epochs' records (JK_EP_*: n of JK_EP_T +
+    // L-1 values).
     const double *dt;
     const double *rp;
     const double *y;
     const double *ivar;
     const double *sig2;
     const double *T;
+    const double *ep;
     // Full-covariance stars (nullptr otherwise): Q^T, n x n row-major, whose
     // rows are the eigenvectors of the data covariance C.  rp, y, T are then
     // rotated into that eigenbasis (Q^T r', Q^T y, Q^T T), ivar and sig2 hold

@@ -87,7 +87,7 @@ __device__ __forceinline__ void jk_sincos_tab_f64(double x, const double2 *__res
     int idx = (int)(ay * (JK_TAB_N / JK_PI));
     idx = min(max(idx, 0), JK_TAB_N);
     const double2 t = tab[idx];
-    const double d = ay - (double)idx * JK_TAB_H;
+    const double d = fma(-(double)idx, JK_TAB_H, ay);
     const double d2 = d * d;
     const double sd = fma(d * d2, fma(d2, 1.0 / 120.0, -1.0 / 6.0), d);
     const double cd = fma(d2, fma(d2, 1.0 / 24.0, -0.5), 1.0);
@@ -101,7 +101,8 @@ __device__ __forceinline__ void jk_sincos_tab_f64(double x, const double2 *__res
 //   sin Ef = sin g_i cos d + cos g_i sin d,  cos Ef = cos g_i cos d - sin g_i sin d
 // with sin d to d^5 and cos d to d^4 (truncation below 2e-18).  d is exact:
 // Ef has 24 significant bits and g_i 42 on a grid of the same scale, so their
-// difference needs fewer than 53.
+// difference needs fewer than 53 (one fma: i H is exact, so the fused form
+// gives the same bits as the product and the difference).
 // The index is clamped into the table whatever Ef is.
 __device__ __forceinline__ void jk_sincos_tab(float Ef, const double2 *__restrict__ tab,
                                               double &s, double &c)
@@ -109,7 +110,7 @@ __device__ __forceinline__ void jk_sincos_tab(float Ef, const double2 *__restric
     int idx = (int)(Ef * JK_TAB_INV_H_F);
     idx = min(max(idx, 0), JK_TAB_N);
     const double2 t = tab[idx];
-    const double d = (double)Ef - (double)idx * JK_TAB_H;
+    const double d = fma(-(double)idx, JK_TAB_H, (double)Ef);
     const double d2 = d * d;
     const double sd = fma(d * d2, fma(d2, 1.0 / 120.0, -1.0 / 6.0), d);
     const double cd = fma(d2, fma(d2, 1.0 / 24.0, -0.5), 1.0);
@@ -256,8 +257,8 @@ __device__ __forceinline__ bool jk_kepler_markley_f64(double x, double e, float 
     const double t = -f0 * r;
     const double b2 = (0.5 * e) * s1 * r;
     // e cos E1 r = r - 1 (r (1 - e cos E1) = 1 to a few ulp; the absolute
-    // error of r - 1 moves d by t^3 5e-16, far below ulp(E))
-    const double b3 = (r - 1.0) * (1.0 / 6.0);
+    // error of r - 1 moves d by t^3 5e-16, far below ulp(E)), over 6 in one fma
+    const double b3 = fma(r, 1.0 / 6.0, -1.0 / 6.0);
     const double b22 = b2 * b2;
     const double c3 = fma(2.0, b22, -b3);
     const double c4 = b2 * fma(5.0, b3 - b22, 1.0 / 12.0);   // -b4 = b2 / 12
@@ -290,7 +291,8 @@ __device__ __forceinline__ void jk_kepler_markley_f32(float x, float e, float om
     const float t = -f0 * __builtin_amdgcn_rcpf(fmaf(-e, c1, 1.0f));
     const float s = fmaf(c1, t, s1);
     cosE = fmaf(-s1, t, c1);
-    sinE = x < 0.0f ? -s : s;
+    // the sign of x flipped into s by bits (no FP64 compare of the phase)
+    sinE = __uint_as_float(__float_as_uint(s) ^ (__float_as_uint(x) & 0x80000000u));
 }
 
 // ---------------------------------------------------------------------------
@@ -318,7 +320,7 @@ __device__ __forceinline__ void jk_kepler_markley_f32(float x, float e, float om
 
 // One prior row's orbit: what every epoch of it shares.
 struct RowOrbit {
-    double e, invP, nP, M0, M0t, s2, lam0, cw, ecw, swsq, dmax;
+    double e, invP, nP, M0, M0t, s2, lam0, cwq, swsq, dmax;
     // FP32 copies for the Kepler starter (e capped below 1 in FP32; 1 - e
     // rounded from its FP64 value, so it keeps its relative accuracy) and for
     // the mixed row's design value, which is combined in FP32.
@@ -369,13 +371,14 @@ __device__ __forceinline__ bool jk_row_orbit(const StarDev &st, int64_t r,
     o.ef = fminf((float)ev, 0.99999994f);
     o.omef = fmaxf((float)(1.0 - ev), 5.9604645e-08f);
     o.a1f = JK_MARKLEY_A1N * __builtin_amdgcn_rcpf(1.0f + o.ef);
-    double sw;
-    jk_sincos_tab_f64(omv, tab, sw, o.cw);
-    o.ecw = ev * o.cw;
-    o.swsq = sw * sqrt((1.0 - ev) * (1.0 + ev));
-    o.cwf = (float)o.cw;
+    double sw, cw;
+    jk_sincos_tab_f64(omv, tab, sw, cw);
+    const double q2 = (1.0 - ev) * (1.0 + ev);
+    o.swsq = sw * sqrt(q2);
+    o.cwq = cw * q2;
+    o.cwf = (float)cw;
     o.swsqf = (float)o.swsq;
-    o.ecwf = (float)o.ecw;
+    o.ecwf = (float)(ev * cw);
     // The FP32 starter sees e rounded to FP32; within 1e-7 of 1 that can put
     // it outside the correction's reach, so such samples take the fallback.
     o.dmax = ev > 0.9999999 ? -1.0 : 1e-3;
@@ -430,10 +433,13 @@ __device__ __forceinline__ double jk_row_epoch(const RowOrbit &o, double dtk, do
         } else {
             bad |= !jk_kepler_markley_f64(x, o.e, o.ef, o.omef, o.a1f, o.dmax, tab, sE, cE);
         }
-        // m = [cos w (cos E - e) - sin w sqrt(1-e^2) sin E] / (1 - e cos E) + e cos w
-        // (one Newton step on the hardware reciprocal: relative 2e-15)
+        // m = [cos w (1-e^2) cos E - sin w sqrt(1-e^2) sin E] / (1 - e cos E)
+        // (one Newton step on the hardware reciprocal: relative 2e-15).
+        // cos f + e = (1-e^2) cos E / (1 - e cos E): one FP64 operation fewer
+        // than cos w (cos E - e) ... + e cos w, and no cancellation between
+        // the two terms in cos w
         const double den = jk_rcp1(fma(-o.e, cE, 1.0));
-        m = fma(fma(o.cw, cE - o.e, -o.swsq * sE), den, o.ecw);
+        m = fma(o.cwq, cE, -o.swsq * sE) * den;
     }
     return m;
 }
@@ -510,8 +516,18 @@ __device__ __forceinline__ double jk_row_finish(const StarDev &st, double lam0,
 }
 
 // With ONE the first trend column is the constant 1 (StarDev::t0_one): its
-// products fold away, with the same roundings (w * 1 = w exactly).
-template <int L, bool PHYS, bool MIXED, bool SAFE = false, bool BOUND = false, bool ONE = false>
+// products fold away, with the same roundings (w * 1 = w exactly), and the
+// bound's sum of the weights is that column's own moment.
+// With REC the epoch loop reads the epochs' records (StarDev::ep: one base
+// address, so few scalar registers and one or two scalar loads per epoch),
+// else the separate arrays.  Same values either way; which is faster is the
+// register allocator's doing: the FP64 rows (their separate arrays spilled
+// scalars into vector lanes: 2^24 rows x 16 epochs 957 -> 927 us with the
+// operations saved above, 2^20 x 37 at L = 5 134 -> 127 us) and the mixed
+// rows of many stars (64 x 2^18 rows 1935 -> 1895 us) take the records, the
+// mixed single-star row the arrays (2^22 x 50: 394 us, with records 415).
+template <int L, bool PHYS, bool MIXED, bool SAFE = false, bool BOUND = false, bool ONE = false,
+          bool REC = !MIXED>
 __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
                                              const double *__restrict__ P,
                                              const void *__restrict__ e_,
@@ -526,7 +542,7 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
     RowOrbit o;
     if (!jk_row_orbit<PHYS>(st, r, P, e_, om_, M0_, s_, tab, o)) return __builtin_nan("");
 
-    constexpr int LT = L > 1 ? L - 1 : 1;
+    constexpr int LT = L > 1 ? L - 1 : 1, LT0 = L - 1;
     double Smm = 0.0, Smr = 0.0;
     double Smt[LT];
     double Stt[LT * LT], Str[LT], Srr = 0.0;
@@ -542,15 +558,19 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
 
     const int N = st.n;
     bool bad = false;
-    double Sw = 0.0;       // sum w (BOUND only)
+    double Sw = 0.0;       // sum w (BOUND only; with ONE it is Stt[0])
     float dmx = 0.0f;      // largest 1 / (1 - e cos E) (BOUND only)
-#pragma unroll 2
+    // four epochs at a time where every fourth renormalises the product and the
+    // registers allow it (2^24 rows x 16 epochs 936 -> 930 us), else two
+#pragma unroll (PHYS && !MIXED && ONE ? 4 : 2)
     for (int k = 0; k < N; ++k) {
-        const double vk = PHYS ? st.sig2[k] + o.s2 : 0.0;
+        const double *__restrict__ ep = st.ep + (size_t)k * (JK_EP_T + LT0);
+        const double vk = PHYS ? (REC ? ep[JK_EP_SIG2] : st.sig2[k]) + o.s2 : 0.0;
         double w = 0.0;
         float denb = 0.0f;
-        const double m = jk_row_epoch<PHYS, MIXED, SAFE>(o, st.dt[k], vk, tab, w, denb, bad);
-        const double rp = st.rp[k];
+        const double m = jk_row_epoch<PHYS, MIXED, SAFE>(o, REC ? ep[JK_EP_DT] : st.dt[k], vk,
+                                                              tab, w, denb, bad);
+        const double rp = REC ? ep[JK_EP_RP] : st.rp[k];
         if constexpr (PHYS) {
             // sum ln w = -ln of the running product of the FP64 variances,
             // renormalised every fourth epoch (frexp scales by a power of
@@ -564,10 +584,10 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
                 pexp += ex;
             }
         } else {
-            w = st.ivar[k];
+            w = REC ? ep[JK_EP_IVAR] : st.ivar[k];
         }
         if constexpr (BOUND) {
-            Sw += w;
+            if constexpr (!ONE) Sw += w;
             dmx = fmaxf(dmx, denb);
         }
         const double wm = w * m;
@@ -576,21 +596,30 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
         if constexpr (L > 1) {
 #pragma unroll
             for (int j = 0; j < L - 1; ++j) {
-                const double Tj = ONE && j == 0 ? 1.0 : st.T[j * N + k];
+                const double Tj =
+                    ONE && j == 0 ? 1.0 : (REC ? ep[JK_EP_T + j] : st.T[j * N + k]);
                 Smt[j] = fma(wm, Tj, Smt[j]);
                 if constexpr (PHYS) {
                     const double wT = w * Tj;
                     Str[j] = fma(wT, rp, Str[j]);
 #pragma unroll
-                    for (int q = 0; q <= j; ++q)
-                        Stt[j * LT + q] =
-                            fma(wT, ONE && q == 0 ? 1.0 : st.T[q * N + k], Stt[j * LT + q]);
+                    for (int q = 0; q <= j; ++q) {
+                        const double Tq =
+                            ONE && q == 0 ? 1.0 : (REC ? ep[JK_EP_T + q] : st.T[q * N + k]);
+                        Stt[j * LT + q] = fma(wT, Tq, Stt[j * LT + q]);
+                    }
                 }
             }
         }
-        if constexpr (PHYS) Srr = fma(w * rp, rp, Srr);
+        if constexpr (PHYS) {
+            if constexpr (MIXED)
+                Srr = fma(w * rp, rp, Srr);
+            else    // r'^2 rounded once, on the host where the record holds it
+                Srr = fma(w, REC ? ep[JK_EP_RP2] : rp * rp, Srr);
+        }
     }
 
+    if constexpr (BOUND && ONE) Sw = PHYS ? Stt[0] : st.S_tt[0];
     if constexpr (!MIXED && !SAFE) {
         if (bad) return jk_lnl_row<L, PHYS, false, true>(st, r, P, e_, om_, M0_, s_, tab);
     }
@@ -779,7 +808,8 @@ __device__ __forceinline__ double jk_rows_split(const StarDev &st, int R, int sw
                             }
                         }
                     }
-                    if constexpr (PHYS) Srr = fma(w * rp, rp, Srr);
+                    if constexpr (PHYS)
+                        Srr = MIXED ? fma(w * rp, rp, Srr) : fma(w, rp * rp, Srr);
                 }
             }
         }
@@ -861,8 +891,8 @@ __device__ double jk_lnl_row_cov(const StarDev &st, int64_t r, const double *__r
     const float a1f = JK_MARKLEY_A1N * __builtin_amdgcn_rcpf(1.0f + ef);
     double sw, cw;
     jk_sincos_tab_f64(omv, tab, sw, cw);
-    const double ecw = ev * cw;
-    const double swsq = sw * sqrt((1.0 - ev) * (1.0 + ev));
+    const double q2 = (1.0 - ev) * (1.0 + ev);
+    const double swsq = sw * sqrt(q2), cwq = cw * q2;
     const double dmax = ev > 0.9999999 ? -1.0 : 1e-3;
     const int N = st.n;
 
@@ -876,7 +906,7 @@ __device__ double jk_lnl_row_cov(const StarDev &st, int64_t r, const double *__r
         else
             bad |= !jk_kepler_markley_f64(x, ev, ef, omef, a1f, dmax, tab, sE, cE);
         const double den = jk_rcp2(fma(-ev, cE, 1.0));
-        s_m[k * JK_COV_LANES] = fma(fma(cw, cE - ev, -swsq * sE), den, ecw);
+        s_m[k * JK_COV_LANES] = fma(cwq, cE, -swsq * sE) * den;
     }
     if constexpr (!SAFE) {
         if (bad) return jk_lnl_row_cov<L, PHYS, true>(st, r, P, e_, om_, M0_, s_, tab, s_m);
@@ -1023,7 +1053,7 @@ __global__ __launch_bounds__(256) void k_lnl(const StarDev st, int64_t n,
         double v;
         if constexpr (BOUND) {
             float b;
-            v = jk_lnl_row<L, PHYS, MIXED, false, true>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
+            v = jk_lnl_row<L, PHYS, MIXED, false, true, ONE>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
             bound[i] = b;
         } else {
             v = jk_lnl_row<L, PHYS, MIXED, false, false, ONE>(st, r, P, e_, om_, M0_, s_, s_tab);
@@ -1189,6 +1219,14 @@ static hipError_t launch_lnl_t(const jk_star *st, int64_t n, const double *P, co
     }
     const int64_t blocks = jk_dense_blocks(n);
     if constexpr (MIXED) {
+        if constexpr (L == 2 || L == 3) {
+            if (bound && st->dev.t0_one) {
+                hipLaunchKernelGGL((k_lnl<L, PHYS, true, true, true>), dim3((unsigned)blocks),
+                                   dim3(256), 0, stream, st->dev, n, P, e, om, M0, s, rows, ll,
+                                   blockmax, bound);
+                return hipGetLastError();
+            }
+        }
         if (bound) {
             hipLaunchKernelGGL((k_lnl<L, PHYS, true, true>), dim3((unsigned)blocks), dim3(256), 0,
                                stream, st->dev, n, P, e, om, M0, s, rows, ll, blockmax, bound);
@@ -1841,7 +1879,8 @@ __device__ __forceinline__ double jk_lnl_row_sel(const StarDev &st, int64_t r,
         *bnd = 0.0f;
         return jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, tab);
     }
-    return jk_lnl_row<L, PHYS, true, false, true>(st, r, P, e_, om_, M0_, s_, tab, bnd);
+    return jk_lnl_row<L, PHYS, true, false, true, false, true>(st, r, P, e_, om_, M0_, s_, tab,
+                                                               bnd);
 }
 
 // Slot `slot` of a star table evaluated in FP64 (exact != 0) or as the launch
@@ -1883,7 +1922,8 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_batch(const StarDe
             } else if constexpr (MIXED) {
                 ll[w.out_offset + j] =
                     st.exact ? jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab)
-                             : jk_lnl_row<L, PHYS, true>(st, r, P, e_, om_, M0_, s_, s_tab);
+                             : jk_lnl_row<L, PHYS, true, false, false, false, true>(
+                                   st, r, P, e_, om_, M0_, s_, s_tab);
             } else {
                 ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
             }
