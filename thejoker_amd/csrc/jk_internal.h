@@ -7,8 +7,9 @@
 
 #include "jk_device.h"
 
-// Largest epoch count of a full-covariance star (jk_star_create_cov): its
-// kernels keep a row's design column, one double per epoch and lane, in LDS.
+// Largest epoch count of a full-covariance star (jk_star_create_cov): the
+// likelihood keeps its eigenvector matrix in LDS, the posterior a row's design
+// column per lane.
 #define JK_COV_NMAX 64
 
 // Host mirror of one star: the StarDev block passed by value to kernels,

@@ -853,147 +853,85 @@ static int jk_split_rows(int64_t n, int N)
 }
 
 // ---------------------------------------------------------------------------
-// Full-covariance row, FP64.  With C = Q diag(lambda) Q^T, C + s^2 I is
+// Full-covariance rows, FP64.  With C = Q diag(lambda) Q^T, C + s^2 I is
 // diagonal in the same eigenbasis (lambda + s^2), and the marginal
 // likelihood ln N(y | M mu, C + s^2 I + M Lambda M^T) does not change under
 // the orthogonal change of basis (|det Q| = 1).  The star's data are stored
-// rotated (StarDev::Qt); the row's design column is computed per epoch as in
-// jk_lnl_row, kept in this lane's column of an LDS buffer (epoch k at
-// s_m[k * JK_COV_LANES]), rotated, m'_i = sum_k Qt[i][k] m_k, and fed to the
-// same moments and finish with the eigenvalues as the variances.  Each lane
-// reads back only its own writes, so no barrier is needed.
+// rotated (StarDev::Qt); the rows' design columns are computed per epoch and
+// rotated, m'_i = sum_k Qt[i][k] m_k, and fed to the same moments and finish
+// with the eigenvalues as the variances.
+//
+// The rotation of a wave's rows is a matrix product, and runs on the matrix
+// cores (FP64 16x16x4): a wave takes 16 rows, lane l evaluating row l & 15 at
+// epoch 4 c + (l >> 4) in step c, which is the product's right operand as it
+// stands; the left one, Q^T in LDS, is read once per step and 16 rows.  The
+// products accumulate in registers (16 eigenvalues a tile) while the next
+// step's Kepler solves run on the vector units, so the N^2 multiply-adds per
+// row cost next to nothing, and the solves bound the kernel as they do the
+// diagonal one.  Against one lane per row (a serial dot product, one LDS read
+// per multiply-add, 64 rows' columns in LDS): 2^18 rows x 40 epochs 182 ->
+// 75 us, 524288 x 64 1383 -> 245 us, 3000 x 64 84 -> 17 us, 2^18 x 5 30 ->
+// 27 us.
 // ---------------------------------------------------------------------------
-#define JK_COV_LANES 64
+#define JK_COV_ROWS 64      // rows per workgroup, 16 a wave
 
-template <int L, bool PHYS, bool SAFE = false>
-__device__ double jk_lnl_row_cov(const StarDev &st, int64_t r, const double *__restrict__ P,
-                                 const void *__restrict__ e_, const void *__restrict__ om_,
-                                 const void *__restrict__ M0_, const void *__restrict__ s_,
-                                 const double2 *__restrict__ tab, double *s_m)
+typedef double jk_f64x4 __attribute__((ext_vector_type(4)));
+
+// Doubles per epoch of the LDS copy of Q (epoch-major): a multiple of 16 at
+// least N, = 16 mod 32, so that the four epochs a step reads fall on
+// different banks.
+__host__ __device__ __forceinline__ int jk_cov_pitch(int N)
 {
-    const double *__restrict__ ecol = static_cast<const double *>(e_);
-    const double *__restrict__ omcol = static_cast<const double *>(om_);
-    const double *__restrict__ M0col = static_cast<const double *>(M0_);
-    const double *__restrict__ scol = static_cast<const double *>(s_);
-    const double Pv = P[r], ev = ecol[r], omv = omcol[r], M0v = M0col[r];
-    const double sv = PHYS ? scol[r] : 0.0;
-    bool valid = isfinite(Pv) && Pv != 0.0 && ev >= 0.0 && ev < 1.0 && isfinite(omv) &&
-                 isfinite(M0v);
-    if (PHYS) valid = valid && isfinite(sv);
-    if (!valid) return __builtin_nan("");
-    const double lam0 = st.k_prior_mode == JK_KPRIOR_FIXED_COMPANION_MASS
-                            ? jk_k_variance(&st, Pv, ev, true)
-                            : st.lam0;
-    const double nP = JK_TWO_PI * jk_rcp2(Pv);
-    const double s2 = sv * sv;
-    const float ef = fminf((float)ev, 0.99999994f);
-    const float omef = fmaxf((float)(1.0 - ev), 5.9604645e-08f);
-    const float a1f = JK_MARKLEY_A1N * __builtin_amdgcn_rcpf(1.0f + ef);
-    double sw, cw;
-    jk_sincos_tab_f64(omv, tab, sw, cw);
-    const double q2 = (1.0 - ev) * (1.0 + ev);
-    const double swsq = sw * sqrt(q2), cwq = cw * q2;
-    const double dmax = ev > 0.9999999 ? -1.0 : 1e-3;
-    const int N = st.n;
+    return (N + 15) / 32 * 32 + 16;
+}
 
-    // the design column in epoch order
-    bool bad = false;
-    for (int k = 0; k < N; ++k) {
-        const double x = jk_reduce_2pi(fma(nP, st.dt[k], -M0v));
-        double sE, cE;
-        if constexpr (SAFE)
-            jk_kepler_poly_f64(x, ev, tab, sE, cE);
-        else
-            bad |= !jk_kepler_markley_f64(x, ev, ef, omef, a1f, dmax, tab, sE, cE);
-        const double den = jk_rcp2(fma(-ev, cE, 1.0));
-        s_m[k * JK_COV_LANES] = fma(cwq, cE, -swsq * sE) * den;
-    }
-    if constexpr (!SAFE) {
-        if (bad) return jk_lnl_row_cov<L, PHYS, true>(st, r, P, e_, om_, M0_, s_, tab, s_m);
-    }
+// Dynamic LDS of k_lnl_cov: Q, then per eigenvalue r', sigma^2 / ivar and T,
+// and dt per epoch.
+__host__ __device__ __forceinline__ int jk_cov_lds_doubles(int N, int L)
+{
+    return (N + 3) / 4 * 4 * jk_cov_pitch(N) + N * (L + 2);
+}
 
-    // moments in the eigenbasis
-    constexpr int LT = L > 1 ? L - 1 : 1;
-    double Smm = 0.0, Smr = 0.0, Srr = 0.0;
-    double Smt[LT], Stt[LT * LT], Str[LT];
-    double prod = 1.0;
-    int pexp = 0;
+// The rotated design values of the wave's rows: acc[t][r] of lane l is
+// eigenvalue 16 t + 4 r + (l >> 4) of row l & 15.  With SAFE, rows marked bad
+// take the bracketed Newton iteration; else bad is set where a row needs it.
+template <bool SAFE>
+__device__ __forceinline__ void jk_cov_rotate(const StarDev &st, const RowOrbit &o, bool valid,
+                                              const double2 *__restrict__ tab,
+                                              const double *s_q, const double *s_dt,
+                                              jk_f64x4 acc[4], bool &bad)
+{
+    const int lane = threadIdx.x & 63, kq = lane >> 4, N = st.n;
+    const int pitch = jk_cov_pitch(N), nt = (N + 15) / 16;
 #pragma unroll
-    for (int j = 0; j < LT; ++j) {
-        Smt[j] = 0.0;
-        Str[j] = 0.0;
-#pragma unroll
-        for (int q = 0; q < LT; ++q) Stt[j * LT + q] = 0.0;
-    }
-    for (int i = 0; i < N; ++i) {
-        const double *__restrict__ q = st.Qt + (size_t)i * N;
+    for (int t = 0; t < 4; ++t) acc[t] = jk_f64x4{0.0, 0.0, 0.0, 0.0};
+    for (int k0 = 0; k0 < N; k0 += 4) {
+        const int k = k0 + kq;
         double m = 0.0;
-        for (int k = 0; k < N; ++k) m = fma(q[k], s_m[k * JK_COV_LANES], m);
-        const double rp = st.rp[i];
-        double w;
-        if constexpr (PHYS) {
-            const double d = st.sig2[i] + s2;
-            w = jk_rcp2(d);
-            int ex;
-            prod = frexp(prod * d, &ex);
-            pexp += ex;
-        } else {
-            w = st.ivar[i];
-        }
-        const double wm = w * m;
-        Smm = fma(wm, m, Smm);
-        Smr = fma(wm, rp, Smr);
-        if constexpr (L > 1) {
-#pragma unroll
-            for (int j = 0; j < L - 1; ++j) {
-                const double Tj = st.T[j * N + i];
-                Smt[j] = fma(wm, Tj, Smt[j]);
-                if constexpr (PHYS) {
-                    const double wT = w * Tj;
-                    Str[j] = fma(wT, rp, Str[j]);
-#pragma unroll
-                    for (int qq = 0; qq <= j; ++qq)
-                        Stt[j * LT + qq] = fma(wT, st.T[qq * N + i], Stt[j * LT + qq]);
-                }
+        if (valid && k < N) {
+            double w;
+            float denb;
+            bool b = false;
+            m = jk_row_epoch<false, false, false>(o, s_dt[k], 0.0, tab, w, denb, b);
+            if constexpr (SAFE) {
+                if (bad) m = jk_row_epoch<false, false, true>(o, s_dt[k], 0.0, tab, w, denb, b);
+            } else {
+                bad |= b;
             }
         }
-        if constexpr (PHYS) Srr = fma(w * rp, rp, Srr);
+        const double *q = s_q + (size_t)k * pitch + (lane & 15);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (t < nt)
+                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(q[16 * t], m, acc[t], 0, 0, 0);
     }
+}
 
-    // G, u, chi0 and the log-constant as in jk_lnl_row
-    double G[L * L], u[L];
-    const double mu0 = st.mu0;
-    const bool fcm = st.k_prior_mode == JK_KPRIOR_FIXED_COMPANION_MASS;
-    G[0] = (fcm ? jk_rcp2(lam0) : st.lam_inv[0]) + Smm;
-    u[0] = fma(-mu0, Smm, Smr);
-    double chi0, lnc, scale = 1.0;
-    if constexpr (PHYS) {
-        chi0 = Srr;
-        lnc = st.ln_c_phys + (double)pexp * JK_LN2;
-        scale = prod;
-    } else {
-        chi0 = st.S_rr;
-        lnc = st.ln_c;
-    }
-    if (fcm) scale *= lam0;
-    chi0 = fma(mu0 * mu0, Smm, fma(-2.0 * mu0, Smr, chi0));
-    if constexpr (L > 1) {
-#pragma unroll
-        for (int j = 1; j < L; ++j) {
-            G[j * L] = Smt[j - 1];
-            G[j] = Smt[j - 1];
-            const double trj = PHYS ? Str[j - 1] : st.S_tr[j - 1];
-            u[j] = fma(-mu0, Smt[j - 1], trj);
-#pragma unroll
-            for (int q = 1; q <= j; ++q) {
-                const double tt = PHYS ? Stt[(j - 1) * LT + (q - 1)] : st.S_tt[(j - 1) * JK_LMAX + (q - 1)];
-                const double g = (q == j ? st.lam_inv[j] : 0.0) + tt;
-                G[j * L + q] = g;
-                G[q * L + j] = g;
-            }
-        }
-    }
-    return jk_finish_lnl<L>(G, u, chi0, lnc, scale, tab + JK_TAB_LOG_OFF);
+// Sum over the four lanes of a row (the same value in each).
+__device__ __forceinline__ double jk_cov_sum(double v)
+{
+    v += __shfl_xor(v, 16, 64);
+    return v + __shfl_xor(v, 32, 64);
 }
 
 // ---------------------------------------------------------------------------
@@ -1104,25 +1042,123 @@ __global__ __launch_bounds__(256) void k_lnl_split(const StarDev st, int64_t n, 
     }
 }
 
-// Full-covariance stars, FP64: one lane per row, 64 lanes per workgroup, the
-// design columns in dynamic LDS (N x 64 doubles).
+// Full-covariance stars, FP64: 16 rows per wave (jk_cov_rotate), the
+// workgroups striding over the rows so that each stages Q and the tables once.
 template <int L, bool PHYS>
-__global__ __launch_bounds__(JK_COV_LANES) void k_lnl_cov(const StarDev st, int64_t n,
-                                                          const double *__restrict__ P,
-                                                          const void *__restrict__ e_,
-                                                          const void *__restrict__ om_,
-                                                          const void *__restrict__ M0_,
-                                                          const void *__restrict__ s_,
-                                                          const int64_t *__restrict__ rows,
-                                                          double *__restrict__ ll)
+__global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev st, int64_t n,
+                                                 const double *__restrict__ P,
+                                                 const void *__restrict__ e_,
+                                                 const void *__restrict__ om_,
+                                                 const void *__restrict__ M0_,
+                                                 const void *__restrict__ s_,
+                                                 const int64_t *__restrict__ rows,
+                                                 double *__restrict__ ll)
 {
     __shared__ double2 s_tab[JK_TAB_LDS64];
-    extern __shared__ double s_m[];
+    extern __shared__ double s_q[];
+    const int N = st.n, pitch = jk_cov_pitch(N), K4 = (N + 3) / 4 * 4;
+    double *s_ep = s_q + K4 * pitch;      // r', sigma^2 (PHYS) or ivar, T per eigenvalue
+    for (int q = threadIdx.x; q < K4 * pitch; q += 256) {
+        const int k = q / pitch, i = q - k * pitch;
+        s_q[q] = k < N && i < N ? st.Qt[(size_t)i * N + k] : 0.0;
+    }
+    for (int q = threadIdx.x; q < N * (L + 2); q += 256) {
+        const int v = q / N, i = q - v * N;
+        s_ep[q] = v == 0 ? st.rp[i]
+                         : (v == 1 ? (PHYS ? st.sig2[i] : st.ivar[i])
+                                   : (v == L + 1 ? st.dt[i] : st.T[(size_t)(v - 2) * N + i]));
+    }
+    const double *s_dt = s_ep + (L + 1) * N;
     jk_stage_tab<false>(s_tab);
-    const int64_t i = (int64_t)blockIdx.x * JK_COV_LANES + threadIdx.x;
-    if (i < n) {
-        const int64_t r = rows ? rows[i] : i;
-        ll[i] = jk_lnl_row_cov<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, s_m + threadIdx.x);
+    const int lane = threadIdx.x & 63, kq = lane >> 4;
+    for (int64_t i0 = (int64_t)blockIdx.x * JK_COV_ROWS; i0 < n;
+         i0 += (int64_t)gridDim.x * JK_COV_ROWS) {
+        const int64_t i = i0 + (threadIdx.x >> 6) * 16 + (lane & 15);
+        RowOrbit o;
+        const bool valid =
+            i < n && jk_row_orbit<PHYS>(st, rows ? rows[i] : i, P, e_, om_, M0_, s_, s_tab, o);
+        jk_f64x4 acc[4];
+        bool bad = false;
+        jk_cov_rotate<false>(st, o, valid, s_tab, s_q, s_dt, acc, bad);
+        if (__any(bad)) {
+            // a row is bad when any of its epochs is
+            const unsigned long long bw = __ballot(bad);
+            bad = ((bw | bw >> 16 | bw >> 32 | bw >> 48) >> (lane & 15)) & 1;
+            jk_cov_rotate<true>(st, o, valid, s_tab, s_q, s_dt, acc, bad);
+        }
+        // moments in the eigenbasis, a quarter of the eigenvalues per lane
+        constexpr int LT = L > 1 ? L - 1 : 1;
+        double Smm = 0.0, Smr = 0.0, Srr = 0.0, prod = 1.0;
+        double Smt[LT], Str[LT], Stt[LT * LT];
+        int pexp = 0;
+#pragma unroll
+        for (int j = 0; j < LT; ++j) {
+            Smt[j] = 0.0;
+            Str[j] = 0.0;
+#pragma unroll
+            for (int q = 0; q < LT; ++q) Stt[j * LT + q] = 0.0;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if (16 * t >= N) break;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int ei = 16 * t + 4 * r + kq;
+                if (ei >= N) continue;
+                const double m = acc[t][r], rp = s_ep[ei];
+                double w = s_ep[N + ei];
+                if constexpr (PHYS) {
+                    const double vk = w + o.s2;
+                    w = jk_rcp1(vk);
+                    prod *= vk;      // at most four factors between renormalisations
+                }
+                const double wm = w * m;
+                Smm = fma(wm, m, Smm);
+                Smr = fma(wm, rp, Smr);
+                if constexpr (L > 1) {
+#pragma unroll
+                    for (int j = 0; j < L - 1; ++j) {
+                        const double Tj = s_ep[(j + 2) * N + ei];
+                        Smt[j] = fma(wm, Tj, Smt[j]);
+                        if constexpr (PHYS) {
+                            const double wT = w * Tj;
+                            Str[j] = fma(wT, rp, Str[j]);
+#pragma unroll
+                            for (int q = 0; q <= j; ++q)
+                                Stt[j * LT + q] = fma(wT, s_ep[(q + 2) * N + ei], Stt[j * LT + q]);
+                        }
+                    }
+                }
+                if constexpr (PHYS) Srr = fma(w * rp, rp, Srr);
+            }
+            if constexpr (PHYS) {
+                int ex;
+                prod = frexp(prod, &ex);
+                pexp += ex;
+            }
+        }
+        Smm = jk_cov_sum(Smm);
+        Smr = jk_cov_sum(Smr);
+#pragma unroll
+        for (int j = 0; j < L - 1; ++j) Smt[j] = jk_cov_sum(Smt[j]);
+        if constexpr (PHYS) {
+            Srr = jk_cov_sum(Srr);
+#pragma unroll
+            for (int j = 0; j < L - 1; ++j) {
+                Str[j] = jk_cov_sum(Str[j]);
+#pragma unroll
+                for (int q = 0; q <= j; ++q) Stt[j * LT + q] = jk_cov_sum(Stt[j * LT + q]);
+            }
+            // mantissas in [1/2, 1): four of them stay far inside the range
+            prod *= __shfl_xor(prod, 16, 64);
+            prod *= __shfl_xor(prod, 32, 64);
+            pexp += __shfl_xor(pexp, 16, 64);
+            pexp += __shfl_xor(pexp, 32, 64);
+        }
+        if (kq == 0 && i < n)
+            ll[i] = valid ? jk_row_finish<L, PHYS, false>(st, o.lam0, Smm, Smr, Srr, Smt, Str, Stt,
+                                                          prod, pexp, 0.0, 0.0f, s_tab, nullptr)
+                          : __builtin_nan("");
     }
 }
 
@@ -1131,10 +1167,13 @@ static hipError_t launch_lnl_cov_t(const jk_star *st, int64_t n, const double *P
                                    const void *om, const void *M0, const void *s,
                                    const int64_t *rows, double *ll, hipStream_t stream)
 {
-    const int64_t blocks = (n + JK_COV_LANES - 1) / JK_COV_LANES;
-    const size_t lds = sizeof(double) * (size_t)st->dev.n * JK_COV_LANES;
-    hipLaunchKernelGGL((k_lnl_cov<L, PHYS>), dim3((unsigned)blocks), dim3(JK_COV_LANES), lds,
-                       stream, st->dev, n, P, e, om, M0, s, rows, ll);
+    // four workgroups per compute unit, then a stride: staging Q and the tables
+    // costs as much as a few rows (2^18 rows x 40: 78 us with 4096 workgroups,
+    // 75 with 1024; 100000 x 64: 75 and 66)
+    const int64_t blocks = std::min<int64_t>((n + JK_COV_ROWS - 1) / JK_COV_ROWS, 1024);
+    const size_t lds = sizeof(double) * jk_cov_lds_doubles(st->dev.n, L);
+    hipLaunchKernelGGL((k_lnl_cov<L, PHYS>), dim3((unsigned)blocks), dim3(256), lds, stream,
+                       st->dev, n, P, e, om, M0, s, rows, ll);
     return hipGetLastError();
 }
 
@@ -1142,8 +1181,7 @@ static hipError_t launch_lnl_cov(const jk_star *st, int64_t n, const double *P, 
                                  const void *om, const void *M0, const void *s,
                                  const int64_t *rows, double *ll, hipStream_t stream)
 {
-    if (st->dev.n > JK_COV_NMAX || (n + JK_COV_LANES - 1) / JK_COV_LANES > 0x7fffffff)
-        return hipErrorInvalidValue;
+    if (st->dev.n > JK_COV_NMAX) return hipErrorInvalidValue;
     const bool phys = st->dev.jitter_mode == JK_JITTER_PHYSICAL;
 #define JK_CCASE(LL)                                                                           \
     case LL:                                                                                   \
@@ -3277,6 +3315,8 @@ __device__ __forceinline__ void jk_posterior_finish(const StarDev &st, int64_t i
     ll_out[i] = -0.5 * (chi0 - zz + (double)N * JK_LN_TWO_PI - sum_ln_w + lnlam + lndet);
 }
 
+#define JK_POST_LANES 64   // lanes per workgroup of the full-covariance posterior
+
 // One accepted row of star st, one lane: a, cov and lnL into slot i of the
 // outputs.  m_col: this lane's LDS column for a full-covariance star.
 __device__ __forceinline__ void jk_posterior_row(const StarDev &st, int64_t i, int64_t r,
@@ -3319,13 +3359,13 @@ __device__ __forceinline__ void jk_posterior_row(const StarDev &st, int64_t i, i
         for (int k = 0; k < N; ++k) {
             double sE, cE;
             jk_kepler_f64(jk_reduce_2pi(fma(nP, st.dt[k], -M0v)), ev, sE, cE);
-            m_col[k * JK_COV_LANES] = jk_design_f64(sE, cE, ev, sq, cw, sw, ecw);
+            m_col[k * JK_POST_LANES] = jk_design_f64(sE, cE, ev, sq, cw, sw, ecw);
         }
     }
     for (int k = 0; k < N; ++k) {
         if (st.Qt) {
             double m = 0.0;
-            for (int q = 0; q < N; ++q) m = fma(st.Qt[(size_t)k * N + q], m_col[q * JK_COV_LANES], m);
+            for (int q = 0; q < N; ++q) m = fma(st.Qt[(size_t)k * N + q], m_col[q * JK_POST_LANES], m);
             x[0] = m;
         } else {
             double sE, cE;
@@ -3516,7 +3556,7 @@ hipError_t jk_launch_linear_posterior(const jk_star *st, int64_t n, const double
         return hipGetLastError();
     }
     const int64_t blocks = (n + 63) / 64;
-    const size_t lds = sizeof(double) * (size_t)st->dev.n * JK_COV_LANES;
+    const size_t lds = sizeof(double) * (size_t)st->dev.n * JK_POST_LANES;
     hipLaunchKernelGGL(k_linear_posterior, dim3((unsigned)blocks), dim3(64), lds, stream, st->dev,
                        n, P, e, om, M0, s, rows, a_out, cov_out, ll_out);
     return hipGetLastError();
