@@ -1042,7 +1042,7 @@ int jk_settle_batch(const jk_batch *batch, int n_seg, const jk_settle_segment *s
     if (batch->jitter_mode == JK_JITTER_PHYSICAL && !s) return JK_EINVAL;
     if (current_device_inited() < 0) return JK_ENODEV;
     std::vector<SegDev> h(n_seg);
-    int64_t max_n = 1, max_nb = 1, mask_words = 0, bsum_n = 0, idx_n = 0;
+    int64_t max_n = 1, idx_n = 0;
     for (int i = 0; i < n_seg; ++i) {
         const jk_settle_segment &g = segs[i];
         if (g.n <= 0 || g.offset < 0 || g.row_begin < 0 || g.star < 0 || g.star >= batch->n_stars)
@@ -1053,19 +1053,13 @@ int jk_settle_batch(const jk_batch *batch, int n_seg, const jk_settle_segment *s
         d.n = g.n;
         d.max_keep = g.n;
         d.idx_off = idx_n;
-        d.mask_off = mask_words;
-        d.nb = jk_reject_bsum_count(g.n);
-        d.bsum_off = bsum_n;
         d.star = g.star;
         d.row0 = g.row_begin;
         u128 state = make_u128(g.state_hi, g.state_lo);
         d.inc = make_u128(g.inc_hi, g.inc_lo);
         jk_host_pcg_jump(state, d.inc, g.stream_offset + 1, &d.s_base);
         idx_n += g.n;
-        mask_words += jk_reject_mask_words(g.n);
-        bsum_n += d.nb;
         if (g.n > max_n) max_n = g.n;
-        if (d.nb > max_nb) max_nb = d.nb;
     }
     int pb = (int)((max_n + 4095) / 4096);
     if (pb > 1024) pb = 1024;
@@ -1073,26 +1067,22 @@ int jk_settle_batch(const jk_batch *batch, int n_seg, const jk_settle_segment *s
     hipStream_t st = (hipStream_t)stream;
     const size_t seg_bytes = sizeof(SegDev) * n_seg;
     const size_t seg_pad = ((seg_bytes + 255) / 256) * 256;
-    const size_t bytes = seg_pad + sizeof(double) * ((size_t)pb * n_seg + 2 * (size_t)n_seg) +
-                         sizeof(uint64_t) * mask_words +
-                         sizeof(int64_t) * (bsum_n + idx_n + 2 * (size_t)n_seg + 1);
+    const size_t bytes = seg_pad + sizeof(double) * (2 * (size_t)pb * n_seg) +
+                         sizeof(int64_t) * (idx_n + 3 * (size_t)n_seg + 1);
     char *scratch = nullptr;
     ScratchLease lease;
     if (scratch_get(st, bytes, (void **)&scratch, &lease) != hipSuccess) return JK_ENOMEM;
     SegDev *d_segs = (SegDev *)scratch;
     double *partials = (double *)(scratch + seg_pad);
-    double *lo = partials + (size_t)pb * n_seg;
-    double *llmax = lo + n_seg;
-    uint64_t *mask = (uint64_t *)(llmax + n_seg);
-    int64_t *bsum = (int64_t *)(mask + mask_words);
-    int64_t *idx = bsum + bsum_n;
+    unsigned long long *key = (unsigned long long *)(partials + 2 * (size_t)pb * n_seg);
+    int64_t *idx = (int64_t *)(key + n_seg);
     int64_t *cum = idx + idx_n;
     int64_t *count1 = cum + n_seg + 1;
     hipError_t err = hipMemcpyAsync(d_segs, h.data(), seg_bytes, hipMemcpyHostToDevice, st);
     if (err == hipSuccess)
-        err = jk_launch_settle_batch(batch, n_seg, d_segs, max_n, max_nb, partials, pb, mask, bsum,
-                                     idx, lo, llmax, cum, count1, P, e, omega, M0, s, rows,
-                                     ll_inout, bound_inout, n_settled_out, st);
+        err = jk_launch_settle_batch(batch, n_seg, d_segs, max_n, partials, pb, idx, key, cum,
+                                     count1, P, e, omega, M0, s, rows, ll_inout, bound_inout,
+                                     n_settled_out, st);
     // The host descriptor array must outlive the queued copy.
     hipError_t err3 = hipStreamSynchronize(st);
     hipError_t err2 = scratch_put(st, scratch, lease);
@@ -1151,8 +1141,8 @@ int jk_settle_reject_batch(const jk_batch *batch, int n_seg, const jk_settle_seg
     hipStream_t st = (hipStream_t)stream;
     const size_t seg_bytes = sizeof(SegDev) * n_seg;
     const size_t seg_pad = ((seg_bytes + 255) / 256) * 256;
-    const size_t bytes = 2 * seg_pad + sizeof(double) * ((size_t)pb * n_seg + (size_t)n_seg) +
-                         2 * sizeof(uint64_t) * mask_words +
+    const size_t bytes = 2 * seg_pad + sizeof(double) * (2 * (size_t)pb * n_seg) +
+                         sizeof(uint64_t) * (mask_words + n_seg) +
                          sizeof(int64_t) * (bsum_n + idx_n + 2 * (size_t)n_seg + 1);
     char *scratch = nullptr;
     ScratchLease lease;
@@ -1160,10 +1150,9 @@ int jk_settle_reject_batch(const jk_batch *batch, int n_seg, const jk_settle_seg
     SegDev *d_settle = (SegDev *)scratch;
     SegDev *d_reject = (SegDev *)(scratch + seg_pad);
     double *partials = (double *)(scratch + 2 * seg_pad);
-    double *lo = partials + (size_t)pb * n_seg;
-    uint64_t *mask = (uint64_t *)(lo + n_seg);
-    uint64_t *open_mask = mask + mask_words;
-    int64_t *bsum = (int64_t *)(open_mask + mask_words);
+    unsigned long long *key = (unsigned long long *)(partials + 2 * (size_t)pb * n_seg);
+    uint64_t *mask = (uint64_t *)(key + n_seg);
+    int64_t *bsum = (int64_t *)(mask + mask_words);
     int64_t *idx = bsum + bsum_n;
     int64_t *cum = idx + idx_n;
     int64_t *count1 = cum + n_seg + 1;
@@ -1172,8 +1161,7 @@ int jk_settle_reject_batch(const jk_batch *batch, int n_seg, const jk_settle_seg
         err = hipMemcpyAsync(d_reject, hr.data(), seg_bytes, hipMemcpyHostToDevice, st);
     if (err == hipSuccess)
         err = jk_launch_settle_reject_batch(batch, n_seg, d_settle, d_reject, max_n, max_nb,
-                                            partials, pb, mask, open_mask, bsum, idx, lo, cum,
-                                            count1, P, e, omega, M0, s, rows, ll_inout,
+                                            partials, pb, mask, bsum, idx, key, cum, count1, P, e, omega, M0, s, rows, ll_inout,
                                             bound_inout, idx_out, n_pass_out, llmax_out,
                                             n_settled_out, st);
     // The host descriptor arrays must outlive the queued copies.
@@ -1200,7 +1188,7 @@ static int settle_new_rows(int mode, const jk_batch *batch, int n_seg,
     if (batch->jitter_mode == JK_JITTER_PHYSICAL && !s) return JK_EINVAL;
     if (current_device_inited() < 0) return JK_ENODEV;
     std::vector<SegDev> h(n_seg);
-    int64_t max_n = 1, max_nb = 1, mask_words = 0, bsum_n = 0, idx_n = 0;
+    int64_t max_n = 1, idx_n = 0;
     for (int i = 0; i < n_seg; ++i) {
         const jk_live_segment &g = segs[i];
         if (g.n < 0 || g.first < 0 || g.first > g.n || g.offset < 0 || g.row_begin < 0 ||
@@ -1214,17 +1202,11 @@ static int settle_new_rows(int mode, const jk_batch *batch, int n_seg,
         d.n = n;
         d.max_keep = n;
         d.idx_off = idx_n;
-        d.mask_off = mask_words;
-        d.nb = jk_reject_bsum_count(n) > 0 ? jk_reject_bsum_count(n) : 1;  // block 0 writes the count
-        d.bsum_off = bsum_n;
         d.star = g.star;
         d.row0 = g.row_begin + g.first;
         d.floor = g.floor;
         idx_n += n;
-        mask_words += jk_reject_mask_words(n);
-        bsum_n += d.nb;
         if (n > max_n) max_n = n;
-        if (d.nb > max_nb) max_nb = d.nb;
     }
     int pb = (int)((max_n + 4095) / 4096);
     if (pb > 1024) pb = 1024;
@@ -1232,34 +1214,28 @@ static int settle_new_rows(int mode, const jk_batch *batch, int n_seg,
     hipStream_t st = (hipStream_t)stream;
     const size_t seg_bytes = sizeof(SegDev) * n_seg;
     const size_t seg_pad = ((seg_bytes + 255) / 256) * 256;
-    const size_t bytes = seg_pad + sizeof(double) * ((size_t)pb * n_seg + (size_t)n_seg) +
-                         sizeof(uint64_t) * mask_words +
-                         sizeof(int64_t) * (bsum_n + idx_n + 2 * (size_t)n_seg + 1);
+    const size_t bytes = seg_pad + sizeof(double) * ((size_t)pb * n_seg) +
+                         sizeof(int64_t) * (idx_n + 2 * (size_t)n_seg + 1);
     char *scratch = nullptr;
     ScratchLease lease;
     if (scratch_get(st, bytes, (void **)&scratch, &lease) != hipSuccess) return JK_ENOMEM;
     SegDev *d_segs = (SegDev *)scratch;
     double *partials = (double *)(scratch + seg_pad);
-    double *lo = partials + (size_t)pb * n_seg;
-    uint64_t *mask = (uint64_t *)(lo + n_seg);
-    int64_t *bsum = (int64_t *)(mask + mask_words);
-    int64_t *idx = bsum + bsum_n;
+    int64_t *idx = (int64_t *)(partials + (size_t)pb * n_seg);
     int64_t *cum = idx + idx_n;
     int64_t *count1 = cum + n_seg + 1;
     hipError_t err = hipMemcpyAsync(d_segs, h.data(), seg_bytes, hipMemcpyHostToDevice, st);
     if (err == hipSuccess && mode == SETTLE_LIVE)
-        err = jk_launch_settle_live_batch(batch, n_seg, d_segs, max_n, max_nb, partials, pb, mask,
-                                          bsum, idx, lo, cum, P, e, omega, M0, s, rows, ll_inout,
-                                          bound_inout, margin, n_settled_out, st);
+        err = jk_launch_settle_live_batch(batch, n_seg, d_segs, max_n, partials, pb, idx, cum, P, e,
+                                          omega, M0, s, rows, ll_inout, bound_inout, margin,
+                                          n_settled_out, st);
     else if (err == hipSuccess && mode == SETTLE_TOL)
-        err = jk_launch_settle_tol_batch(batch, n_seg, d_segs, max_n, max_nb, mask, bsum, idx, cum,
-                                         P, e, omega, M0, s, rows, ll_inout, bound_inout, tol,
-                                         n_settled_out, st);
+        err = jk_launch_settle_tol_batch(batch, n_seg, d_segs, max_n, idx, cum, P, e, omega, M0, s,
+                                         rows, ll_inout, bound_inout, tol, n_settled_out, st);
     else if (err == hipSuccess)
-        err = jk_launch_settle_pruned_batch(batch, n_seg, d_segs, max_n, max_nb, partials, pb,
-                                            mask, bsum, idx, lo, cum, count1, P, e, omega, M0, s,
-                                            rows, ll_inout, bound_inout, window, margin,
-                                            n_settled_out, st);
+        err = jk_launch_settle_pruned_batch(batch, n_seg, d_segs, max_n, partials, pb, idx, cum,
+                                            count1, P, e, omega, M0, s, rows, ll_inout,
+                                            bound_inout, window, margin, n_settled_out, st);
     // The host descriptor array must outlive the queued copy.
     hipError_t err3 = hipStreamSynchronize(st);
     hipError_t err2 = scratch_put(st, scratch, lease);
@@ -1314,8 +1290,9 @@ struct jk_seg_plan {
     hipEvent_t staged;                         // the last staging copy has been read
     char *mem;                                 // device: descriptors + scratch
     SegDev *d_settle, *d_reject;
-    double *partials, *lo, *llmax;
-    uint64_t *mask, *open_mask;
+    double *partials;
+    unsigned long long *key;
+    uint64_t *mask;
     int64_t *bsum, *idx, *cum, *count1;
 };
 
@@ -1406,8 +1383,8 @@ int jk_seg_plan_create(const jk_batch *batch, int n_seg, const jk_settle_segment
     const size_t seg_bytes = sizeof(SegDev) * n_seg;
     const size_t seg_pad = ((seg_bytes + 255) / 256) * 256;
     const size_t bytes = 2 * seg_pad +
-                         sizeof(double) * ((size_t)pb * n_seg + 2 * (size_t)n_seg) +
-                         2 * sizeof(uint64_t) * mask_words +
+                         sizeof(double) * (2 * (size_t)pb * n_seg) +
+                         sizeof(uint64_t) * (mask_words + n_seg) +
                          sizeof(int64_t) * (bsum_n + idx_n + 2 * (size_t)n_seg + 1);
     if (hipMalloc((void **)&p->mem, bytes) != hipSuccess ||
         hipHostMalloc((void **)&p->pinned, 2 * seg_bytes, hipHostMallocDefault) != hipSuccess ||
@@ -1418,11 +1395,9 @@ int jk_seg_plan_create(const jk_batch *batch, int n_seg, const jk_settle_segment
     p->d_settle = (SegDev *)p->mem;
     p->d_reject = (SegDev *)(p->mem + seg_pad);
     p->partials = (double *)(p->mem + 2 * seg_pad);
-    p->lo = p->partials + (size_t)pb * n_seg;
-    p->llmax = p->lo + n_seg;
-    p->mask = (uint64_t *)(p->llmax + n_seg);
-    p->open_mask = p->mask + mask_words;
-    p->bsum = (int64_t *)(p->open_mask + mask_words);
+    p->key = (unsigned long long *)(p->partials + 2 * (size_t)pb * n_seg);
+    p->mask = (uint64_t *)(p->key + n_seg);
+    p->bsum = (int64_t *)(p->mask + mask_words);
     p->idx = p->bsum + bsum_n;
     p->cum = p->idx + idx_n;
     p->count1 = p->cum + n_seg + 1;
@@ -1466,10 +1441,9 @@ int jk_seg_plan_settle(const jk_seg_plan *p, const double *P, const double *e,
         return JK_EINVAL;
     if (p->batch->jitter_mode == JK_JITTER_PHYSICAL && !s) return JK_EINVAL;
     if (current_device_inited() < 0) return JK_ENODEV;
-    return check_hip(jk_launch_settle_batch(p->batch, p->n_seg, p->d_settle, p->max_n, p->max_nb,
-                                            p->partials, p->pb, p->mask, p->bsum, p->idx, p->lo,
-                                            p->llmax, p->cum, p->count1, P, e, omega, M0, s, rows,
-                                            ll_inout, bound_inout, n_settled_out,
+    return check_hip(jk_launch_settle_batch(p->batch, p->n_seg, p->d_settle, p->max_n, p->partials,
+                                            p->pb, p->idx, p->key, p->cum, p->count1, P, e, omega,
+                                            M0, s, rows, ll_inout, bound_inout, n_settled_out,
                                             (hipStream_t)stream));
 }
 
@@ -1486,9 +1460,8 @@ int jk_seg_plan_settle_reject(const jk_seg_plan *p, const double *P, const doubl
     if (current_device_inited() < 0) return JK_ENODEV;
     return check_hip(jk_launch_settle_reject_batch(
         p->batch, p->n_seg, p->d_settle, p->d_reject, p->max_n, p->max_nb, p->partials, p->pb,
-        p->mask, p->open_mask, p->bsum, p->idx, p->lo, p->cum, p->count1, P, e, omega, M0, s, rows,
-        ll_inout, bound_inout, idx_out, n_pass_out, llmax_out, n_settled_out,
-        (hipStream_t)stream));
+        p->mask, p->bsum, p->idx, p->key, p->cum, p->count1, P, e, omega, M0, s, rows, ll_inout,
+        bound_inout, idx_out, n_pass_out, llmax_out, n_settled_out, (hipStream_t)stream));
 }
 
 int jk_seg_plan_reject(const jk_seg_plan *p, const double *ll, int64_t *idx_out,

@@ -72,19 +72,17 @@ hipError_t jk_launch_linear_posterior(const jk_star *st, int64_t n, const double
                                       const double *s, const int64_t *rows, double *a_out,
                                       double *cov_out, double *ll_out, hipStream_t stream);
 hipError_t jk_launch_settle_tol_batch(const jk_batch *b, int n_seg, const SegDev *d_segs,
-                                      int64_t max_n, int64_t max_nb, uint64_t *mask,
-                                      int64_t *bsum, int64_t *idx, int64_t *cum, const double *P,
+                                      int64_t max_n, int64_t *idx, int64_t *cum, const double *P,
                                       const double *e, const double *om, const double *M0,
                                       const double *s, const int64_t *rows, double *ll,
                                       float *bound, float tol, int64_t *n_settled,
                                       hipStream_t stream);
 hipError_t jk_launch_settle_pruned_batch(const jk_batch *b, int n_seg, const SegDev *d_segs,
-                                         int64_t max_n, int64_t max_nb, double *partials, int pb,
-                                         uint64_t *mask, int64_t *bsum, int64_t *idx,
-                                         double *level, int64_t *cum, int64_t *count1,
-                                         const double *P, const double *e, const double *om,
-                                         const double *M0, const double *s, const int64_t *rows,
-                                         double *ll, float *bound, double window, double margin,
+                                         int64_t max_n, double *partials, int pb, int64_t *idx,
+                                         int64_t *cum, int64_t *count1, const double *P,
+                                         const double *e, const double *om, const double *M0,
+                                         const double *s, const int64_t *rows, double *ll,
+                                         float *bound, double window, double margin,
                                          int64_t *n_settled, hipStream_t stream);
 hipError_t jk_launch_debug_row(const jk_star *st, const double *row, double *MT, double *Ainv,
                                double *A, double *a, double *b, double *B, double *Binv,
@@ -137,29 +135,29 @@ hipError_t jk_launch_prior_fill(int64_t n, int64_t row0, uint64_t seed, double P
                                 float *e32, float *om32, float *M032, float *s32,
                                 hipStream_t stream);
 int jk_seg_flag_blocks(int64_t max_n);
+// partials: 2 pb n_seg values in this and the settle_reject launch (lo, then the
+// maximum of the FP64 rows).
 hipError_t jk_launch_settle_batch(const jk_batch *b, int n_seg, const SegDev *d_segs,
-                                  int64_t max_n, int64_t max_nb, double *partials, int pb,
-                                  uint64_t *mask, int64_t *bsum, int64_t *idx, double *lo,
-                                  double *llmax, int64_t *cum, int64_t *count1, const double *P,
-                                  const double *e, const double *om, const double *M0,
-                                  const double *s, const int64_t *rows, double *ll, float *bound,
-                                  int64_t *n_settled, hipStream_t stream);
+                                  int64_t max_n, double *partials, int pb, int64_t *idx,
+                                  unsigned long long *key, int64_t *cum, int64_t *count1,
+                                  const double *P, const double *e, const double *om,
+                                  const double *M0, const double *s, const int64_t *rows,
+                                  double *ll, float *bound, int64_t *n_settled,
+                                  hipStream_t stream);
 hipError_t jk_launch_settle_live_batch(const jk_batch *b, int n_seg, const SegDev *d_segs,
-                                       int64_t max_n, int64_t max_nb, double *partials, int pb,
-                                       uint64_t *mask, int64_t *bsum, int64_t *idx, double *lo,
+                                       int64_t max_n, double *partials, int pb, int64_t *idx,
                                        int64_t *cum, const double *P, const double *e,
                                        const double *om, const double *M0, const double *s,
                                        const int64_t *rows, double *ll, float *bound,
                                        double margin, int64_t *n_settled, hipStream_t stream);
 hipError_t jk_launch_settle_reject_batch(const jk_batch *b, int n_seg, const SegDev *d_settle,
                                          const SegDev *d_reject, int64_t max_n, int64_t max_nb,
-                                         double *partials, int pb, uint64_t *mask,
-                                         uint64_t *open_mask, int64_t *bsum, int64_t *idx,
-                                         double *lo, int64_t *cum, int64_t *count1,
-                                         const double *P, const double *e, const double *om,
-                                         const double *M0, const double *s, const int64_t *rows,
-                                         double *ll, float *bound, int64_t *idx_out,
-                                         int64_t *n_pass_out, double *llmax_out,
+                                         double *partials, int pb, uint64_t *mask, int64_t *bsum,
+                                         int64_t *idx, unsigned long long *key, int64_t *cum,
+                                         int64_t *count1, const double *P, const double *e,
+                                         const double *om, const double *M0, const double *s,
+                                         const int64_t *rows, double *ll, float *bound,
+                                         int64_t *idx_out, int64_t *n_pass_out, double *llmax_out,
                                          int64_t *n_settled, hipStream_t stream);
 hipError_t jk_launch_polish(const jk_star *st, int64_t n, const double *P, const double *e,
                             const double *om, const double *M0, const double *s,

@@ -562,7 +562,8 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
     float dmx = 0.0f;      // largest 1 / (1 - e cos E) (BOUND only)
     // four epochs at a time where every fourth renormalises the product and the
     // registers allow it (2^24 rows x 16 epochs 936 -> 930 us), else two
-#pragma unroll (PHYS && !MIXED && ONE ? 4 : 2)
+    constexpr int U = PHYS && !MIXED && ONE ? 4 : 2;
+#pragma unroll U
     for (int k = 0; k < N; ++k) {
         const double *__restrict__ ep = st.ep + (size_t)k * (JK_EP_T + LT0);
         const double vk = PHYS ? (REC ? ep[JK_EP_SIG2] : st.sig2[k]) + o.s2 : 0.0;
@@ -1570,16 +1571,29 @@ __global__ __launch_bounds__(256) void k_window_flags(const double *__restrict__
 
 #define JK_WORDS_PER_BLOCK 4096   // 16 words per thread
 
+// This thread's share of the set bits of a workgroup's words, its loads in
+// flight together.
+__device__ __forceinline__ int64_t jk_count_words(const uint64_t *__restrict__ mask, int64_t w0,
+                                                  int64_t nwords)
+{
+    uint64_t v[JK_WORDS_PER_BLOCK / 256];
+#pragma unroll
+    for (int q = 0; q < JK_WORDS_PER_BLOCK / 256; ++q) {
+        const int64_t w = w0 + q * 256 + threadIdx.x;
+        v[q] = w < nwords ? mask[w] : 0ull;
+    }
+    int64_t c = 0;
+#pragma unroll
+    for (int q = 0; q < JK_WORDS_PER_BLOCK / 256; ++q) c += __popcll(v[q]);
+    return c;
+}
+
 __global__ __launch_bounds__(256) void k_reject_bsum(const uint64_t *__restrict__ mask,
                                                      int64_t nwords, int64_t *__restrict__ bsum)
 {
     __shared__ int64_t red[4];
     const int64_t w0 = (int64_t)blockIdx.x * JK_WORDS_PER_BLOCK;
-    int64_t c = 0;
-    for (int k = threadIdx.x; k < JK_WORDS_PER_BLOCK; k += 256) {
-        const int64_t w = w0 + k;
-        if (w < nwords) c += __popcll(mask[w]);
-    }
+    int64_t c = jk_count_words(mask, w0, nwords);
     c = wave_sum_i64(c);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
     __syncthreads();
@@ -2295,20 +2309,21 @@ __global__ __launch_bounds__(256) void k_seg_flags(const double *__restrict__ ll
     }
 }
 
+// With add_from, add_to[segment] += add_from[segment] as well.
 __global__ __launch_bounds__(256) void k_seg_bsum(const SegDev *__restrict__ segs,
                                                   const uint64_t *__restrict__ mask,
-                                                  int64_t *__restrict__ bsum)
+                                                  int64_t *__restrict__ bsum,
+                                                  const int64_t *__restrict__ add_from = nullptr,
+                                                  int64_t *__restrict__ add_to = nullptr)
 {
     __shared__ int64_t red[4];
     const SegDev sg = segs[blockIdx.y];
+    if (add_from && blockIdx.x == 0 && threadIdx.x == 0)
+        add_to[blockIdx.y] += add_from[blockIdx.y];
     if ((int64_t)blockIdx.x >= sg.nb) return;
     const int64_t nwords = (sg.n + 63) / 64;
     const int64_t w0 = (int64_t)blockIdx.x * JK_WORDS_PER_BLOCK;
-    int64_t c = 0;
-    for (int k = threadIdx.x; k < JK_WORDS_PER_BLOCK; k += 256) {
-        const int64_t w = w0 + k;
-        if (w < nwords) c += __popcll(mask[sg.mask_off + w]);
-    }
+    int64_t c = jk_count_words(mask + sg.mask_off, w0, nwords);
     c = wave_sum_i64(c);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
     __syncthreads();
@@ -2405,10 +2420,115 @@ hipError_t jk_launch_reject_batch(const double *ll, int n_seg, const SegDev *d_s
     hipLaunchKernelGGL(k_seg_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, d_segs, llmax_out,
                        AT, DT, mask, zero_u);
     hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum);
+                       mask, bsum, nullptr, nullptr);
     hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
                        mask, bsum, idx_out, n_pass_out);
     return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Lists of rows to re-evaluate in FP64.  Their order does not matter (each row
+// is evaluated by itself and written to its own place), so the kernels that
+// pick the rows append them to the segment's list as they find them: a wave
+// gathers its rows in LDS and claims room for up to JK_APPEND_CAP of them with
+// one atomic, its workgroup for the rest.  Flag words with a block-count and an ordered compaction pass
+// took two launches and a pass over the words more (2^21 rows: 7 + 6.5 + 6 us
+// for each of four lists; 8 us this way).
+// ---------------------------------------------------------------------------
+#define JK_APPEND_CAP 512
+
+struct WaveAppend {
+    int64_t *buf;      // the wave's JK_APPEND_CAP entries of LDS
+    int n;             // entries held, the same in every lane
+};
+
+__device__ __forceinline__ void jk_append_flush(WaveAppend &w, int64_t *__restrict__ list,
+                                                int64_t *__restrict__ count)
+{
+    const int lane = threadIdx.x & 63;
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd((unsigned long long *)count, (unsigned long long)w.n);
+    base = __shfl(base, 0, 64);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int q = lane; q < w.n; q += 64) list[base + q] = w.buf[q];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    w.n = 0;
+}
+
+// Every lane of the wave: appends i where keep is set.
+__device__ __forceinline__ void jk_append(WaveAppend &w, bool keep, int64_t i,
+                                          int64_t *__restrict__ list,
+                                          int64_t *__restrict__ count)
+{
+    const uint64_t word = __ballot(keep);
+    if (word == 0) return;
+    const int lane = threadIdx.x & 63;
+    if (keep) w.buf[w.n + __popcll(word & ((1ull << lane) - 1ull))] = i;
+    w.n += __popcll(word);
+    if (w.n > JK_APPEND_CAP - 64) jk_append_flush(w, list, count);
+}
+
+// What the workgroup's four waves still hold, with one atomic for all of them
+// (an atomic per wave on the segment's one counter took 20 us for 2048 waves).
+// Every wave of the workgroup, once, at the end.
+__device__ __forceinline__ void jk_append_end(WaveAppend &w, int64_t *__restrict__ list,
+                                              int64_t *__restrict__ count)
+{
+    __shared__ int held[4];
+    __shared__ unsigned long long base;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    if (lane == 0) held[wid] = w.n;
+    __syncthreads();
+    const int total = held[0] + held[1] + held[2] + held[3];
+    if (total == 0) return;
+    if (threadIdx.x == 0)
+        base = atomicAdd((unsigned long long *)count, (unsigned long long)total);
+    __syncthreads();
+    int64_t at = (int64_t)base;
+    for (int k = 0; k < wid; ++k) at += held[k];
+    for (int q = lane; q < w.n; q += 64) list[at + q] = w.buf[q];
+}
+
+// The NaN-propagating maximum of a segment's partials, in every thread of a
+// 256-thread workgroup: each workgroup of the pass that uses it reduces the
+// (at most 1024) partials itself, which is cheaper than a launch of its own.
+__device__ __forceinline__ double jk_partials_max(const double *__restrict__ partials, int pb,
+                                                  double *red)
+{
+    double m = -INFINITY;
+    for (int i = threadIdx.x; i < pb; i += 256) m = jk_nanmax(m, partials[i]);
+    m = wave_nanmax(m);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    return jk_nanmax(jk_nanmax(red[0], red[1]), jk_nanmax(red[2], red[3]));
+}
+
+// FP64 values as unsigned integers in the same order, every NaN above all
+// numbers, 0 below: the maximum of re-evaluated rows by integer atomics.
+__device__ __forceinline__ unsigned long long jk_max_key(double v)
+{
+    if (v != v) return ~0ull;
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    return (b >> 63) ? ~b : b | (1ull << 63);
+}
+
+__device__ __forceinline__ double jk_max_of_key(unsigned long long k)
+{
+    if (k == ~0ull) return __builtin_nan("");
+    if (k == 0ull) return -INFINITY;
+    return __longlong_as_double((long long)((k >> 63) ? k & ~(1ull << 63) : ~k));
+}
+
+__device__ __forceinline__ void jk_wave_max_key(double v, bool some, unsigned long long *key)
+{
+    unsigned long long k = some ? jk_max_key(v) : 0ull;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(k, off, 64);
+        k = o > k ? o : k;
+    }
+    if ((threadIdx.x & 63) == 0 && k != 0ull) atomicMax(key, k);
 }
 
 // Segmented FP64 re-evaluation window (jk_polish_f64 per segment): flags,
@@ -2438,13 +2558,17 @@ __global__ __launch_bounds__(256) void k_seg_window_flags(const double *__restri
 
 // Padded exclusive prefix of the per-segment counts: cum[s] = sum over t < s
 // of count[t] rounded up to a multiple of 64, so that a wavefront of the
-// scatter below never straddles two segments.  One workgroup.
-__global__ __launch_bounds__(256) void k_seg_count_scan(const int64_t *__restrict__ count,
-                                                        int n_seg, int64_t *__restrict__ cum)
+// scatter below never straddles two segments.  One workgroup of 256; cum is
+// its LDS or device memory (the scatter scans up to JK_SCAN_SEGS segments
+// itself, a launch of one workgroup scans more).
+#define JK_SCAN_SEGS 64
+
+__device__ __forceinline__ void jk_count_scan(const int64_t *__restrict__ count, int n_seg,
+                                              int64_t *cum)
 {
     __shared__ int64_t wsum[4];
     const int per = (n_seg + 255) / 256;
-    const int lo = threadIdx.x * per;
+    const int lo = min((int)threadIdx.x * per, n_seg);
     const int hi = min(lo + per, n_seg);
     int64_t mine = 0;
     for (int i = lo; i < hi; ++i) mine += (count[i] + 63) & ~(int64_t)63;
@@ -2459,6 +2583,13 @@ __global__ __launch_bounds__(256) void k_seg_count_scan(const int64_t *__restric
         run += (count[i] + 63) & ~(int64_t)63;
     }
     if (threadIdx.x == 255) cum[n_seg] = run;
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void k_seg_count_scan(const int64_t *__restrict__ count,
+                                                        int n_seg, int64_t *__restrict__ cum)
+{
+    jk_count_scan(count, n_seg, cum);
 }
 
 // The segment of padded position j0: the last one that starts at or before it.
@@ -2489,8 +2620,9 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_seg_scatter_f64(const 
                                                          const SegDev *__restrict__ segs,
                                                          int n_seg,
                                                          const int64_t *__restrict__ count,
-                                                         const int64_t *__restrict__ cum,
+                                                         const int64_t *__restrict__ cum_in,
                                                          const int64_t *__restrict__ idx,
+                                                         unsigned long long *__restrict__ key,
                                                          const double *__restrict__ P,
                                                          const void *__restrict__ e_,
                                                          const void *__restrict__ om_,
@@ -2502,7 +2634,13 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_seg_scatter_f64(const 
 {
     __shared__ double2 s_tab[JK_TAB_LDS64];
     __shared__ SplitLds<L, PHYS, false> sh;
+    __shared__ int64_t s_cum[JK_SCAN_SEGS + 1];
     const int lane = threadIdx.x & 63;
+    const int64_t *cum = cum_in;
+    if (!cum_in) {
+        jk_count_scan(count, n_seg, s_cum);
+        cum = s_cum;
+    }
     const int64_t total_waves = cum[n_seg] >> 6;
     if (total_waves <= JK_SPLIT_SCATTER_WAVES) {
         // Few rows: each 64 positions over 64 / R workgroups, a row's epochs
@@ -2528,6 +2666,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_seg_scatter_f64(const 
                 ll[sg.off + p] = v;
                 if (bound) bound[sg.off + p] = 0.0f;
             }
+            if (key && sl < 64) jk_wave_max_key(v, some && sl < R, key + sidx);
         }
         return;
     }
@@ -2539,46 +2678,56 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_seg_scatter_f64(const 
         const int sidx = __builtin_amdgcn_readfirstlane(jk_seg_of(cum, n_seg, j0));
         const SegDev &sg = segs[sidx];
         const int64_t local = j0 - cum[sidx] + lane;
-        if (local < count[sidx]) {
+        const bool some = local < count[sidx];
+        double v = 0.0;
+        if (some) {
             const int64_t p = idx[sg.idx_off + local];
             const int64_t q = sg.row0 + p;
             const int64_t r = rows ? rows[q] : q;
-            ll[sg.off + p] = jk_lnl_row<L, PHYS, false>(stars[sg.star], r, P, e_, om_, M0_, s_, s_tab);
+            v = jk_lnl_row<L, PHYS, false>(stars[sg.star], r, P, e_, om_, M0_, s_, s_tab);
+            ll[sg.off + p] = v;
             if (bound) bound[sg.off + p] = 0.0f;
         }
+        if (key) jk_wave_max_key(v, some, key + sidx);
     }
 }
 
 template <int L, bool PHYS>
 static void launch_seg_scatter_t(const jk_batch *b, int n_seg, const SegDev *d_segs,
                                  const int64_t *count, const int64_t *cum, const int64_t *idx,
-                                 int gx, const double *P, const void *e, const void *om,
-                                 const void *M0, const void *s, const int64_t *rows, double *ll,
-                                 float *bound, hipStream_t stream)
+                                 unsigned long long *key, int gx, const double *P, const void *e,
+                                 const void *om, const void *M0, const void *s,
+                                 const int64_t *rows, double *ll, float *bound,
+                                 hipStream_t stream)
 {
     hipLaunchKernelGGL((k_seg_scatter_f64<L, PHYS>), dim3(gx), dim3(256), 0, stream, b->d_stars,
-                       d_segs, n_seg, count, cum, idx, P, e, om, M0, s, rows, ll, bound);
+                       d_segs, n_seg, count, cum, idx, key, P, e, om, M0, s, rows, ll, bound);
 }
 
-// FP64 re-evaluation of every segment's compacted list idx (counts in count)
-// as one flat launch; bound entries of re-evaluated rows are set to zero.
+// FP64 re-evaluation of every segment's list idx (counts in count) as one flat
+// launch; bound entries of re-evaluated rows are set to zero, and key (if
+// given) receives each segment's maximum over them (jk_max_key).
 static hipError_t launch_seg_scatter(const jk_batch *b, int n_seg, const SegDev *d_segs,
                                      const int64_t *count, int64_t *cum, const int64_t *idx,
                                      const double *P, const double *e, const double *om,
                                      const double *M0, const double *s, const int64_t *rows,
-                                     double *ll, float *bound, hipStream_t stream)
+                                     double *ll, float *bound, hipStream_t stream,
+                                     unsigned long long *key = nullptr)
 {
-    hipLaunchKernelGGL(k_seg_count_scan, dim3(1), dim3(256), 0, stream, count, n_seg, cum);
+    if (n_seg > JK_SCAN_SEGS)
+        hipLaunchKernelGGL(k_seg_count_scan, dim3(1), dim3(256), 0, stream, count, n_seg, cum);
+    else
+        cum = nullptr;
     const int gx = 2048;
     const bool phys = b->jitter_mode == JK_JITTER_PHYSICAL;
 #define JK_SCASE2(LL)                                                                             \
     case LL:                                                                                      \
         if (phys)                                                                                 \
-            launch_seg_scatter_t<LL, true>(b, n_seg, d_segs, count, cum, idx, gx, P, e, om, M0, s, \
-                                           rows, ll, bound, stream);                              \
+            launch_seg_scatter_t<LL, true>(b, n_seg, d_segs, count, cum, idx, key, gx, P, e, om,   \
+                                           M0, s, rows, ll, bound, stream);                       \
         else                                                                                      \
-            launch_seg_scatter_t<LL, false>(b, n_seg, d_segs, count, cum, idx, gx, P, e, om, M0,   \
-                                            s, rows, ll, bound, stream);                          \
+            launch_seg_scatter_t<LL, false>(b, n_seg, d_segs, count, cum, idx, key, gx, P, e, om,  \
+                                            M0, s, rows, ll, bound, stream);                      \
         break;
     switch (b->L) {
         JK_SCASE2(1)
@@ -2612,7 +2761,7 @@ hipError_t jk_launch_polish_batch(const jk_batch *b, int n_seg, const SegDev *d_
     hipLaunchKernelGGL(k_seg_window_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, d_segs, llmax,
                        window, mask);
     hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum);
+                       mask, bsum, nullptr, nullptr);
     hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
                        mask, bsum, idx, n_polished);
     return launch_seg_scatter(b, n_seg, d_segs, n_polished, cum, idx, P, e, om, M0, s, rows, ll,
@@ -2635,26 +2784,60 @@ hipError_t jk_launch_polish_batch(const jk_batch *b, int n_seg, const SegDev *d_
 // with every row's FP64 likelihood, and every row within 40 of mx is within
 // 1e-3 of its FP64 lnL.
 // ---------------------------------------------------------------------------
+// lo = max(ll - b) over the rows that bound the maximum from below (b >= 0), in
+// partials, and (partials2 given) the maximum over the rows no settling
+// re-evaluates (b = 0) in partials2.  The first workgroup of a segment clears
+// the counters of the passes that follow.
 __global__ __launch_bounds__(256) void k_seg_lo_partial(const double *__restrict__ ll,
                                                         const float *__restrict__ bound,
                                                         const SegDev *__restrict__ segs,
-                                                        double *__restrict__ partials, int pb)
+                                                        double *__restrict__ partials,
+                                                        double *__restrict__ partials2, int pb,
+                                                        int64_t *__restrict__ count1,
+                                                        int64_t *__restrict__ count2,
+                                                        unsigned long long *__restrict__ key)
 {
-    __shared__ double red[4];
+    __shared__ double red[4], red2[4];
     const SegDev sg = segs[blockIdx.y];
-    double m = -INFINITY;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        count1[blockIdx.y] = 0;
+        if (count2) count2[blockIdx.y] = 0;
+        if (key) key[blockIdx.y] = 0ull;
+    }
+    double m = -INFINITY, m2 = -INFINITY;
     const int64_t stride = (int64_t)pb * 256;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < sg.n; i += stride) {
-        const float b = bound[sg.off + i];
-        // an upper-bound row gives no lower bound on the maximum
-        if (!(b < 0.0f)) m = jk_nanmax(m, ll[sg.off + i] - (double)b);
+    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < sg.n;
+         i0 += JK_FLAG_UNROLL * stride) {
+        float bs[JK_FLAG_UNROLL];
+        double xs[JK_FLAG_UNROLL];
+#pragma unroll
+        for (int u = 0; u < JK_FLAG_UNROLL; ++u) {
+            const int64_t i = i0 + u * stride;
+            bs[u] = i < sg.n ? bound[sg.off + i] : -1.0f;
+            xs[u] = i < sg.n ? ll[sg.off + i] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < JK_FLAG_UNROLL; ++u) {
+            // an upper-bound row gives no lower bound on the maximum
+            if (!(bs[u] < 0.0f)) {
+                m = jk_nanmax(m, xs[u] - (double)bs[u]);
+                if (!(bs[u] > 0.0f)) m2 = jk_nanmax(m2, xs[u]);
+            }
+        }
     }
     m = wave_nanmax(m);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    if (partials2) m2 = wave_nanmax(m2);
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6] = m;
+        red2[threadIdx.x >> 6] = m2;
+    }
     __syncthreads();
-    if (threadIdx.x == 0)
-        partials[(int64_t)blockIdx.y * pb + blockIdx.x] =
-            jk_nanmax(jk_nanmax(red[0], red[1]), jk_nanmax(red[2], red[3]));
+    if (threadIdx.x == 0) {
+        const int64_t o = (int64_t)blockIdx.y * pb + blockIdx.x;
+        partials[o] = jk_nanmax(jk_nanmax(red[0], red[1]), jk_nanmax(red[2], red[3]));
+        if (partials2)
+            partials2[o] = jk_nanmax(jk_nanmax(red2[0], red2[1]), jk_nanmax(red2[2], red2[3]));
+    }
 }
 
 // Rows the settling re-evaluates besides the shell of the maximum: those that
@@ -2664,50 +2847,82 @@ __global__ __launch_bounds__(256) void k_seg_lo_partial(const double *__restrict
 #define JK_LIVE_WINDOW 40.0
 #define JK_LIVE_TOL 1e-3f
 
-__global__ __launch_bounds__(256) void k_seg_shell_flags(const double *__restrict__ ll,
-                                                         const float *__restrict__ bound,
-                                                         const SegDev *__restrict__ segs,
-                                                         const double *__restrict__ lo,
-                                                         uint64_t *__restrict__ mask)
+// The list kernels below share a frame: the segment's level from its partials,
+// then strides of the grid with the loads of JK_FLAG_UNROLL of them together.
+// ROW(x, b, i): whether row i with value x and bound b goes on the list.
+#define JK_LIST_ROWS(NEED_X, ROW)                                                              \
+    __shared__ int64_t s_buf[4][JK_APPEND_CAP];                                                \
+    WaveAppend wa{s_buf[threadIdx.x >> 6], 0};                                                 \
+    const int lane = threadIdx.x & 63;                                                         \
+    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;                                 \
+    const int64_t T = (int64_t)gridDim.x * 256;                                                \
+    int64_t *list = idx + sg.idx_off, *cnt = count + blockIdx.y;                               \
+    for (int64_t base0 = g - lane; base0 < sg.n; base0 += JK_FLAG_UNROLL * T) {                \
+        double xs[JK_FLAG_UNROLL];                                                             \
+        float bs[JK_FLAG_UNROLL];                                                              \
+        _Pragma("unroll") for (int u = 0; u < JK_FLAG_UNROLL; ++u) {                           \
+            const int64_t i = base0 + u * T + lane;                                            \
+            xs[u] = NEED_X && i < sg.n ? ll[sg.off + i] : 0.0;                                 \
+            bs[u] = i < sg.n ? bound[sg.off + i] : 0.0f;                                       \
+        }                                                                                      \
+        _Pragma("unroll") for (int u = 0; u < JK_FLAG_UNROLL; ++u) {                           \
+            const int64_t i = base0 + u * T + lane;                                            \
+            const double x = xs[u];                                                            \
+            const float b = bs[u];                                                             \
+            jk_append(wa, i < sg.n && (ROW), i, list, cnt);                                    \
+        }                                                                                      \
+    }                                                                                          \
+    jk_append_end(wa, list, cnt)
+
+__global__ __launch_bounds__(256) void k_seg_shell_list(const double *__restrict__ ll,
+                                                        const float *__restrict__ bound,
+                                                        const SegDev *__restrict__ segs,
+                                                        const double *__restrict__ partials, int pb,
+                                                        int64_t *__restrict__ count,
+                                                        int64_t *__restrict__ idx)
 {
+    __shared__ double red[4];
     const SegDev sg = segs[blockIdx.y];
-    const int lane = threadIdx.x & 63;
-    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t T = (int64_t)gridDim.x * 256;
-    if (g - lane >= sg.n) return;
-    const double l0 = lo[blockIdx.y];
-    for (int64_t base = g - lane; base < sg.n; base += T) {
-        const int64_t i = base + lane;
-        bool keep = false;
-        if (i < sg.n) {
-            const float b = bound[sg.off + i];
-            const double x = ll[sg.off + i];
-            const double hi = x + (double)b;
-            // could be the maximum; or within JK_LIVE_WINDOW of it with a
-            // bound above JK_LIVE_TOL (an upper-bound row: x bounds it from
-            // above only)
-            keep = b > 0.0f ? (!(hi < l0) || (b > JK_LIVE_TOL && !(hi < l0 - JK_LIVE_WINDOW)))
-                            : (b < 0.0f && !(x < l0 - JK_LIVE_WINDOW));
-        }
-        const uint64_t word = __ballot(keep);
-        if (lane == 0) mask[sg.mask_off + (base >> 6)] = word;
-    }
+    if ((int64_t)blockIdx.x * 256 >= sg.n) return;
+    const double l0 = jk_partials_max(partials + (int64_t)blockIdx.y * pb, pb, red);
+    // could be the maximum; or within JK_LIVE_WINDOW of it with a bound above
+    // JK_LIVE_TOL (an upper-bound row: x bounds it from above only)
+    JK_LIST_ROWS(true, b > 0.0f ? (!(x + (double)b < l0) ||
+                                   (b > JK_LIVE_TOL && !(x + (double)b < l0 - JK_LIVE_WINDOW)))
+                                : (b < 0.0f && !(x < l0 - JK_LIVE_WINDOW)));
 }
 
-__global__ __launch_bounds__(256) void k_seg_uncertain_flags(const double *__restrict__ ll,
-                                                             const float *__restrict__ bound,
-                                                             const SegDev *__restrict__ segs,
-                                                             const double *__restrict__ llmax,
-                                                             u128 AT, u128 DT,
-                                                             uint64_t *__restrict__ mask)
+// The FP64 maximum of a settled segment: over the rows that were FP64 before
+// (partials2) and those the settling re-evaluated (key).  A row left with a
+// bound lies below lo, and so does not hold it.
+__device__ __forceinline__ double jk_settled_max(const double *__restrict__ partials2, int pb,
+                                                 const unsigned long long *__restrict__ key,
+                                                 double *red)
 {
+    return jk_nanmax(jk_partials_max(partials2 + (int64_t)blockIdx.y * pb, pb, red),
+                     jk_max_of_key(key[blockIdx.y]));
+}
+
+__global__ __launch_bounds__(256) void k_seg_uncertain_list(const double *__restrict__ ll,
+                                                            const float *__restrict__ bound,
+                                                            const SegDev *__restrict__ segs,
+                                                            const double *__restrict__ partials2,
+                                                            int pb,
+                                                            const unsigned long long *__restrict__ key,
+                                                            u128 AT, u128 DT,
+                                                            int64_t *__restrict__ count,
+                                                            int64_t *__restrict__ idx)
+{
+    __shared__ double red[4];
+    __shared__ int64_t s_buf[4][JK_APPEND_CAP];
     const SegDev sg = segs[blockIdx.y];
+    if ((int64_t)blockIdx.x * 256 >= sg.n) return;
+    const double mx = jk_settled_max(partials2, pb, key, red);
+    const bool live = !(mx != mx);     // a NaN maximum rejects every row anyway
+    WaveAppend wa{s_buf[threadIdx.x >> 6], 0};
     const int lane = threadIdx.x & 63;
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t T = (int64_t)gridDim.x * 256;
-    if (g - lane >= sg.n) return;
-    const double mx = llmax[blockIdx.y];
-    const bool live = !(mx != mx);     // a NaN maximum rejects every row anyway
     u128 s = pcg_thread_start(sg.s_base, sg.inc);
     for (int64_t base = g - lane; base < sg.n; base += T) {
         const int64_t i = base + lane;
@@ -2724,10 +2939,10 @@ __global__ __launch_bounds__(256) void k_seg_uncertain_flags(const double *__res
                 keep = jk_accept(ll[sg.off + i] - mx, uu);
             }
         }
-        const uint64_t word = __ballot(keep);
-        if (lane == 0) mask[sg.mask_off + (base >> 6)] = word;
+        jk_append(wa, keep, i, idx + sg.idx_off, count + blockIdx.y);
         s = pcg_affine(s, AT, DT, sg.inc);
     }
+    jk_append_end(wa, idx + sg.idx_off, count + blockIdx.y);
 }
 
 __global__ void k_seg_add_counts(const int64_t *__restrict__ a, int64_t *__restrict__ b, int n)
@@ -2737,41 +2952,29 @@ __global__ void k_seg_add_counts(const int64_t *__restrict__ a, int64_t *__restr
 }
 
 hipError_t jk_launch_settle_batch(const jk_batch *b, int n_seg, const SegDev *d_segs,
-                                  int64_t max_n, int64_t max_nb, double *partials, int pb,
-                                  uint64_t *mask, int64_t *bsum, int64_t *idx, double *lo,
-                                  double *llmax, int64_t *cum, int64_t *count1, const double *P,
-                                  const double *e, const double *om, const double *M0,
-                                  const double *s, const int64_t *rows, double *ll, float *bound,
-                                  int64_t *n_settled, hipStream_t stream)
+                                  int64_t max_n, double *partials, int pb, int64_t *idx,
+                                  unsigned long long *key, int64_t *cum, int64_t *count1,
+                                  const double *P, const double *e, const double *om,
+                                  const double *M0, const double *s, const int64_t *rows,
+                                  double *ll, float *bound, int64_t *n_settled,
+                                  hipStream_t stream)
 {
     if (n_seg <= 0) return hipSuccess;
     const int fb = jk_seg_flag_blocks(max_n);
+    double *partials2 = partials + (size_t)pb * n_seg;
     // 1. the rows that could hold the FP64 maximum
     hipLaunchKernelGGL(k_seg_lo_partial, dim3(pb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
-                       partials, pb);
-    hipLaunchKernelGGL(k_seg_max_final, dim3(n_seg), dim3(64), 0, stream, partials, pb, lo);
-    hipLaunchKernelGGL(k_seg_shell_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
-                       lo, mask);
-    hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum);
-    hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum, idx, count1);
+                       partials, partials2, pb, count1, n_settled, key);
+    hipLaunchKernelGGL(k_seg_shell_list, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
+                       partials, pb, count1, idx);
     hipError_t err = launch_seg_scatter(b, n_seg, d_segs, count1, cum, idx, P, e, om, M0, s, rows,
-                                        ll, bound, stream);
+                                        ll, bound, stream, key);
     if (err != hipSuccess) return err;
-    // 2. the FP64 maximum
-    hipLaunchKernelGGL(k_seg_max_partial, dim3(pb, n_seg), dim3(256), 0, stream, ll, d_segs,
-                       partials, pb);
-    hipLaunchKernelGGL(k_seg_max_final, dim3(n_seg), dim3(64), 0, stream, partials, pb, llmax);
-    // 3. the rows whose decision the bound leaves open
+    // 2. the rows whose decision the bound leaves open
     u128 AT, DT;
     jk_pcg_jump_coeffs((uint64_t)fb * 256, &AT, &DT);
-    hipLaunchKernelGGL(k_seg_uncertain_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound,
-                       d_segs, llmax, AT, DT, mask);
-    hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum);
-    hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum, idx, n_settled);
+    hipLaunchKernelGGL(k_seg_uncertain_list, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound,
+                       d_segs, partials2, pb, key, AT, DT, n_settled, idx);
     err = launch_seg_scatter(b, n_seg, d_segs, n_settled, cum, idx, P, e, om, M0, s, rows, ll,
                              bound, stream);
     if (err != hipSuccess) return err;
@@ -2792,38 +2995,28 @@ hipError_t jk_launch_settle_batch(const jk_batch *b, int n_seg, const SegDev *d_
 // The maximum row itself is always re-evaluated.  A NaN in lo re-evaluates
 // every new row still in mixed precision.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_seg_live_flags(const double *__restrict__ ll,
-                                                        const float *__restrict__ bound,
-                                                        const SegDev *__restrict__ segs,
-                                                        const double *__restrict__ lo,
-                                                        double margin,
-                                                        uint64_t *__restrict__ mask)
+__global__ __launch_bounds__(256) void k_seg_live_list(const double *__restrict__ ll,
+                                                       const float *__restrict__ bound,
+                                                       const SegDev *__restrict__ segs,
+                                                       const double *__restrict__ partials, int pb,
+                                                       double margin, int64_t *__restrict__ count,
+                                                       int64_t *__restrict__ idx)
 {
+    __shared__ double red[4];
     const SegDev sg = segs[blockIdx.y];
-    const int lane = threadIdx.x & 63;
-    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t T = (int64_t)gridDim.x * 256;
-    if (g - lane >= sg.n) return;
-    const double thr = jk_nanmax(lo[blockIdx.y], sg.floor) - margin;
-    for (int64_t base = g - lane; base < sg.n; base += T) {
-        const int64_t i = base + lane;
-        bool keep = false;
-        if (i < sg.n) {
-            const float b = bound[sg.off + i];
-            // an upper-bound row (b < 0): its value bounds lnL from above
-            keep = b != 0.0f && !(ll[sg.off + i] + (double)fmaxf(b, 0.0f) < thr);
-        }
-        const uint64_t word = __ballot(keep);
-        if (lane == 0) mask[sg.mask_off + (base >> 6)] = word;
-    }
+    if ((int64_t)blockIdx.x * 256 >= sg.n) return;
+    const double lo = jk_partials_max(partials + (int64_t)blockIdx.y * pb, pb, red);
+    const double thr = jk_nanmax(lo, sg.floor) - margin;
+    // an upper-bound row (b < 0): its value bounds lnL from above
+    JK_LIST_ROWS(true, b != 0.0f && !(x + (double)fmaxf(b, 0.0f) < thr));
 }
 
 // ---------------------------------------------------------------------------
 // Settling and rejection in one sequence (jk_settle_reject_batch): after the
 // rows that could hold the maximum are settled and the FP64 maximum found
-// (steps 1-2 of jk_settle_batch), one pass draws every row's uniform once
-// and decides it -- directly where the bound leaves no doubt, else flags it
-// open.  The open rows (a few per million) are re-evaluated in FP64 and
+// (step 1 of jk_settle_batch), one pass draws every row's uniform once
+// and decides it -- directly where the bound leaves no doubt, else puts it on
+// the list of open rows.  The open rows (a few per million) are re-evaluated in FP64 and
 // their decisions set from a uniform jumped to their index.  The accepted
 // set is the one jk_settle_batch + jk_reject_batch give, with one pass over
 // the rows and one PCG64 stream fewer.
@@ -2831,17 +3024,23 @@ __global__ __launch_bounds__(256) void k_seg_live_flags(const double *__restrict
 __global__ __launch_bounds__(256) void k_seg_decide(const double *__restrict__ ll,
                                                     const float *__restrict__ bound,
                                                     const SegDev *__restrict__ segs,
-                                                    const double *__restrict__ llmax,
-                                                    u128 AT, u128 DT,
+                                                    const double *__restrict__ partials2, int pb,
+                                                    const unsigned long long *__restrict__ key,
+                                                    u128 AT, u128 DT, double *__restrict__ llmax,
                                                     uint64_t *__restrict__ mask,
-                                                    uint64_t *__restrict__ open_mask)
+                                                    int64_t *__restrict__ count,
+                                                    int64_t *__restrict__ idx)
 {
+    __shared__ double red[4];
+    __shared__ int64_t s_buf[4][JK_APPEND_CAP];
     const SegDev sg = segs[blockIdx.y];
+    if ((int64_t)blockIdx.x * 256 >= sg.n) return;
+    const double mx = jk_settled_max(partials2, pb, key, red);
+    if (blockIdx.x == 0 && threadIdx.x == 0) llmax[blockIdx.y] = mx;
+    WaveAppend wa{s_buf[threadIdx.x >> 6], 0};
     const int lane = threadIdx.x & 63;
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t T = (int64_t)gridDim.x * 256;
-    if (g - lane >= sg.n) return;
-    const double mx = llmax[blockIdx.y];
     u128 s = pcg_thread_start(sg.s_base, sg.inc);
     for (int64_t base0 = g - lane; base0 < sg.n; base0 += JK_FLAG_UNROLL * T) {
         // the loads of JK_FLAG_UNROLL strides first
@@ -2876,14 +3075,13 @@ __global__ __launch_bounds__(256) void k_seg_decide(const double *__restrict__ l
                     acc = jk_accept(x - mx, uu);
                 }
             }
-            const uint64_t wa = __ballot(acc), wo = __ballot(open);
-            if (lane == 0) {
-                mask[sg.mask_off + (base >> 6)] = wa;
-                open_mask[sg.mask_off + (base >> 6)] = wo;
-            }
+            const uint64_t word = __ballot(acc);
+            if (lane == 0) mask[sg.mask_off + (base >> 6)] = word;
+            jk_append(wa, open, i, idx + sg.idx_off, count + blockIdx.y);
             s = pcg_affine(s, AT, DT, sg.inc);
         }
     }
+    jk_append_end(wa, idx + sg.idx_off, count + blockIdx.y);
 }
 
 // The decisions of the open rows, now in FP64: each row's uniform from the
@@ -2910,63 +3108,47 @@ __global__ __launch_bounds__(256) void k_seg_patch(const SegDev *__restrict__ se
 
 hipError_t jk_launch_settle_reject_batch(const jk_batch *b, int n_seg, const SegDev *d_settle,
                                          const SegDev *d_reject, int64_t max_n, int64_t max_nb,
-                                         double *partials, int pb, uint64_t *mask,
-                                         uint64_t *open_mask, int64_t *bsum, int64_t *idx,
-                                         double *lo, int64_t *cum, int64_t *count1,
-                                         const double *P, const double *e, const double *om,
-                                         const double *M0, const double *s, const int64_t *rows,
-                                         double *ll, float *bound, int64_t *idx_out,
-                                         int64_t *n_pass_out, double *llmax_out,
+                                         double *partials, int pb, uint64_t *mask, int64_t *bsum,
+                                         int64_t *idx, unsigned long long *key, int64_t *cum,
+                                         int64_t *count1, const double *P, const double *e,
+                                         const double *om, const double *M0, const double *s,
+                                         const int64_t *rows, double *ll, float *bound,
+                                         int64_t *idx_out, int64_t *n_pass_out, double *llmax_out,
                                          int64_t *n_settled, hipStream_t stream)
 {
     if (n_seg <= 0) return hipSuccess;
     const int fb = jk_seg_flag_blocks(max_n);
+    double *partials2 = partials + (size_t)pb * n_seg;
     // 1. the rows that could hold the FP64 maximum, settled
     hipLaunchKernelGGL(k_seg_lo_partial, dim3(pb, n_seg), dim3(256), 0, stream, ll, bound,
-                       d_settle, partials, pb);
-    hipLaunchKernelGGL(k_seg_max_final, dim3(n_seg), dim3(64), 0, stream, partials, pb, lo);
-    hipLaunchKernelGGL(k_seg_shell_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound,
-                       d_settle, lo, mask);
-    hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_settle,
-                       mask, bsum);
-    hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream,
-                       d_settle, mask, bsum, idx, count1);
+                       d_settle, partials, partials2, pb, count1, n_settled, key);
+    hipLaunchKernelGGL(k_seg_shell_list, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound,
+                       d_settle, partials, pb, count1, idx);
     hipError_t err = launch_seg_scatter(b, n_seg, d_settle, count1, cum, idx, P, e, om, M0, s,
-                                        rows, ll, bound, stream);
+                                        rows, ll, bound, stream, key);
     if (err != hipSuccess) return err;
-    // 2. the FP64 maximum
-    hipLaunchKernelGGL(k_seg_max_partial, dim3(pb, n_seg), dim3(256), 0, stream, ll, d_settle,
-                       partials, pb);
-    hipLaunchKernelGGL(k_seg_max_final, dim3(n_seg), dim3(64), 0, stream, partials, pb,
-                       llmax_out);
-    // 3. every row decided or flagged open, one uniform each
+    // 2. every row decided against the FP64 maximum or listed as open, one
+    // uniform each
     u128 AT, DT;
     jk_pcg_jump_coeffs((uint64_t)fb * 256, &AT, &DT);
     hipLaunchKernelGGL(k_seg_decide, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_settle,
-                       llmax_out, AT, DT, mask, open_mask);
-    // 4. the open rows in FP64, then their decisions
-    hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_settle,
-                       open_mask, bsum);
-    hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream,
-                       d_settle, open_mask, bsum, idx, n_settled);
+                       partials2, pb, key, AT, DT, llmax_out, mask, n_settled, idx);
+    // 3. the open rows in FP64, then their decisions
     err = launch_seg_scatter(b, n_seg, d_settle, n_settled, cum, idx, P, e, om, M0, s, rows, ll,
                              bound, stream);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(k_seg_patch, dim3(4, n_seg), dim3(256), 0, stream, d_settle, n_settled,
                        idx, ll, llmax_out, mask);
-    // 5. the ordered compaction of the accepted rows
+    // 4. the ordered compaction of the accepted rows
     hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_reject,
-                       mask, bsum);
+                       mask, bsum, count1, n_settled);
     hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream,
                        d_reject, mask, bsum, idx_out, n_pass_out);
-    hipLaunchKernelGGL(k_seg_add_counts, dim3((n_seg + 255) / 256), dim3(256), 0, stream, count1,
-                       n_settled, n_seg);
     return hipGetLastError();
 }
 
 hipError_t jk_launch_settle_live_batch(const jk_batch *b, int n_seg, const SegDev *d_segs,
-                                       int64_t max_n, int64_t max_nb, double *partials, int pb,
-                                       uint64_t *mask, int64_t *bsum, int64_t *idx, double *lo,
+                                       int64_t max_n, double *partials, int pb, int64_t *idx,
                                        int64_t *cum, const double *P, const double *e,
                                        const double *om, const double *M0, const double *s,
                                        const int64_t *rows, double *ll, float *bound,
@@ -2975,14 +3157,9 @@ hipError_t jk_launch_settle_live_batch(const jk_batch *b, int n_seg, const SegDe
     if (n_seg <= 0) return hipSuccess;
     const int fb = jk_seg_flag_blocks(max_n);
     hipLaunchKernelGGL(k_seg_lo_partial, dim3(pb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
-                       partials, pb);
-    hipLaunchKernelGGL(k_seg_max_final, dim3(n_seg), dim3(64), 0, stream, partials, pb, lo);
-    hipLaunchKernelGGL(k_seg_live_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
-                       lo, margin, mask);
-    hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum);
-    hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum, idx, n_settled);
+                       partials, nullptr, pb, n_settled, nullptr, nullptr);
+    hipLaunchKernelGGL(k_seg_live_list, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
+                       partials, pb, margin, n_settled, idx);
     return launch_seg_scatter(b, n_seg, d_segs, n_settled, cum, idx, P, e, om, M0, s, rows, ll,
                               bound, stream);
 }
@@ -2994,30 +3171,19 @@ hipError_t jk_launch_settle_live_batch(const jk_batch *b, int n_seg, const SegDe
 // within tol of its FP64 lnL, whatever its distance from the maximum: the
 // form for lnL arrays handed to a caller.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_seg_tol_flags(const float *__restrict__ bound,
-                                                       const SegDev *__restrict__ segs, float tol,
-                                                       uint64_t *__restrict__ mask)
+__global__ __launch_bounds__(256) void k_seg_tol_list(const double *__restrict__ ll,
+                                                      const float *__restrict__ bound,
+                                                      const SegDev *__restrict__ segs, float tol,
+                                                      int64_t *__restrict__ count,
+                                                      int64_t *__restrict__ idx)
 {
     const SegDev sg = segs[blockIdx.y];
-    const int lane = threadIdx.x & 63;
-    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t T = (int64_t)gridDim.x * 256;
-    if (g - lane >= sg.n) return;
-    for (int64_t base = g - lane; base < sg.n; base += T) {
-        const int64_t i = base + lane;
-        bool keep = false;
-        if (i < sg.n) {
-            const float b = bound[sg.off + i];
-            keep = b < 0.0f || b > tol || b != b;
-        }
-        const uint64_t word = __ballot(keep);
-        if (lane == 0) mask[sg.mask_off + (base >> 6)] = word;
-    }
+    if ((int64_t)blockIdx.x * 256 >= sg.n) return;
+    JK_LIST_ROWS(false, b < 0.0f || b > tol || b != b);
 }
 
 hipError_t jk_launch_settle_tol_batch(const jk_batch *b, int n_seg, const SegDev *d_segs,
-                                      int64_t max_n, int64_t max_nb, uint64_t *mask,
-                                      int64_t *bsum, int64_t *idx, int64_t *cum, const double *P,
+                                      int64_t max_n, int64_t *idx, int64_t *cum, const double *P,
                                       const double *e, const double *om, const double *M0,
                                       const double *s, const int64_t *rows, double *ll,
                                       float *bound, float tol, int64_t *n_settled,
@@ -3025,12 +3191,10 @@ hipError_t jk_launch_settle_tol_batch(const jk_batch *b, int n_seg, const SegDev
 {
     if (n_seg <= 0) return hipSuccess;
     const int fb = jk_seg_flag_blocks(max_n);
-    hipLaunchKernelGGL(k_seg_tol_flags, dim3(fb, n_seg), dim3(256), 0, stream, bound, d_segs, tol,
-                       mask);
-    hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum);
-    hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum, idx, n_settled);
+    hipLaunchKernelGGL(k_fill_i64, dim3((n_seg + 255) / 256), dim3(256), 0, stream, n_settled,
+                       n_seg, (int64_t)0);
+    hipLaunchKernelGGL(k_seg_tol_list, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
+                       tol, n_settled, idx);
     return launch_seg_scatter(b, n_seg, d_segs, n_settled, cum, idx, P, e, om, M0, s, rows, ll,
                               bound, stream);
 }
@@ -3049,14 +3213,25 @@ hipError_t jk_launch_settle_tol_batch(const jk_batch *b, int n_seg, const SegDev
 __global__ __launch_bounds__(256) void k_seg_hi_partial(const double *__restrict__ ll,
                                                         const float *__restrict__ bound,
                                                         const SegDev *__restrict__ segs,
-                                                        double *__restrict__ partials, int pb)
+                                                        double *__restrict__ partials, int pb,
+                                                        int64_t *__restrict__ count)
 {
     __shared__ double red[4];
     const SegDev sg = segs[blockIdx.y];
+    if (blockIdx.x == 0 && threadIdx.x == 0) count[blockIdx.y] = 0;
     double m = -INFINITY;
     const int64_t stride = (int64_t)pb * 256;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < sg.n; i += stride)
-        m = jk_nanmax(m, ll[sg.off + i] + (double)fmaxf(bound[sg.off + i], 0.0f));
+    for (int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x; i0 < sg.n;
+         i0 += JK_FLAG_UNROLL * stride) {
+        double xs[JK_FLAG_UNROLL];
+#pragma unroll
+        for (int u = 0; u < JK_FLAG_UNROLL; ++u) {
+            const int64_t i = i0 + u * stride;
+            xs[u] = i < sg.n ? ll[sg.off + i] + (double)fmaxf(bound[sg.off + i], 0.0f) : -INFINITY;
+        }
+#pragma unroll
+        for (int u = 0; u < JK_FLAG_UNROLL; ++u) m = jk_nanmax(m, xs[u]);
+    }
     m = wave_nanmax(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -3065,64 +3240,45 @@ __global__ __launch_bounds__(256) void k_seg_hi_partial(const double *__restrict
             jk_nanmax(jk_nanmax(red[0], red[1]), jk_nanmax(red[2], red[3]));
 }
 
-// Upper-bound rows (b < 0) not below level[segment] - margin; every
+// Upper-bound rows (b < 0) not below the segment's level - margin; every
 // upper-bound row when the level is NaN.
-__global__ __launch_bounds__(256) void k_seg_upper_flags(const double *__restrict__ ll,
-                                                         const float *__restrict__ bound,
-                                                         const SegDev *__restrict__ segs,
-                                                         const double *__restrict__ level,
-                                                         double margin,
-                                                         uint64_t *__restrict__ mask)
+__global__ __launch_bounds__(256) void k_seg_upper_list(const double *__restrict__ ll,
+                                                        const float *__restrict__ bound,
+                                                        const SegDev *__restrict__ segs,
+                                                        const double *__restrict__ partials, int pb,
+                                                        double margin, int64_t *__restrict__ count,
+                                                        int64_t *__restrict__ idx)
 {
+    __shared__ double red[4];
     const SegDev sg = segs[blockIdx.y];
-    const int lane = threadIdx.x & 63;
-    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t T = (int64_t)gridDim.x * 256;
-    if (g - lane >= sg.n) return;
-    const double thr = level[blockIdx.y] - margin;
-    for (int64_t base = g - lane; base < sg.n; base += T) {
-        const int64_t i = base + lane;
-        bool keep = false;
-        if (i < sg.n) keep = bound[sg.off + i] < 0.0f && !(ll[sg.off + i] < thr);
-        const uint64_t word = __ballot(keep);
-        if (lane == 0) mask[sg.mask_off + (base >> 6)] = word;
-    }
+    if ((int64_t)blockIdx.x * 256 >= sg.n) return;
+    const double thr = jk_partials_max(partials + (int64_t)blockIdx.y * pb, pb, red) - margin;
+    JK_LIST_ROWS(true, b < 0.0f && !(x < thr));
 }
 
 hipError_t jk_launch_settle_pruned_batch(const jk_batch *b, int n_seg, const SegDev *d_segs,
-                                         int64_t max_n, int64_t max_nb, double *partials, int pb,
-                                         uint64_t *mask, int64_t *bsum, int64_t *idx,
-                                         double *level, int64_t *cum, int64_t *count1,
-                                         const double *P, const double *e, const double *om,
-                                         const double *M0, const double *s, const int64_t *rows,
-                                         double *ll, float *bound, double window, double margin,
+                                         int64_t max_n, double *partials, int pb, int64_t *idx,
+                                         int64_t *cum, int64_t *count1, const double *P,
+                                         const double *e, const double *om, const double *M0,
+                                         const double *s, const int64_t *rows, double *ll,
+                                         float *bound, double window, double margin,
                                          int64_t *n_settled, hipStream_t stream)
 {
     if (n_seg <= 0) return hipSuccess;
     const int fb = jk_seg_flag_blocks(max_n);
     // 1. the rows whose bound reaches the window below the upper bound on the maximum
     hipLaunchKernelGGL(k_seg_hi_partial, dim3(pb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
-                       partials, pb);
-    hipLaunchKernelGGL(k_seg_max_final, dim3(n_seg), dim3(64), 0, stream, partials, pb, level);
-    hipLaunchKernelGGL(k_seg_upper_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
-                       level, window, mask);
-    hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum);
-    hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum, idx, count1);
+                       partials, pb, count1);
+    hipLaunchKernelGGL(k_seg_upper_list, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
+                       partials, pb, window, count1, idx);
     hipError_t err = launch_seg_scatter(b, n_seg, d_segs, count1, cum, idx, P, e, om, M0, s, rows,
                                         ll, bound, stream);
     if (err != hipSuccess) return err;
     // 2. the rows whose bound reaches the margin below the lower bound on the maximum
     hipLaunchKernelGGL(k_seg_lo_partial, dim3(pb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
-                       partials, pb);
-    hipLaunchKernelGGL(k_seg_max_final, dim3(n_seg), dim3(64), 0, stream, partials, pb, level);
-    hipLaunchKernelGGL(k_seg_upper_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
-                       level, margin, mask);
-    hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum);
-    hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum, idx, n_settled);
+                       partials, nullptr, pb, n_settled, nullptr, nullptr);
+    hipLaunchKernelGGL(k_seg_upper_list, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_segs,
+                       partials, pb, margin, n_settled, idx);
     err = launch_seg_scatter(b, n_seg, d_segs, n_settled, cum, idx, P, e, om, M0, s, rows, ll,
                              bound, stream);
     if (err != hipSuccess) return err;
