@@ -60,3 +60,28 @@ def test_settled_rejection_equals_fp64(gpu, n_seg, nan_rows):
         assert np.array_equal(lm.cpu().numpy()[z], ll.cpu().numpy()[z], equal_nan=True)
     if nan_rows:
         assert np.isnan(mxw[sizes > 100]).all() and np.isfinite(mxw[sizes <= 100]).all()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025, 262145, (3 << 19) - 1, 3 << 19,
+                               (3 << 19) + 1])
+@pytest.mark.parametrize("kind", ["peaked", "flat", "nan"])
+def test_reject_dispatch_edges(gpu, n, kind):
+    """Both forms of the rejection flags around the row count where they meet,
+    against numpy, through the call that reduces the maximum and the one that
+    is given it."""
+    g = np.random.default_rng(n)
+    ll = -(g.random(n) * (1e5 if kind == "peaked" else 3.0))
+    if kind == "nan":
+        ll[n // 2] = np.nan
+    rng = np.random.default_rng(5)
+    state = D.pcg64_state(rng)
+    u = rng.uniform(size=n)
+    with np.errstate(invalid="ignore"):
+        want = np.where(np.exp(ll - ll.max()) > u)[0]
+    d = torch.as_tensor(ll, device="cuda")
+    idx, n_pass, mx = D.reject(d, state, n)
+    assert n_pass == len(want) and np.array_equal(idx, want)
+    assert np.array_equal(mx, ll.max(), equal_nan=True)
+    top = torch.as_tensor([ll.max()], dtype=torch.float64, device="cuda")
+    idx, n_pass, _ = D.reject(d, state, 100, llmax=top)
+    assert n_pass == len(want) and np.array_equal(idx, want[:100])

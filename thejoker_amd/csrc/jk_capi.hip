@@ -535,15 +535,10 @@ static int reject_impl(const double *ll, int64_t n, const double *llmax_in, uint
     double *partials = (double *)scratch;
     uint64_t *mask = (uint64_t *)(scratch + sizeof(double) * np);
     int64_t *bsum = (int64_t *)(scratch + sizeof(double) * np + sizeof(uint64_t) * nwords);
-    hipError_t err = hipSuccess;
-    const double *mx = llmax_in;
-    if (!mx) {
-        err = jk_launch_max(ll, n, partials, np, llmax_out, st);
-        mx = llmax_out;
-    }
-    if (err == hipSuccess)
-        err = jk_launch_reject(ll, n, mx, make_u128(state_hi, state_lo), make_u128(inc_hi, inc_lo),
-                               offset, max_keep, idx_out, n_pass_out, mask, bsum, st);
+    if (!llmax_in) jk_launch_max_partials(ll, n, partials, np, st);
+    hipError_t err = jk_launch_reject(ll, n, llmax_in, partials, np, llmax_out,
+                                      make_u128(state_hi, state_lo), make_u128(inc_hi, inc_lo),
+                                      offset, max_keep, idx_out, n_pass_out, mask, bsum, st);
     hipError_t err2 = scratch_put(st, scratch, lease);
     if (err != hipSuccess) return JK_EHIP;
     return check_hip(err2);

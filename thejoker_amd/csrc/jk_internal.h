@@ -59,8 +59,11 @@ hipError_t jk_launch_lnl_mixed(const jk_star *st, int64_t n, const double *P, co
 hipError_t jk_launch_max(const double *ll, int64_t n, double *partials, int n_partials,
                          double *max_out, hipStream_t stream);
 int jk_max_partials_count(int64_t n);
-hipError_t jk_launch_reject(const double *ll, int64_t n, const double *llmax, u128 state, u128 inc,
-                            uint64_t offset, int64_t max_keep, int64_t *idx_out,
+void jk_launch_max_partials(const double *ll, int64_t n, double *partials, int n_partials,
+                            hipStream_t stream);
+hipError_t jk_launch_reject(const double *ll, int64_t n, const double *llmax,
+                            const double *partials, int np, double *llmax_out, u128 state,
+                            u128 inc, uint64_t offset, int64_t max_keep, int64_t *idx_out,
                             int64_t *n_pass_out, uint64_t *mask_scratch,
                             int64_t *bsum_scratch, hipStream_t stream);
 int64_t jk_reject_mask_words(int64_t n);

@@ -1367,6 +1367,12 @@ int jk_max_partials_count(int64_t n)
     return (int)b;
 }
 
+void jk_launch_max_partials(const double *ll, int64_t n, double *partials, int n_partials,
+                            hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_max_partial, dim3(n_partials), dim3(256), 0, stream, ll, n, partials);
+}
+
 hipError_t jk_launch_max(const double *ll, int64_t n, double *partials, int n_partials,
                          double *max_out, hipStream_t stream)
 {
@@ -1447,6 +1453,72 @@ __device__ __forceinline__ bool jk_accept(double x, double u)
 // wave's words row by row instead of lane by lane.
 #define JK_REJECT_DENSE 128
 
+// The NaN-propagating maximum of an array's (a segment's) partials, in every thread of a
+// 256-thread workgroup: each workgroup of the pass that uses it reduces the
+// (at most 1024) partials itself, which is cheaper than a launch of its own.
+__device__ __forceinline__ double jk_partials_max(const double *__restrict__ partials, int pb,
+                                                  double *red)
+{
+    double m = -INFINITY;
+    for (int i = threadIdx.x; i < pb; i += 256) m = jk_nanmax(m, partials[i]);
+    m = wave_nanmax(m);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    return jk_nanmax(jk_nanmax(red[0], red[1]), jk_nanmax(red[2], red[3]));
+}
+
+// The maximum the rejection flags compare with: *llmax if given, else reduced
+// from np partials and, by the first workgroup, left in *llmax_out.
+__device__ __forceinline__ double jk_reject_max(const double *__restrict__ llmax,
+                                                const double *__restrict__ partials, int np,
+                                                double *__restrict__ llmax_out)
+{
+    __shared__ double red[4];
+    if (llmax) return *llmax;
+    const double mx = jk_partials_max(partials, np, red);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *llmax_out = mx;
+    return mx;
+}
+
+// The rejection flags row by row, four rows per lane a grid stride apart: for
+// up to JK_REJECT_ROWS_MAX rows, where one lane per 64 rows (k_reject_words)
+// leaves most of the device idle while each lane walks its own rows.  Peaked
+// / flat likelihood, this way against one lane per word: 2^12 rows 4.6 / 5.0
+// against 12 / 24 us, 2^18 7.4 / 7.4 against 16 / 28, 2^20 12 / 13 against 16
+// / 29, 2^21 19 / 20 against 17 / 36, 2^22 32 / 34 against 18 / 37.
+#define JK_REJECT_ROWS_MAX ((int64_t)3 << 19)
+
+__global__ __launch_bounds__(256) void k_reject_rows(const double *__restrict__ ll, int64_t n,
+                                                     const double *__restrict__ llmax,
+                                                     const double *__restrict__ partials, int np,
+                                                     double *__restrict__ llmax_out, u128 s_base,
+                                                     u128 inc, u128 AT, u128 DT,
+                                                     uint64_t *__restrict__ mask)
+{
+    const double mx = jk_reject_max(llmax, partials, np, llmax_out);
+    const int lane = threadIdx.x & 63;
+    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t T = (int64_t)gridDim.x * 256;
+    double xs[JK_FLAG_UNROLL];
+#pragma unroll
+    for (int u = 0; u < JK_FLAG_UNROLL; ++u) {
+        const int64_t i = g + u * T;
+        xs[u] = i < n ? ll[i] - mx : -INFINITY;
+    }
+    u128 s = pcg_thread_start(s_base, inc);
+#pragma unroll
+    for (int u = 0; u < JK_FLAG_UNROLL; ++u) {
+        const int64_t base = g - lane + u * T;     // the same for every lane of the wave
+        if (base >= n) break;
+        bool keep = false;
+        if (xs[u] >= JK_REJECT_FLOOR) keep = jk_accept(xs[u], pcg_to_double(pcg_output(s)));
+        const uint64_t word = __ballot(keep);
+        if (lane == 0) mask[base >> 6] = word;
+        if (u + 1 < JK_FLAG_UNROLL) s = pcg_affine(s, AT, DT, inc);
+    }
+}
+
 // The rejection flags with one lane per 64-row mask word: lane g owns rows
 // [64 g, 64 g + 64), so a wave owns 4096 contiguous rows.  First the wave
 // marks, with coalesced loads and one ballot per 64 rows, the rows with
@@ -1466,14 +1538,16 @@ __device__ __forceinline__ bool jk_accept(double x, double u)
 // its own 64 rows).
 __global__ __launch_bounds__(256) void k_reject_words(const double *__restrict__ ll, int64_t n,
                                                       const double *__restrict__ llmax,
+                                                      const double *__restrict__ partials, int np,
+                                                      double *__restrict__ llmax_out,
                                                       u128 s_base, u128 inc,
                                                       uint64_t *__restrict__ mask)
 {
+    const double mx = jk_reject_max(llmax, partials, np, llmax_out);
     const int t = threadIdx.x, lane = t & 63;
     const int64_t g = (int64_t)blockIdx.x * 256 + t;
     const int64_t w0 = (g - lane) * 64;          // the wave's first row
     if (w0 >= n) return;                         // the whole wave
-    const double mx = *llmax;
     const int64_t r0 = g * 64;
     // the workgroup's jump, the same for every lane: 256 lanes x 64 rows
     u128 s = s_base;
@@ -1779,16 +1853,27 @@ hipError_t jk_launch_uniform(u128 state, u128 inc, uint64_t offset, int64_t n, d
     return hipGetLastError();
 }
 
-hipError_t jk_launch_reject(const double *ll, int64_t n, const double *llmax, u128 state, u128 inc,
-                            uint64_t offset, int64_t max_keep, int64_t *idx_out,
+// llmax: the maximum, or nullptr and it is reduced from np (at most 1024)
+// partials and left in *llmax_out.
+hipError_t jk_launch_reject(const double *ll, int64_t n, const double *llmax,
+                            const double *partials, int np, double *llmax_out, u128 state,
+                            u128 inc, uint64_t offset, int64_t max_keep, int64_t *idx_out,
                             int64_t *n_pass_out, uint64_t *mask, int64_t *bsum,
                             hipStream_t stream)
 {
     const u128 s_base = h_jump(state, inc, offset + 1);
     const int64_t nwords = jk_reject_mask_words(n);
     const int64_t nb = jk_reject_bsum_count(n);
-    hipLaunchKernelGGL(k_reject_words, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, stream,
-                       ll, n, llmax, s_base, inc, mask);
+    if (n <= JK_REJECT_ROWS_MAX) {
+        const unsigned grid = (unsigned)((n + 256 * JK_FLAG_UNROLL - 1) / (256 * JK_FLAG_UNROLL));
+        u128 AT, DT;
+        jk_pcg_jump_coeffs((uint64_t)grid * 256, &AT, &DT);
+        hipLaunchKernelGGL(k_reject_rows, dim3(grid), dim3(256), 0, stream, ll, n, llmax, partials,
+                           np, llmax_out, s_base, inc, AT, DT, mask);
+    } else {
+        hipLaunchKernelGGL(k_reject_words, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0,
+                           stream, ll, n, llmax, partials, np, llmax_out, s_base, inc, mask);
+    }
     hipLaunchKernelGGL(k_reject_bsum, dim3((unsigned)nb), dim3(256), 0, stream, mask, nwords, bsum);
     hipLaunchKernelGGL(k_reject_compact, dim3((unsigned)nb), dim3(256), 0, stream, mask, nwords, bsum,
                        (int)nb, max_keep, idx_out, n_pass_out);
@@ -1817,25 +1902,30 @@ hipError_t jk_launch_lnl_reject_f64(const jk_star *st, int64_t n, const double *
     const int64_t parts = jk_lnl_partials(n, st->dev.n);
     double *partials = (double *)scratch;       // one per likelihood wave or workgroup
     double *partials2 = partials + parts;       // second level, at most 1024
+    const double *level = partials;             // at most 1024 for the rejection step
+    int64_t n_level = parts;
     uint64_t *mask = (uint64_t *)(partials2 + 1024);
     int64_t *bsum = (int64_t *)(mask + jk_reject_mask_words(n));
     hipError_t err;
     if (st->dev.Qt) {
-        // full covariance: the maximum in its own two-level pass over ll
+        // full covariance: the partial maxima in a pass over ll
         err = launch_lnl_cov(st, n, P, e, om, M0, s, rows, ll, stream);
         if (err != hipSuccess) return err;
-        err = jk_launch_max(ll, n, partials2, jk_max_partials_count(n), llmax_out, stream);
+        level = partials2;
+        n_level = jk_max_partials_count(n);
+        jk_launch_max_partials(ll, n, partials2, (int)n_level, stream);
     } else {
         err = launch_lnl_dispatch<false>(st, n, P, e, om, M0, s, rows, ll, partials, nullptr,
                                          stream);
         if (err != hipSuccess) return err;
-        // the partial maxima reduced like any array (two parallel levels)
-        err = jk_launch_max(partials, parts, partials2, jk_max_partials_count(parts), llmax_out,
-                            stream);
+        if (parts > 1024) {
+            level = partials2;
+            n_level = jk_max_partials_count(parts);
+            jk_launch_max_partials(partials, parts, partials2, (int)n_level, stream);
+        }
     }
-    if (err != hipSuccess) return err;
-    return jk_launch_reject(ll, n, llmax_out, state, inc, offset, max_keep, idx_out, n_pass_out,
-                            mask, bsum, stream);
+    return jk_launch_reject(ll, n, nullptr, level, (int)n_level, llmax_out, state, inc, offset,
+                            max_keep, idx_out, n_pass_out, mask, bsum, stream);
 }
 
 template <int L, bool PHYS>
@@ -2487,21 +2577,6 @@ __device__ __forceinline__ void jk_append_end(WaveAppend &w, int64_t *__restrict
     int64_t at = (int64_t)base;
     for (int k = 0; k < wid; ++k) at += held[k];
     for (int q = lane; q < w.n; q += 64) list[at + q] = w.buf[q];
-}
-
-// The NaN-propagating maximum of a segment's partials, in every thread of a
-// 256-thread workgroup: each workgroup of the pass that uses it reduces the
-// (at most 1024) partials itself, which is cheaper than a launch of its own.
-__device__ __forceinline__ double jk_partials_max(const double *__restrict__ partials, int pb,
-                                                  double *red)
-{
-    double m = -INFINITY;
-    for (int i = threadIdx.x; i < pb; i += 256) m = jk_nanmax(m, partials[i]);
-    m = wave_nanmax(m);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    return jk_nanmax(jk_nanmax(red[0], red[1]), jk_nanmax(red[2], red[3]));
 }
 
 // FP64 values as unsigned integers in the same order, every NaN above all
