@@ -8,8 +8,7 @@
 #include "jk_device.h"
 
 // Largest epoch count of a full-covariance star (jk_star_create_cov): the
-// likelihood keeps its eigenvector matrix in LDS, the posterior a row's design
-// column per lane.
+// likelihood and the posterior keep its eigenvector matrix in LDS.
 #define JK_COV_NMAX 64
 
 // Host mirror of one star: the StarDev block passed by value to kernels,

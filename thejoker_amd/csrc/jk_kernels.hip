@@ -1,18 +1,18 @@
 // jk_kernels.hip -- gfx950 kernels of The Joker's likelihood + rejection path.
 //
-//  k_lnl_split             the same for few rows, a row's epochs over many lanes.
 //  k_lnl<L, PHYS, MIXED>   fused per-sample marginal lnL: phase, Kepler solve,
 //                          design column, moments, L x L Cholesky, lnL.  One
 //                          lane per prior sample; the star's epoch arrays are
 //                          wave-uniform and read through scalar loads.
+//  k_lnl_split             the same for few rows, a row's epochs over many lanes.
 //  k_max_partial / final   NaN-propagating max (np.max).
-//  k_reject_words          numpy-PCG64 uniforms generated in registers for the
+//  k_reject_words / rows   numpy-PCG64 uniforms generated in registers for the
 //                          rows that can pass, exp(ll - max) > u, one 64-bit
-//                          mask word per lane.
+//                          mask word per lane (rows: four rows per lane).
 //  k_reject_bsum/compact   order-preserving compaction of the mask words.
 //  k_uniform               the raw uniforms (tests / callers).
-//  k_linear_posterior      a = G^-1 rhs and G^-1 for accepted rows (one wave
-//                          per row for diagonal-covariance stars).
+//  k_linear_posterior      a = G^-1 rhs and G^-1 for accepted rows (16
+//                          lanes per row).
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
@@ -3471,290 +3471,400 @@ hipError_t jk_launch_prior_fill(int64_t n, int64_t row0, uint64_t seed, double P
 }
 
 // ---------------------------------------------------------------------------
-// Linear-parameter posterior for a few rows (accepted samples): FP64, one
-// lane per row, runtime L <= JK_LMAX.  Lambda[0] is not clipped here
-// (fast_likelihood.pyx:519-521).
+// Linear-parameter posterior of accepted rows, FP64.  Lambda[0] is not clipped
+// here (fast_likelihood.pyx:519-521).
+//
+// Hundreds to thousands of rows of up to a few hundred epochs: the time is one
+// row's chain of dependent operations, not the arithmetic.  A group of 16
+// lanes takes a row's epochs, lane l the epochs l, l + 16, ..., with the
+// Kepler solve of the FP64 likelihood rows (LDS tables) and L at compile time,
+// so the sums stay in registers.  The lanes' sums are combined by a butterfly
+// of DPP moves that halves the number of quantities a lane holds at each step
+// (NP - 1 exchanges for NP quantities, instead of 4 NP), they go to LDS, and
+// one wave finishes the workgroup's rows, a lane per row.  The order of every
+// sum depends on the row's star only, so the one-star and the many-star
+// launches give the same bits.  16 lanes per row: at 64 a row's setup and its
+// exchanges took 200 us of 65536 rows of 6 epochs (now 22), with 2048 rows of
+// 64 epochs at 12 us (now 8.2).  Against a wave per row with the sums in
+// scratch and the library's sine and cosine, L = 3: 2048 rows of 6 epochs
+// 37 -> 6.0 us, of 64 36 -> 8.2, of 200 47 -> 15; 65536 rows of 64 epochs
+// 738 -> 42.  Full covariance (was a lane per row, the rotation from global
+// memory): 2048 rows of 64 epochs 237 -> 14 us, 65536 327 -> 112.
 // ---------------------------------------------------------------------------
-// The end of a row's linear posterior from its sums over the epochs (G lower
-// triangle, rhs, u, chi0, sum ln w): the prior added, Cholesky, cov = G^-1,
-// a = cov rhs, and the row's lnL.
-__device__ __forceinline__ void jk_posterior_finish(const StarDev &st, int64_t i, double lam0,
-                                                    double *G, double *rhs, const double *u,
-                                                    double chi0, double sum_ln_w,
+#define JK_POST_WG 256                 // threads per workgroup
+#define JK_POST_G 16                   // lanes per row (one DPP row)
+#define JK_POST_NG (JK_POST_WG / JK_POST_G)   // rows in flight per workgroup
+#define JK_POST_RPG 4                  // most rows per group: NG x 4 lanes finish
+#define JK_POST_FULL 16384             // rows that fill the chip at one per group
+
+// The quantities of a row, in order: chi0, sum ln w, rhs[L], u[L], G's lower
+// triangle by rows; padded to a power of two for the butterfly.
+template <int L>
+struct PostSums {
+    static constexpr int NQ = 2 + 2 * L + L * (L + 1) / 2;
+    static constexpr int LG = NQ <= 8 ? 3 : NQ <= 16 ? 4 : NQ <= 32 ? 5 : 6;
+    static constexpr int NP = 1 << LG;
+};
+
+// The end of a row's linear posterior from its sums over the epochs: the prior
+// added, Cholesky, cov = G^-1, a = cov rhs, and the row's lnL.
+template <int L>
+__device__ __forceinline__ void jk_posterior_finish(const StarDev &st, int64_t i, double Pv,
+                                                    double ev, const double *__restrict__ q,
+                                                    const double2 *__restrict__ ltab,
                                                     double *__restrict__ a_out,
                                                     double *__restrict__ cov_out,
                                                     double *__restrict__ ll_out)
 {
-    const int L = st.L, N = st.n;
-    double lnlam = log(lam0) + st.ln_lam_trend;
-    G[0] += 1.0 / lam0;
-    rhs[0] += st.mu0 / lam0;
-    for (int a = 1; a < L; ++a) {
-        G[a * JK_LMAX + a] += st.lam_inv[a];
-        rhs[a] += st.mu[a] * st.lam_inv[a];
+    const double lam0 = st.k_prior_mode == JK_KPRIOR_FIXED_COMPANION_MASS
+                            ? jk_k_variance(&st, Pv, ev, false)
+                            : st.lam0;
+    double G[L][L], rhs[L], u[L];
+#pragma unroll
+    for (int a = 0; a < L; ++a) {
+        rhs[a] = q[2 + a];
+        u[a] = q[2 + L + a];
+#pragma unroll
+        for (int b = 0; b <= a; ++b) G[a][b] = q[2 + 2 * L + a * (a + 1) / 2 + b];
     }
-    // Cholesky G = R R^T (lower, in place).
-    double lndet = 0.0;
+    const double il0 = 1.0 / lam0;
+    G[0][0] += il0;
+    rhs[0] = fma(st.mu0, il0, rhs[0]);
+#pragma unroll
+    for (int a = 1; a < L; ++a) {
+        G[a][a] += st.lam_inv[a];
+        rhs[a] = fma(st.mu[a], st.lam_inv[a], rhs[a]);
+    }
+    // Cholesky G = R R^T (lower, in place; the diagonal holds 1 / R_jj);
+    // lam0 det G as a mantissa and an exponent.
+    int dexp;
+    double detm = frexp(lam0, &dexp);
     bool ok = true;
-    for (int j = 0; j < L && ok; ++j) {
-        double d = G[j * JK_LMAX + j];
-        for (int k = 0; k < j; ++k) d -= G[j * JK_LMAX + k] * G[j * JK_LMAX + k];
-        if (!(d > 0.0)) { ok = false; break; }
-        d = sqrt(d);
-        G[j * JK_LMAX + j] = d;
-        lndet += 2.0 * log(d);
-        for (int q = j + 1; q < L; ++q) {
-            double v = G[q * JK_LMAX + j];
-            for (int k = 0; k < j; ++k) v -= G[q * JK_LMAX + k] * G[j * JK_LMAX + k];
-            G[q * JK_LMAX + j] = v / d;
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+        double d = G[j][j];
+#pragma unroll
+        for (int k = 0; k < j; ++k) d = fma(-G[j][k], G[j][k], d);
+        ok = ok && d > 0.0;
+        int ex;
+        detm = frexp(detm * d, &ex);
+        dexp += ex;
+        const double ri = 1.0 / sqrt(d);
+        G[j][j] = ri;
+#pragma unroll
+        for (int c = j + 1; c < L; ++c) {
+            double v = G[c][j];
+#pragma unroll
+            for (int k = 0; k < j; ++k) v = fma(-G[c][k], G[j][k], v);
+            G[c][j] = v * ri;
         }
     }
+    double *__restrict__ ao = a_out + i * L;
+    double *__restrict__ co = cov_out + i * L * L;
     if (!ok) {
-        for (int q = 0; q < L; ++q) a_out[i * L + q] = __builtin_nan("");
-        for (int q = 0; q < L * L; ++q) cov_out[i * L * L + q] = __builtin_nan("");
+        for (int c = 0; c < L; ++c) ao[c] = __builtin_nan("");
+        for (int c = 0; c < L * L; ++c) co[c] = __builtin_nan("");
         ll_out[i] = INFINITY;
         return;
     }
-    // Rinv (lower) by forward substitution, then cov = Rinv^T Rinv.
-    double Ri[JK_LMAX * JK_LMAX];
-    for (int q = 0; q < JK_LMAX * JK_LMAX; ++q) Ri[q] = 0.0;
-    for (int c = 0; c < L; ++c) {
-        for (int a = c; a < L; ++a) {
-            double v = a == c ? 1.0 : 0.0;
-            for (int k = c; k < a; ++k) v -= G[a * JK_LMAX + k] * Ri[k * JK_LMAX + c];
-            Ri[a * JK_LMAX + c] = v / G[a * JK_LMAX + a];
-        }
-    }
-    for (int a = 0; a < L; ++a)
-        for (int b = 0; b < L; ++b) {
-            double v = 0.0;
-            for (int k = (a > b ? a : b); k < L; ++k) v += Ri[k * JK_LMAX + a] * Ri[k * JK_LMAX + b];
-            cov_out[i * L * L + a * L + b] = v;
-        }
-    // z = R^-1 u for chi2; a = cov rhs.
+    // R^-1 (lower) by forward substitution, z = R^-1 u for chi2.
+    double Ri[L][L];
     double zz = 0.0;
+#pragma unroll
+    for (int c = 0; c < L; ++c) {
+        Ri[c][c] = G[c][c];
+#pragma unroll
+        for (int a = c + 1; a < L; ++a) {
+            double v = 0.0;
+#pragma unroll
+            for (int k = c; k < a; ++k) v = fma(-G[a][k], Ri[k][c], v);
+            Ri[a][c] = v * G[a][a];
+        }
+    }
+#pragma unroll
     for (int a = 0; a < L; ++a) {
         double v = 0.0;
-        for (int k = 0; k <= a; ++k) v += Ri[a * JK_LMAX + k] * u[k];
-        zz += v * v;
+#pragma unroll
+        for (int k = 0; k <= a; ++k) v = fma(Ri[a][k], u[k], v);
+        zz = fma(v, v, zz);
     }
-    for (int a = 0; a < L; ++a) {
-        double v = 0.0;
-        for (int b = 0; b < L; ++b) v += cov_out[i * L * L + a * L + b] * rhs[b];
-        a_out[i * L + a] = v;
-    }
-    ll_out[i] = -0.5 * (chi0 - zz + (double)N * JK_LN_TWO_PI - sum_ln_w + lnlam + lndet);
+    // cov = R^-T R^-1 (symmetric), a = cov rhs.
+    double am[L];
+#pragma unroll
+    for (int a = 0; a < L; ++a) am[a] = 0.0;
+#pragma unroll
+    for (int a = 0; a < L; ++a)
+#pragma unroll
+        for (int b = 0; b <= a; ++b) {
+            double v = 0.0;
+#pragma unroll
+            for (int k = a; k < L; ++k) v = fma(Ri[k][a], Ri[k][b], v);
+            co[a * L + b] = v;
+            am[a] = fma(v, rhs[b], am[a]);
+            if (b < a) {
+                co[b * L + a] = v;
+                am[b] = fma(v, rhs[a], am[b]);
+            }
+        }
+#pragma unroll
+    for (int a = 0; a < L; ++a) ao[a] = am[a];
+    const double lnd = jk_log_tab(detm, ltab) + (double)dexp * JK_LN2;
+    ll_out[i] = -0.5 * (q[0] - zz + (double)st.n * JK_LN_TWO_PI - q[1] + st.ln_lam_trend + lnd);
 }
 
-#define JK_POST_LANES 64   // lanes per workgroup of the full-covariance posterior
-
-// One accepted row of star st, one lane: a, cov and lnL into slot i of the
-// outputs.  m_col: this lane's LDS column for a full-covariance star.
-__device__ __forceinline__ void jk_posterior_row(const StarDev &st, int64_t i, int64_t r,
-                                                 const double *__restrict__ P,
-                                                 const double *__restrict__ E_,
-                                                 const double *__restrict__ OM,
-                                                 const double *__restrict__ MM,
-                                                 const double *__restrict__ S,
-                                                 double *__restrict__ a_out,
-                                                 double *__restrict__ cov_out,
-                                                 double *__restrict__ ll_out, double *m_col)
+// sin E, cos E and the design value of one epoch.
+__device__ __forceinline__ double jk_posterior_design(double dtk, double nP, double M0v, double ev,
+                                                      float ef, float omef, float a1f, double dmax,
+                                                      double sq, double cw, double sw, double ecw,
+                                                      const double2 *__restrict__ tab)
 {
-    const int L = st.L, N = st.n;
-    const double Pv = P[r], ev = E_[r], omv = OM[r], M0v = MM[r];
-    const double sv = st.jitter_mode == JK_JITTER_PHYSICAL ? S[r] : 0.0;
-    double G[JK_LMAX * JK_LMAX], rhs[JK_LMAX], u[JK_LMAX];
-    for (int q = 0; q < JK_LMAX * JK_LMAX; ++q) G[q] = 0.0;
-    for (int q = 0; q < JK_LMAX; ++q) { rhs[q] = 0.0; u[q] = 0.0; }
+    const double x = jk_reduce_2pi(fma(nP, dtk, -M0v));
+    double sE, cE;
+    if (!jk_kepler_markley_f64(x, ev, ef, omef, a1f, dmax, tab, sE, cE))
+        jk_kepler_poly_f64(x, ev, tab, sE, cE);
+    return jk_design_f64(sE, cE, ev, sq, cw, sw, ecw);
+}
 
+// v of the lane that DPP control CTRL names (all lanes active).
+template <int CTRL>
+__device__ __forceinline__ double jk_dpp(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// One step of the butterfly over v[0 .. 2 HALF): the lanes with `up` keep the
+// upper half, the others the lower, each adding its partner's partials of it;
+// a single quantity (HALF == 0) is added to the partner's.
+template <int HALF, int CTRL>
+__device__ __forceinline__ void jk_post_fold(double *v, bool up)
+{
+    if constexpr (HALF == 0) {
+        v[0] += jk_dpp<CTRL>(v[0]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < HALF; ++j) {
+            const double keep = up ? v[j + HALF] : v[j], send = up ? v[j] : v[j + HALF];
+            v[j] = keep + jk_dpp<CTRL>(send);
+        }
+    }
+}
+
+// One row's sums over the epochs by a group of JK_POST_G lanes, into q[NQ] of
+// LDS; pe = (P, e), P NaN for an invalid row.  live: false for a group with no
+// row (it only takes part in the exchanges).  COV (a full-covariance star,
+// n <= JK_COV_NMAX): the design column is computed in epoch order in m_col (n
+// doubles of LDS of this group) and rotated into the eigenbasis the star's
+// data are in, with s_Q the eigenvectors (element (k, c) of Q^T at
+// c (n | 1) + k).
+template <int L, bool COV>
+__device__ __forceinline__ void jk_posterior_sums(const StarDev &st, int64_t r,
+                                                  const double *__restrict__ P,
+                                                  const double *__restrict__ E_,
+                                                  const double *__restrict__ OM,
+                                                  const double *__restrict__ MM,
+                                                  const double *__restrict__ S,
+                                                  const double2 *__restrict__ tab, double *m_col,
+                                                  const double *s_Q, bool live, double *q, double2 *pe)
+{
+    constexpr int NQ = PostSums<L>::NQ, NP = PostSums<L>::NP, G = JK_POST_G;
+    const int lane = threadIdx.x & (G - 1);
+    const bool phys = st.jitter_mode == JK_JITTER_PHYSICAL;
+    const double Pv = P[r], ev = E_[r], omv = OM[r], M0v = MM[r];
+    const double sv = phys ? S[r] : 0.0;
     const bool valid = isfinite(Pv) && Pv != 0.0 && ev >= 0.0 && ev < 1.0 && isfinite(omv) &&
                        isfinite(M0v) && isfinite(sv);
-    if (!valid) {
-        for (int q = 0; q < L; ++q) a_out[i * L + q] = __builtin_nan("");
-        for (int q = 0; q < L * L; ++q) cov_out[i * L * L + q] = __builtin_nan("");
+    const int N = valid && live ? st.n : 0;
+    if (lane == 0 && live) *pe = make_double2(valid ? Pv : __builtin_nan(""), ev);
+    double sw, cw;
+    jk_sincos_tab_f64(omv, tab, sw, cw);
+    const double ecw = ev * cw, sq = sqrt((1.0 - ev) * (1.0 + ev));
+    const double nP = JK_TWO_PI / Pv, s2 = sv * sv;
+    // the FP32 starter's copies, as in jk_row_orbit
+    const float ef = fminf((float)ev, 0.99999994f);
+    const float omef = fmaxf((float)(1.0 - ev), 5.9604645e-08f);
+    const float a1f = JK_MARKLEY_A1N * __builtin_amdgcn_rcpf(1.0f + ef);
+    const double dmax = ev > 0.9999999 ? -1.0 : 1e-3;
+    if constexpr (COV) {
+        for (int k = lane; k < N; k += G)
+            m_col[k] = jk_posterior_design(st.dt[k], nP, M0v, ev, ef, omef, a1f, dmax, sq, cw, sw,
+                                           ecw, tab);
+        // one wave's LDS writes and reads are in order
+        __builtin_amdgcn_wave_barrier();
+        double acc[JK_COV_NMAX / G];
+#pragma unroll
+        for (int j = 0; j < JK_COV_NMAX / G; ++j) acc[j] = 0.0;
+        const int QP = N | 1;
+        for (int c = 0; c < N; ++c) {
+            const double mc = m_col[c];
+#pragma unroll
+            for (int j = 0; j < JK_COV_NMAX / G; ++j)
+                acc[j] = fma(s_Q[c * QP + min(lane + j * G, N - 1)], mc, acc[j]);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < JK_COV_NMAX / G; ++j)
+            if (lane + j * G < N) m_col[lane + j * G] = acc[j];
+        __builtin_amdgcn_wave_barrier();
+    }
+    double v[NP];
+#pragma unroll
+    for (int j = 0; j < NP; ++j) v[j] = 0.0;
+#pragma unroll 1
+    for (int k = lane; k < N; k += G) {
+        double x[L];
+        if constexpr (COV) {
+            x[0] = m_col[k];
+        } else {
+            x[0] = jk_posterior_design(st.dt[k], nP, M0v, ev, ef, omef, a1f, dmax, sq, cw, sw, ecw,
+                                       tab);
+        }
+#pragma unroll
+        for (int j = 1; j < L; ++j) x[j] = st.T[(j - 1) * N + k];
+        const double iv = st.ivar[k], yk = st.y[k];
+        const double w = phys ? iv / fma(s2, iv, 1.0) : iv;
+        const double rr = fma(-st.mu0, x[0], st.rp[k]);
+        v[0] = fma(w * rr, rr, v[0]);
+        v[1] += jk_log_tab(w, tab + JK_TAB_LOG_OFF);
+#pragma unroll
+        for (int a = 0; a < L; ++a) {
+            const double wx = w * x[a];
+            v[2 + a] = fma(wx, yk, v[2 + a]);
+            v[2 + L + a] = fma(wx, rr, v[2 + L + a]);
+#pragma unroll
+            for (int b = 0; b <= a; ++b)
+                v[2 + 2 * L + a * (a + 1) / 2 + b] = fma(wx, x[b], v[2 + 2 * L + a * (a + 1) / 2 + b]);
+        }
+    }
+    // partners: lane ^ 8 (row_ror 8), ^ 7 (half mirror), ^ 2 and ^ 1 (quad
+    // permutes), which between them reach all 16 lanes
+    jk_post_fold<NP / 2, 0x128>(v, lane & 8);
+    jk_post_fold<NP / 4, 0x141>(v, lane & 4);
+    jk_post_fold<NP / 8, 0x4e>(v, lane & 2);
+    jk_post_fold<NP / 16, 0xb1>(v, lane & 1);
+    constexpr int K = NP > G ? NP / G : 1;   // quantities a lane ends with
+    const int q0 = lane * NP / G;
+#pragma unroll
+    for (int j = 0; j < K; ++j)
+        if (q0 + j < NQ && live) q[q0 + j] = v[j];
+}
+
+// Doubles from one group's design column to the next's (full covariance).
+__host__ __device__ inline int jk_post_cov_pitch(int N, int NP)
+{
+    return N > NP ? N | 1 : NP | 1;
+}
+
+// This workgroup's rows of [i0, n), rpg per group; star(i): the row's star.
+template <int L, bool COV, typename Star>
+__device__ __forceinline__ void jk_posterior_rows(Star star, int64_t i0, int64_t n, int rpg,
+                                                  const double *__restrict__ P,
+                                                  const double *__restrict__ E_,
+                                                  const double *__restrict__ OM,
+                                                  const double *__restrict__ MM,
+                                                  const double *__restrict__ S,
+                                                  const int64_t *__restrict__ rows,
+                                                  double *__restrict__ a_out,
+                                                  double *__restrict__ cov_out,
+                                                  double *__restrict__ ll_out, double *s_m)
+{
+    constexpr int NP = PostSums<L>::NP, RWG = COV ? 1 : JK_POST_NG * JK_POST_RPG;
+    __shared__ double2 s_tab[JK_TAB_LDS64];
+    // odd pitch: the finishing lanes read one quantity of many rows at a time
+    __shared__ double s_qd[RWG * (NP + 1)];
+    __shared__ double2 s_pe[COV ? JK_POST_NG : RWG];
+    // a full-covariance star's rows (one per group): the eigenvectors, then
+    // each group's design column, which its sums then replace
+    double *s_q = s_qd;
+    int qp = NP + 1;
+    if constexpr (COV) {
+        const StarDev &st = star(0);
+        const int N = st.n, QP = N | 1;
+        s_q = s_m + N * QP;
+        qp = jk_post_cov_pitch(N, NP);
+        for (int t = threadIdx.x; t < N * N; t += JK_POST_WG)
+            s_m[(t % N) * QP + t / N] = st.Qt[t];
+    }
+    jk_stage_tab<false>(s_tab);
+    const int group = threadIdx.x / JK_POST_G;
+    const int64_t ib = i0 + (int64_t)blockIdx.x * (JK_POST_NG * rpg);
+#pragma unroll 1
+    for (int t = 0; t < rpg; ++t) {
+        const int slot = t * JK_POST_NG + group;
+        const bool live = ib + slot < n;
+        const int64_t i = live ? ib + slot : n - 1;
+        const StarDev &st = star(i);
+        jk_posterior_sums<L, COV>(st, rows ? rows[i] : i, P, E_, OM, MM, S, s_tab,
+                                  s_q + slot * qp, s_m, live,
+                                  s_q + slot * qp, s_pe + slot);
+    }
+    __syncthreads();
+    const int slot = threadIdx.x;
+    const int64_t i = ib + slot;
+    if (slot >= JK_POST_NG * rpg || i >= n) return;
+    const double2 pe = s_pe[slot];
+    if (isnan(pe.x)) {
+        for (int c = 0; c < L; ++c) a_out[i * L + c] = __builtin_nan("");
+        for (int c = 0; c < L * L; ++c) cov_out[i * L * L + c] = __builtin_nan("");
         ll_out[i] = __builtin_nan("");
         return;
     }
-    const double lam0 = st.k_prior_mode == JK_KPRIOR_FIXED_COMPANION_MASS
-                            ? jk_k_variance(&st, Pv, ev, false)
-                            : st.lam0;
-    double sw, cw;
-    sincos(omv, &sw, &cw);
-    const double ecw = ev * cw, sq = sqrt((1.0 - ev) * (1.0 + ev));
-    const double nP = JK_TWO_PI / Pv;
-    double chi0 = 0.0, sum_ln_w = 0.0;
-    double x[JK_LMAX];
-    // full covariance: the design column in epoch order, kept in this lane's
-    // LDS column (m_col), then rotated into the eigenbasis the star's data are in
-    if (st.Qt) {
-        for (int k = 0; k < N; ++k) {
-            double sE, cE;
-            jk_kepler_f64(jk_reduce_2pi(fma(nP, st.dt[k], -M0v)), ev, sE, cE);
-            m_col[k * JK_POST_LANES] = jk_design_f64(sE, cE, ev, sq, cw, sw, ecw);
-        }
-    }
-    for (int k = 0; k < N; ++k) {
-        if (st.Qt) {
-            double m = 0.0;
-            for (int q = 0; q < N; ++q) m = fma(st.Qt[(size_t)k * N + q], m_col[q * JK_POST_LANES], m);
-            x[0] = m;
-        } else {
-            double sE, cE;
-            jk_kepler_f64(jk_reduce_2pi(fma(nP, st.dt[k], -M0v)), ev, sE, cE);
-            x[0] = jk_design_f64(sE, cE, ev, sq, cw, sw, ecw);
-        }
-        for (int j = 1; j < L; ++j) x[j] = st.T[(j - 1) * N + k];
-        const double iv = st.ivar[k];
-        const double w = st.jitter_mode == JK_JITTER_PHYSICAL ? iv / fma(sv * sv, iv, 1.0) : iv;
-        double rr = st.rp[k] - st.mu0 * x[0];
-        chi0 = fma(w * rr, rr, chi0);
-        sum_ln_w += log(w);
-        for (int a = 0; a < L; ++a) {
-            const double wx = w * x[a];
-            rhs[a] = fma(wx, st.y[k], rhs[a]);
-            u[a] = fma(wx, rr, u[a]);
-            for (int b = 0; b <= a; ++b) G[a * JK_LMAX + b] = fma(wx, x[b], G[a * JK_LMAX + b]);
-        }
-    }
-    jk_posterior_finish(st, i, lam0, G, rhs, u, chi0, sum_ln_w, a_out, cov_out, ll_out);
+    jk_posterior_finish<L>(star(i), i, pe.x, pe.y, s_q + slot * qp, s_tab + JK_TAB_LOG_OFF,
+                           a_out, cov_out, ll_out);
 }
 
-// One accepted row of a diagonal-covariance star per wave: lane l takes the
-// epochs l, l + 64, ..., the 64 partial sums of each quantity are combined by
-// the same butterfly in every launch (so the one-star and the many-star
-// launches give the same bits), and lane 0 finishes the row.  A row's epochs
-// then cost one wave about N / 64 epoch steps, instead of one lane N.
-__device__ __forceinline__ double jk_wave_sum(double v)
-{
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-__device__ __forceinline__ void jk_posterior_row_wave(const StarDev &st, int64_t i, int64_t r,
-                                                      const double *__restrict__ P,
-                                                      const double *__restrict__ E_,
-                                                      const double *__restrict__ OM,
-                                                      const double *__restrict__ MM,
-                                                      const double *__restrict__ S,
-                                                      double *__restrict__ a_out,
-                                                      double *__restrict__ cov_out,
-                                                      double *__restrict__ ll_out)
-{
-    const int lane = threadIdx.x & 63;
-    const int L = st.L, N = st.n;
-    const double Pv = P[r], ev = E_[r], omv = OM[r], M0v = MM[r];
-    const double sv = st.jitter_mode == JK_JITTER_PHYSICAL ? S[r] : 0.0;
-    const bool valid = isfinite(Pv) && Pv != 0.0 && ev >= 0.0 && ev < 1.0 && isfinite(omv) &&
-                       isfinite(M0v) && isfinite(sv);
-    if (!valid) {
-        if (lane == 0) {
-            for (int q = 0; q < L; ++q) a_out[i * L + q] = __builtin_nan("");
-            for (int q = 0; q < L * L; ++q) cov_out[i * L * L + q] = __builtin_nan("");
-            ll_out[i] = __builtin_nan("");
-        }
-        return;
-    }
-    const double lam0 = st.k_prior_mode == JK_KPRIOR_FIXED_COMPANION_MASS
-                            ? jk_k_variance(&st, Pv, ev, false)
-                            : st.lam0;
-    double sw, cw;
-    sincos(omv, &sw, &cw);
-    const double ecw = ev * cw, sq = sqrt((1.0 - ev) * (1.0 + ev));
-    const double nP = JK_TWO_PI / Pv;
-    double G[JK_LMAX * JK_LMAX], rhs[JK_LMAX], u[JK_LMAX], x[JK_LMAX];
-    for (int q = 0; q < JK_LMAX * JK_LMAX; ++q) G[q] = 0.0;
-    for (int q = 0; q < JK_LMAX; ++q) { rhs[q] = 0.0; u[q] = 0.0; }
-    double chi0 = 0.0, sum_ln_w = 0.0;
-    for (int k = lane; k < N; k += 64) {
-        double sE, cE;
-        jk_kepler_f64(jk_reduce_2pi(fma(nP, st.dt[k], -M0v)), ev, sE, cE);
-        x[0] = jk_design_f64(sE, cE, ev, sq, cw, sw, ecw);
-        for (int j = 1; j < L; ++j) x[j] = st.T[(j - 1) * N + k];
-        const double iv = st.ivar[k];
-        const double w = st.jitter_mode == JK_JITTER_PHYSICAL ? iv / fma(sv * sv, iv, 1.0) : iv;
-        const double rr = st.rp[k] - st.mu0 * x[0];
-        chi0 = fma(w * rr, rr, chi0);
-        sum_ln_w += log(w);
-        for (int a = 0; a < L; ++a) {
-            const double wx = w * x[a];
-            rhs[a] = fma(wx, st.y[k], rhs[a]);
-            u[a] = fma(wx, rr, u[a]);
-            for (int b = 0; b <= a; ++b) G[a * JK_LMAX + b] = fma(wx, x[b], G[a * JK_LMAX + b]);
-        }
-    }
-    chi0 = jk_wave_sum(chi0);
-    sum_ln_w = jk_wave_sum(sum_ln_w);
-    for (int a = 0; a < L; ++a) {
-        rhs[a] = jk_wave_sum(rhs[a]);
-        u[a] = jk_wave_sum(u[a]);
-        for (int b = 0; b <= a; ++b) G[a * JK_LMAX + b] = jk_wave_sum(G[a * JK_LMAX + b]);
-    }
-    if (lane == 0)
-        jk_posterior_finish(st, i, lam0, G, rhs, u, chi0, sum_ln_w, a_out, cov_out, ll_out);
-}
-
-// Diagonal-covariance rows of one star, one wave (a 64-thread block) per row.
-__global__ __launch_bounds__(64) void k_linear_posterior_wave(const StarDev st, int64_t n,
-                                                              const double *__restrict__ P,
-                                                              const double *__restrict__ E_,
-                                                              const double *__restrict__ OM,
-                                                              const double *__restrict__ MM,
-                                                              const double *__restrict__ S,
-                                                              const int64_t *__restrict__ rows,
-                                                              double *__restrict__ a_out,
-                                                              double *__restrict__ cov_out,
-                                                              double *__restrict__ ll_out,
-                                                              int64_t i0)
-{
-    const int64_t i = i0 + blockIdx.x;
-    if (i >= n) return;
-    jk_posterior_row_wave(st, i, rows ? rows[i] : i, P, E_, OM, MM, S, a_out, cov_out, ll_out);
-}
-
-// Rows per launch of the one-wave-per-row posterior kernels (the grid's
-// blocks x 64 threads stay far inside 2^32).
-#define JK_POST_CHUNK ((int64_t)1 << 24)
-
-__global__ __launch_bounds__(64) void k_linear_posterior(const StarDev st, int64_t n,
-                                                         const double *__restrict__ P,
-                                                         const double *__restrict__ E_,
-                                                         const double *__restrict__ OM,
-                                                         const double *__restrict__ MM,
-                                                         const double *__restrict__ S,
-                                                         const int64_t *__restrict__ rows,
-                                                         double *__restrict__ a_out,
-                                                         double *__restrict__ cov_out,
-                                                         double *__restrict__ ll_out)
+template <int L, bool COV>
+__global__ __launch_bounds__(JK_POST_WG) void k_linear_posterior(
+    const StarDev st, int64_t i0, int64_t n, int rpg, const double *__restrict__ P,
+    const double *__restrict__ E_, const double *__restrict__ OM, const double *__restrict__ MM,
+    const double *__restrict__ S, const int64_t *__restrict__ rows, double *__restrict__ a_out,
+    double *__restrict__ cov_out, double *__restrict__ ll_out)
 {
     extern __shared__ double s_m[];
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    jk_posterior_row(st, i, rows ? rows[i] : i, P, E_, OM, MM, S, a_out, cov_out, ll_out,
-                     s_m + threadIdx.x);
+    jk_posterior_rows<L, COV>([&](int64_t) -> const StarDev & { return st; }, i0, n, rpg, P, E_,
+                              OM, MM, S, rows, a_out, cov_out, ll_out, s_m);
 }
 
 // Accepted rows of many stars of a table in one launch: row i belongs to
 // table entry star_idx[i] (diagonal-covariance stars only).
-__global__ __launch_bounds__(64) void k_linear_posterior_batch(const StarDev *__restrict__ stars,
-                                                               const int32_t *__restrict__ star_idx,
-                                                               int64_t n,
-                                                               const double *__restrict__ P,
-                                                               const double *__restrict__ E_,
-                                                               const double *__restrict__ OM,
-                                                               const double *__restrict__ MM,
-                                                               const double *__restrict__ S,
-                                                               const int64_t *__restrict__ rows,
-                                                               double *__restrict__ a_out,
-                                                               double *__restrict__ cov_out,
-                                                               double *__restrict__ ll_out,
-                                                               int64_t i0)
+template <int L>
+__global__ __launch_bounds__(JK_POST_WG) void k_linear_posterior_batch(
+    const StarDev *__restrict__ stars, const int32_t *__restrict__ star_idx, int64_t i0, int64_t n,
+    int rpg, const double *__restrict__ P, const double *__restrict__ E_,
+    const double *__restrict__ OM, const double *__restrict__ MM, const double *__restrict__ S,
+    const int64_t *__restrict__ rows, double *__restrict__ a_out, double *__restrict__ cov_out,
+    double *__restrict__ ll_out)
 {
-    const int64_t i = i0 + blockIdx.x;
-    if (i >= n) return;
-    jk_posterior_row_wave(stars[star_idx[i]], i, rows[i], P, E_, OM, MM, S, a_out, cov_out,
-                          ll_out);
+    jk_posterior_rows<L, false>([&](int64_t i) -> const StarDev & { return stars[star_idx[i]]; },
+                                i0, n, rpg, P, E_, OM, MM, S, rows, a_out, cov_out, ll_out,
+                                nullptr);
 }
+
+// Rows per launch of the posterior kernels (the grid's threads stay far inside
+// 2^32).
+#define JK_POST_CHUNK ((int64_t)1 << 24)
+
+// One row per group until that fills the chip, then more: a workgroup stages
+// the tables once, and its finishing wave has more lanes at work.
+static int jk_post_rpg(int64_t n)
+{
+    const int64_t r = n / JK_POST_FULL;
+    return r < 1 ? 1 : r > JK_POST_RPG ? JK_POST_RPG : (int)r;
+}
+
+#define JK_POST_SWITCH(L_, LAUNCH)                                                                 \
+    switch (L_) {                                                                                  \
+    case 1: LAUNCH(1); break;                                                                      \
+    case 2: LAUNCH(2); break;                                                                      \
+    case 3: LAUNCH(3); break;                                                                      \
+    case 4: LAUNCH(4); break;                                                                      \
+    case 5: LAUNCH(5); break;                                                                      \
+    case 6: LAUNCH(6); break;                                                                      \
+    case 7: LAUNCH(7); break;                                                                      \
+    case 8: LAUNCH(8); break;                                                                      \
+    default: return hipErrorInvalidValue;                                                          \
+    }
 
 hipError_t jk_launch_linear_posterior_batch(const jk_batch *b, int64_t n, const int32_t *star_idx,
                                             const double *P, const double *e, const double *om,
@@ -3762,12 +3872,17 @@ hipError_t jk_launch_linear_posterior_batch(const jk_batch *b, int64_t n, const 
                                             const int64_t *rows, double *a_out, double *cov_out,
                                             double *ll_out, hipStream_t stream)
 {
-    if (n <= 0) return hipSuccess;
+    const int rpg = jk_post_rpg(n), rwg = JK_POST_NG * rpg;
     for (int64_t i0 = 0; i0 < n; i0 += JK_POST_CHUNK) {
         const int64_t nb = n - i0 < JK_POST_CHUNK ? n - i0 : JK_POST_CHUNK;
-        hipLaunchKernelGGL(k_linear_posterior_batch, dim3((unsigned)nb), dim3(64), 0, stream,
-                           b->d_stars, star_idx, n, P, e, om, M0, s, rows, a_out, cov_out,
-                           ll_out, i0);
+        const dim3 grid((unsigned)((nb + rwg - 1) / rwg));
+        const int64_t end = i0 + nb;
+#define LAUNCH(LL)                                                                                 \
+    hipLaunchKernelGGL(k_linear_posterior_batch<LL>, grid, dim3(JK_POST_WG), 0, stream,    \
+                       b->d_stars, star_idx, i0, end, rpg, P, e, om, M0, s, rows, a_out, cov_out,  \
+                       ll_out)
+        JK_POST_SWITCH(b->L, LAUNCH)
+#undef LAUNCH
     }
     return hipGetLastError();
 }
@@ -3777,19 +3892,27 @@ hipError_t jk_launch_linear_posterior(const jk_star *st, int64_t n, const double
                                       const double *s, const int64_t *rows, double *a_out,
                                       double *cov_out, double *ll_out, hipStream_t stream)
 {
-    if (n <= 0) return hipSuccess;
-    if (!st->dev.Qt) {
-        for (int64_t i0 = 0; i0 < n; i0 += JK_POST_CHUNK) {
-            const int64_t nb = n - i0 < JK_POST_CHUNK ? n - i0 : JK_POST_CHUNK;
-            hipLaunchKernelGGL(k_linear_posterior_wave, dim3((unsigned)nb), dim3(64), 0, stream,
-                               st->dev, n, P, e, om, M0, s, rows, a_out, cov_out, ll_out, i0);
-        }
-        return hipGetLastError();
+    const bool cov = st->dev.Qt != nullptr;
+    const int rpg = cov ? 1 : jk_post_rpg(n), rwg = JK_POST_NG * rpg;
+    const int N = st->dev.n;
+    for (int64_t i0 = 0; i0 < n; i0 += JK_POST_CHUNK) {
+        const int64_t nb = n - i0 < JK_POST_CHUNK ? n - i0 : JK_POST_CHUNK;
+        const dim3 grid((unsigned)((nb + rwg - 1) / rwg));
+        const int64_t end = i0 + nb;
+#define LAUNCH(LL)                                                                                 \
+    if (cov)                                                                                       \
+        hipLaunchKernelGGL((k_linear_posterior<LL, true>), grid, dim3(JK_POST_WG),                 \
+                           sizeof(double) * (N * (N | 1) + JK_POST_NG * jk_post_cov_pitch(         \
+                                                                      N, PostSums<LL>::NP)),       \
+                           stream, st->dev, i0, end, rpg, P, e, om, M0, s, rows, a_out, cov_out,   \
+                           ll_out);                                                                \
+    else                                                                                           \
+        hipLaunchKernelGGL((k_linear_posterior<LL, false>), grid, dim3(JK_POST_WG), 0,     \
+                           stream, st->dev, i0, end, rpg, P, e, om, M0, s, rows, a_out, cov_out,   \
+                           ll_out)
+        JK_POST_SWITCH(st->dev.L, LAUNCH)
+#undef LAUNCH
     }
-    const int64_t blocks = (n + 63) / 64;
-    const size_t lds = sizeof(double) * (size_t)st->dev.n * JK_POST_LANES;
-    hipLaunchKernelGGL(k_linear_posterior, dim3((unsigned)blocks), dim3(64), lds, stream, st->dev,
-                       n, P, e, om, M0, s, rows, a_out, cov_out, ll_out);
     return hipGetLastError();
 }
 
