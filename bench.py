@@ -21,7 +21,7 @@ Further legs (each an object of the same line; --workload picks one):
                against the plain path's;
   batched   -- 1024 stars, M ~ U{3..64}, baselines U[200, 3000] d, half
                binaries, poly_trend = 2, 2^20 shared rows: one autotuned
-               persistent launch, mixed vs FP64 rates, errors, acceptance
+               launch, mixed vs FP64 rates, errors, acceptance
                flips after FP64 re-evaluation of the live sets;
   serving   -- Poisson arrivals at 200 stars/s, M log-uniform on [3, 200],
                2^26-row device cache, iterative_rejection_sample to 256

@@ -339,13 +339,14 @@ int jk_batch_set_star(jk_batch *batch, int slot, const jk_star *star, void *stre
  * iterative_rejection_sample (thejoker.py:259-370) uses it per request. */
 int jk_batch_set_exact(jk_batch *batch, int slot, int exact, void *stream);
 
-/* Persistent work-queue launch over device-resident work items.
+/* One launch over device-resident work items, a workgroup per item or, where
+ * the items are few, per part of an item's rows.
  * precision 0: FP64; 1: mixed (as jk_lnl_mixed).  The columns are the FP64
  * ones in both cases.  bound_out (mixed only, optional): per-row error bounds as in
  * jk_lnl_mixed, at the same offsets as ll_out.  block: threads per workgroup
- * (64, 128 or 256); grid: workgroups (0 = 8 per compute unit).  workspace:
- * NULL or 256 device bytes (the queue counter; pass one to keep the call free
- * of allocation). */
+ * (64, 128 or 256); grid: workgroups taken to fill the device (0 = 8 per
+ * compute unit): items are split while that leaves at most twice as many.
+ * workspace: not used (may be NULL); the call allocates nothing. */
 int jk_lnl_batch(const jk_batch *batch, int precision, int64_t n_items,
                  const jk_work_item *items, const double *P, const void *e, const void *omega,
                  const void *M0, const void *s, const int64_t *rows, double *ll_out,

@@ -3,7 +3,7 @@
 The reference evaluates one star at a time (TheJoker._make_joker_helper ->
 CJokerHelper, thejoker.py:87-91).  Here a set of stars with the same number
 of linear parameters is gathered into a device star table (``jk_batch``) and
-evaluated by one persistent work-queue launch over (star, row tile) items
+evaluated by one launch over (star, row tile) items
 (``jk_lnl_batch``); the rejection step of every star runs as one segmented
 launch sequence (``jk_reject_batch``), each star with its own numpy PCG64
 stream.  :func:`autotune` picks the launch shape (threads per workgroup,
@@ -64,7 +64,8 @@ SEGMENT_DTYPE = np.dtype([("offset", "<i8"), ("n", "<i8"), ("max_keep", "<i8"),
 
 
 class LaunchShape:
-    """Threads per workgroup, workgroups (0 = 8 per CU), rows per work item."""
+    """Threads per workgroup, workgroups taken to fill the device (0 = 8 per
+    CU; few items are split to reach them), rows per work item."""
 
     def __init__(self, block=256, grid=0, tile=2048):
         self.block, self.grid, self.tile = int(block), int(grid), int(tile)
@@ -763,7 +764,7 @@ class SegPlan:
 
 
 class StepGraph:
-    """One rejection-sampling step of many stars -- the persistent lnL launch
+    """One rejection-sampling step of many stars -- the lnL launch
     (with error bounds in mixed precision), the FP64 settling and the
     segmented rejection step -- captured once in a HIP graph (through
     torch.cuda.CUDAGraph) and replayed with new numpy PCG64 streams.  Nothing

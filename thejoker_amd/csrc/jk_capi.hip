@@ -35,7 +35,7 @@ void *g_noalloc_scratch[64] = {nullptr};   // device address of `scratch` per de
 // arrays: a copy on the default stream waits for every launch queued there.
 // On its own stream the upload waits for its copy only (though where the
 // runtime copies with a kernel, that kernel still needs a free compute unit,
-// which a persistent launch occupying the device does not leave).
+// which a likelihood launch that fills the device does not leave at once).
 hipStream_t g_upload_stream[64] = {nullptr};
 
 int check_hip(hipError_t e) { return e == hipSuccess ? JK_OK : JK_EHIP; }
@@ -826,7 +826,7 @@ int jk_batch_destroy(jk_batch *b)
 int jk_lnl_batch(const jk_batch *batch, int precision, int64_t n_items, const jk_work_item *items,
                  const double *P, const void *e, const void *omega, const void *M0, const void *s,
                  const int64_t *rows, double *ll_out, float *bound_out, int block, int grid,
-                 void *workspace, void *stream)
+                 void * /*workspace*/, void *stream)
 {
     if (!batch || n_items < 0 || (precision != 0 && precision != 1)) return JK_EINVAL;
     if (bound_out && precision != 1) return JK_EINVAL;
@@ -843,21 +843,15 @@ int jk_lnl_batch(const jk_batch *batch, int precision, int64_t n_items, const jk
             return JK_EHIP;
         grid = 8 * cus;
     }
-    hipStream_t st = (hipStream_t)stream;
-    void *ws = workspace;
-    if (!ws && hipMallocAsync(&ws, 256, st) != hipSuccess) return JK_ENOMEM;
-    hipError_t err = jk_launch_lnl_batch(batch, precision, n_items, items, P, e, omega, M0, s, rows,
-                                         ll_out, bound_out, block, grid, (unsigned *)ws, st);
-    hipError_t err2 = workspace ? hipSuccess : hipFreeAsync(ws, st);
-    if (err != hipSuccess) return JK_EHIP;
-    return check_hip(err2);
+    return check_hip(jk_launch_lnl_batch(batch, precision, n_items, items, P, e, omega, M0, s, rows,
+                                         ll_out, bound_out, block, grid, (hipStream_t)stream));
 }
 
 int jk_lnl_prune_batch(const jk_batch *batch, const jk_batch *probes, const double *prune,
                        int precision, int64_t n_items, const jk_work_item *items, const double *P,
                        const void *e, const void *omega, const void *M0, const void *s,
                        double *ll_out, float *bound_out, uint64_t *n_full_out, int block,
-                       int grid, void *workspace, void *stream)
+                       int grid, void * /*workspace*/, void *stream)
 {
     if (!batch || !probes || n_items < 0 || (precision != 0 && precision != 1)) return JK_EINVAL;
     if (precision == 1 && !bound_out) return JK_EINVAL;
@@ -877,16 +871,10 @@ int jk_lnl_prune_batch(const jk_batch *batch, const jk_batch *probes, const doub
             return JK_EHIP;
         grid = 8 * cus;
     }
-    hipStream_t st = (hipStream_t)stream;
-    void *ws = workspace;
-    if (!ws && hipMallocAsync(&ws, 256, st) != hipSuccess) return JK_ENOMEM;
-    hipError_t err = jk_launch_lnl_prune_batch(batch, probes, prune, precision, n_items, items, P,
+    return check_hip(jk_launch_lnl_prune_batch(batch, probes, prune, precision, n_items, items, P,
                                                e, omega, M0, s, ll_out, bound_out,
                                                (unsigned long long *)n_full_out, block, grid,
-                                               (unsigned *)ws, st);
-    hipError_t err2 = workspace ? hipSuccess : hipFreeAsync(ws, st);
-    if (err != hipSuccess) return JK_EHIP;
-    return check_hip(err2);
+                                               (hipStream_t)stream));
 }
 
 static int reject_batch_impl(const double *ll, int n_seg, const jk_segment *segs,

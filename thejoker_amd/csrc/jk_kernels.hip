@@ -1995,13 +1995,56 @@ hipError_t jk_launch_polish(const jk_star *st, int64_t n, const double *P, const
 }
 
 // ---------------------------------------------------------------------------
-// Many stars per launch: a persistent work queue.  Each workgroup takes the
-// next (star, row tile) item from a device counter, reads the star's
-// constants through scalar loads (the item index is made wave-uniform with
-// readfirstlane) and evaluates the tile one lane per row.  Every workgroup
-// exits once the counter passes n_items.
+// Many stars per launch: one workgroup per work item (star, row tile), or per
+// part of an item's rows, in the items' order; it reads the star's constants
+// through scalar loads and evaluates its rows one lane per row.  The hardware
+// dispatcher hands the entries out: a persistent grid that took them from a
+// device counter paid about 10 ns per fetch (one address, so one after
+// another: 20 us before the last of 2048 workgroups had its first item, as
+// much for the fetches that found the queue empty) and a launch to clear the
+// counter, more than staging the tables again costs.
 // ---------------------------------------------------------------------------
-__global__ void k_zero_u32(unsigned *p) { *p = 0u; }
+// Entries [first, first + gridDim.x) of a launch: each work item as 1 <<
+// lg_parts parts.
+struct WorkSplit {
+    int64_t first;
+    unsigned lg_parts;
+};
+
+// The rows [lo, hi) that entry q takes of its item's n_rows: parts of whole
+// workgroup passes.
+__device__ __forceinline__ void jk_split_item(const WorkSplit &ws, int64_t q, int n_rows, int &lo,
+                                              int &hi)
+{
+    lo = 0;
+    hi = n_rows;
+    if (ws.lg_parts) {
+        const unsigned parts = 1u << ws.lg_parts, part = (unsigned)q & (parts - 1), bd = blockDim.x;
+        const int64_t passes = (n_rows + (int64_t)bd - 1) / bd;
+        const int64_t chunk = ((passes + parts - 1) >> ws.lg_parts) * bd;
+        lo = (int)std::min<int64_t>(n_rows, part * chunk);
+        hi = (int)std::min<int64_t>(n_rows, (part + 1) * chunk);
+    }
+}
+
+// Parts per item: two, four or eight where that leaves at most 2 grid entries
+// (grid: 8 workgroups per CU unless the caller says otherwise), so that few
+// items still fill the chip and end together.  Whole items from the counter ->
+// parts from the dispatcher, 2048 rows per item: 40 items (FP64, 3 to 12
+// epochs, L = 2) 67 -> 27 us, 500 82 -> 37, 2400 155 -> 132; mixed, 3 to 64
+// epochs, L = 3: 40 items 210 -> 28, 600 268 -> 122, 8192 1425 -> 1411.  More
+// parts than that cost more than they level out: 2400 FP64 items in 8 parts
+// 240 us.  A pruned launch takes at most four: an item's survivors are
+// gathered to fill waves, and there are fewer in a smaller part (2^21 rows of
+// 100 epochs, the whole call with its rejection: 345 us whole, 337 in two,
+// 335 in four, 340 in eight).
+#define JK_ITEM_LAUNCH ((int64_t)1 << 23)   // entries per launch (x 256 threads < 2^32)
+static unsigned jk_item_parts(int64_t n_items, int grid)
+{
+    unsigned lg = 0;
+    while (lg < 3 && (n_items << (lg + 1)) <= 2 * (int64_t)grid) ++lg;
+    return lg;
+}
 
 // One row of a mixed-precision batched launch: in FP64 with error bound 0
 // for a star whose table slot is marked exact (jk_batch_set_exact; a star
@@ -2033,7 +2076,7 @@ __global__ void k_set_exact(StarDev *stars, int slot, int exact) { stars[slot].e
 template <int L, bool PHYS, bool MIXED, bool BOUND>
 __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_batch(const StarDev *__restrict__ stars,
                                                    const jk_work_item *__restrict__ items,
-                                                   int64_t n_items, unsigned *__restrict__ counter,
+                                                   WorkSplit ws,
                                                    const double *__restrict__ P,
                                                    const void *__restrict__ e_,
                                                    const void *__restrict__ om_,
@@ -2043,32 +2086,28 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_batch(const StarDe
                                                    double *__restrict__ ll,
                                                    float *__restrict__ bound)
 {
-    __shared__ unsigned s_item;
     __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
+    const int64_t q0 = ws.first + blockIdx.x;
+    const jk_work_item w = items[q0 >> ws.lg_parts];
+    int lo, hi;
+    jk_split_item(ws, q0, w.n_rows, lo, hi);
+    if (lo >= hi) return;
     jk_stage_tab<MIXED>(s_tab);
-    for (;;) {
-        if (threadIdx.x == 0) s_item = atomicAdd(counter, 1u);
-        __syncthreads();
-        const int64_t it = (int64_t)__builtin_amdgcn_readfirstlane(s_item);
-        __syncthreads();
-        if (it >= n_items) break;
-        const jk_work_item w = items[it];
-        const StarDev &st = stars[w.star];
-        for (int j = threadIdx.x; j < w.n_rows; j += blockDim.x) {
-            const int64_t q = w.row_begin + j;
-            const int64_t r = rows ? rows[q] : q;
-            if constexpr (BOUND) {
-                float b;
-                ll[w.out_offset + j] = jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
-                bound[w.out_offset + j] = b;
-            } else if constexpr (MIXED) {
-                ll[w.out_offset + j] =
-                    st.exact ? jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab)
-                             : jk_lnl_row<L, PHYS, true, false, false, false, true>(
-                                   st, r, P, e_, om_, M0_, s_, s_tab);
-            } else {
-                ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
-            }
+    const StarDev &st = stars[w.star];
+    for (int j = lo + threadIdx.x; j < hi; j += blockDim.x) {
+        const int64_t q = w.row_begin + j;
+        const int64_t r = rows ? rows[q] : q;
+        if constexpr (BOUND) {
+            float b;
+            ll[w.out_offset + j] = jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
+            bound[w.out_offset + j] = b;
+        } else if constexpr (MIXED) {
+            ll[w.out_offset + j] =
+                st.exact ? jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab)
+                         : jk_lnl_row<L, PHYS, true, false, false, false, true>(
+                               st, r, P, e_, om_, M0_, s_, s_tab);
+        } else {
+            ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
         }
     }
 }
@@ -2083,19 +2122,19 @@ template <int L, bool PHYS, bool MIXED>
 static void launch_batch_t(const jk_batch *b, int64_t n_items, const jk_work_item *items,
                            const double *P, const void *e, const void *om, const void *M0,
                            const void *s, const int64_t *rows, double *ll, float *bound,
-                           int block, int grid, unsigned *counter, hipStream_t stream)
+                           int block, int grid, hipStream_t stream)
 {
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, stream, counter);
-    if constexpr (MIXED) {
-        if (bound) {
-            hipLaunchKernelGGL((k_lnl_batch<L, PHYS, true, true>), dim3(grid), dim3(block), 0,
-                               stream, b->d_stars, items, n_items, counter, P, e, om, M0, s, rows,
-                               ll, bound);
-            return;
-        }
+    WorkSplit ws{0, jk_item_parts(n_items, grid)};
+    const int64_t entries = n_items << ws.lg_parts;
+    for (; ws.first < entries; ws.first += JK_ITEM_LAUNCH) {
+        const dim3 blocks((unsigned)std::min(entries - ws.first, JK_ITEM_LAUNCH));
+        if (MIXED && bound)
+            hipLaunchKernelGGL((k_lnl_batch<L, PHYS, MIXED, MIXED>), blocks, dim3(block), 0, stream,
+                               b->d_stars, items, ws, P, e, om, M0, s, rows, ll, bound);
+        else
+            hipLaunchKernelGGL((k_lnl_batch<L, PHYS, MIXED, false>), blocks, dim3(block), 0, stream,
+                               b->d_stars, items, ws, P, e, om, M0, s, rows, ll, nullptr);
     }
-    hipLaunchKernelGGL((k_lnl_batch<L, PHYS, MIXED, false>), dim3(grid), dim3(block), 0, stream,
-                       b->d_stars, items, n_items, counter, P, e, om, M0, s, rows, ll, nullptr);
 }
 
 template <bool MIXED>
@@ -2103,7 +2142,7 @@ static hipError_t launch_batch_dispatch(const jk_batch *b, int64_t n_items,
                                         const jk_work_item *items, const double *P,
                                         const void *e, const void *om, const void *M0,
                                         const void *s, const int64_t *rows, double *ll,
-                                        float *bd, int block, int grid, unsigned *counter,
+                                        float *bd, int block, int grid,
                                         hipStream_t stream)
 {
     const bool phys = b->jitter_mode == JK_JITTER_PHYSICAL;
@@ -2111,10 +2150,10 @@ static hipError_t launch_batch_dispatch(const jk_batch *b, int64_t n_items,
     case LL:                                                                                      \
         if (phys)                                                                                 \
             launch_batch_t<LL, true, MIXED>(b, n_items, items, P, e, om, M0, s, rows, ll, bd,      \
-                                            block, grid, counter, stream);                        \
+                                            block, grid, stream);                        \
         else                                                                                      \
             launch_batch_t<LL, false, MIXED>(b, n_items, items, P, e, om, M0, s, rows, ll, bd,     \
-                                             block, grid, counter, stream);                       \
+                                             block, grid, stream);                       \
         break;
     switch (b->L) {
         JK_BCASE(1)
@@ -2136,14 +2175,14 @@ hipError_t jk_launch_lnl_batch(const jk_batch *b, int precision, int64_t n_items
                                const jk_work_item *items, const double *P, const void *e,
                                const void *om, const void *M0, const void *s,
                                const int64_t *rows, double *ll, float *bound, int block, int grid,
-                               unsigned *counter, hipStream_t stream)
+                               hipStream_t stream)
 {
     if (n_items <= 0) return hipSuccess;
     if (precision == 0)
         return launch_batch_dispatch<false>(b, n_items, items, P, e, om, M0, s, rows, ll, nullptr,
-                                            block, grid, counter, stream);
+                                            block, grid, stream);
     return launch_batch_dispatch<true>(b, n_items, items, P, e, om, M0, s, rows, ll, bound, block,
-                                       grid, counter, stream);
+                                       grid, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -2169,8 +2208,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const 
                                                          const StarDev *__restrict__ probes,
                                                          const double2 *__restrict__ prune,
                                                          const jk_work_item *__restrict__ items,
-                                                         int64_t n_items,
-                                                         unsigned *__restrict__ counter,
+                                                         WorkSplit ws,
                                                          const double *__restrict__ P,
                                                          const void *__restrict__ e_,
                                                          const void *__restrict__ om_,
@@ -2180,92 +2218,88 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const 
                                                          float *__restrict__ bound,
                                                          unsigned long long *__restrict__ n_full)
 {
-    __shared__ unsigned s_item;
     __shared__ int s_n;
     __shared__ int s_list[JK_PRUNE_LIST];
     __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
+    const int64_t q0 = ws.first + blockIdx.x;
+    const jk_work_item w = items[q0 >> ws.lg_parts];
+    int lo, hi;
+    jk_split_item(ws, q0, w.n_rows, lo, hi);
+    if (lo >= hi) return;
     jk_stage_tab<MIXED>(s_tab);
-    for (;;) {
-        if (threadIdx.x == 0) s_item = atomicAdd(counter, 1u);
-        __syncthreads();
-        const int64_t it = (int64_t)__builtin_amdgcn_readfirstlane(s_item);
-        __syncthreads();
-        if (it >= n_items) break;
-        const jk_work_item w = items[it];
-        const StarDev &st = stars[w.star];
-        const double2 pr = prune[w.star];
-        if (!(pr.x > -INFINITY)) {
-            for (int j = threadIdx.x; j < w.n_rows; j += blockDim.x) {
-                const int64_t r = w.row_begin + j;
-                if constexpr (MIXED) {
-                    float b;
-                    ll[w.out_offset + j] =
-                        jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
-                    bound[w.out_offset + j] = b;
-                } else {
-                    ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
-                    if (bound) bound[w.out_offset + j] = 0.0f;
-                }
-            }
-            if (n_full && threadIdx.x == 0)
-                atomicAdd(n_full + w.star, (unsigned long long)w.n_rows);
-            continue;
-        }
-        const StarDev &pb = probes[w.star];
-        unsigned n_surv = 0;
-        if (threadIdx.x == 0) s_n = 0;
-        __syncthreads();
-        for (int base = 0; base < w.n_rows; base += blockDim.x) {
-            const int j = base + (int)threadIdx.x;
-            if (j < w.n_rows) {
-                const int64_t r = w.row_begin + j;
-                double v;
-                if constexpr (MIXED) {
-                    float b;
-                    v = jk_lnl_row<L, PHYS, true, false, true>(pb, r, P, e_, om_, M0_, s_, s_tab, &b);
-                    v += (double)b + pr.y;
-                } else {
-                    v = jk_lnl_row<L, PHYS, false>(pb, r, P, e_, om_, M0_, s_, s_tab);
-                    // FP64 rounding of both evaluations, far below this slack
-                    v += pr.y + 1e-9 * (1.0 + fabs(v));
-                }
-                if (isfinite(v) && v < pr.x) {
-                    ll[w.out_offset + j] = v;
-                    if (bound) bound[w.out_offset + j] = JK_BOUND_UPPER;
-                } else {
-                    s_list[atomicAdd(&s_n, 1)] = j;
-                }
-            }
-            __syncthreads();
-            // Survivors gather over chunks and are evaluated once another
-            // chunk might overflow the list, or at the item's end: the full
-            // evaluations then run on whole waves.
-            const int ns = s_n;
-            __syncthreads();   // every thread holds ns before the next append
-            if (ns > JK_PRUNE_LIST - (int)blockDim.x || base + (int)blockDim.x >= w.n_rows) {
-                n_surv += (unsigned)ns;
-                for (int k = threadIdx.x; k < ns; k += blockDim.x) {
-                    const int jj = s_list[k];
-                    const int64_t r = w.row_begin + jj;
-                    if constexpr (MIXED) {
-                        float b;
-                        ll[w.out_offset + jj] =
-                            jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
-                        bound[w.out_offset + jj] = b;
-                    } else {
-                        ll[w.out_offset + jj] =
-                            jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
-                        if (bound) bound[w.out_offset + jj] = 0.0f;
-                    }
-                }
-                __syncthreads();   // every read of s_list before it is reset
-                if (threadIdx.x == 0) s_n = 0;
-                __syncthreads();
+    const StarDev &st = stars[w.star];
+    const double2 pr = prune[w.star];
+    if (!(pr.x > -INFINITY)) {
+        for (int j = lo + (int)threadIdx.x; j < hi; j += blockDim.x) {
+            const int64_t r = w.row_begin + j;
+            if constexpr (MIXED) {
+                float b;
+                ll[w.out_offset + j] =
+                    jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
+                bound[w.out_offset + j] = b;
+            } else {
+                ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
+                if (bound) bound[w.out_offset + j] = 0.0f;
             }
         }
-        if (n_full && threadIdx.x == 0 && n_surv)
-            atomicAdd(n_full + w.star, (unsigned long long)n_surv);
+        if (n_full && threadIdx.x == 0)
+            atomicAdd(n_full + w.star, (unsigned long long)(hi - lo));
+        return;
     }
+    const StarDev &pb = probes[w.star];
+    unsigned n_surv = 0;
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    for (int base = lo; base < hi; base += blockDim.x) {
+        const int j = base + (int)threadIdx.x;
+        if (j < hi) {
+            const int64_t r = w.row_begin + j;
+            double v;
+            if constexpr (MIXED) {
+                float b;
+                v = jk_lnl_row<L, PHYS, true, false, true>(pb, r, P, e_, om_, M0_, s_, s_tab, &b);
+                v += (double)b + pr.y;
+            } else {
+                v = jk_lnl_row<L, PHYS, false>(pb, r, P, e_, om_, M0_, s_, s_tab);
+                // FP64 rounding of both evaluations, far below this slack
+                v += pr.y + 1e-9 * (1.0 + fabs(v));
+            }
+            if (isfinite(v) && v < pr.x) {
+                ll[w.out_offset + j] = v;
+                if (bound) bound[w.out_offset + j] = JK_BOUND_UPPER;
+            } else {
+                s_list[atomicAdd(&s_n, 1)] = j;
+            }
+        }
+        __syncthreads();
+        // Survivors gather over chunks and are evaluated once another
+        // chunk might overflow the list, or at the item's end: the full
+        // evaluations then run on whole waves.
+        const int ns = s_n;
+        __syncthreads();   // every thread holds ns before the next append
+        if (ns > JK_PRUNE_LIST - (int)blockDim.x || base + (int)blockDim.x >= hi) {
+            n_surv += (unsigned)ns;
+            for (int k = threadIdx.x; k < ns; k += blockDim.x) {
+                const int jj = s_list[k];
+                const int64_t r = w.row_begin + jj;
+                if constexpr (MIXED) {
+                    float b;
+                    ll[w.out_offset + jj] =
+                        jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
+                    bound[w.out_offset + jj] = b;
+                } else {
+                    ll[w.out_offset + jj] =
+                        jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
+                    if (bound) bound[w.out_offset + jj] = 0.0f;
+                }
+            }
+            __syncthreads();   // every read of s_list before it is reset
+            if (threadIdx.x == 0) s_n = 0;
+            __syncthreads();
+        }
+    }
+    if (n_full && threadIdx.x == 0 && n_surv)
+        atomicAdd(n_full + w.star, (unsigned long long)n_surv);
 }
 
 template <int L, bool PHYS, bool MIXED>
@@ -2273,12 +2307,15 @@ static void launch_prune_t(const jk_batch *b, const jk_batch *pb, const double2 
                            int64_t n_items, const jk_work_item *items, const double *P,
                            const void *e, const void *om, const void *M0, const void *s,
                            double *ll, float *bound, unsigned long long *n_full, int block,
-                           int grid, unsigned *counter, hipStream_t stream)
+                           int grid, hipStream_t stream)
 {
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, stream, counter);
-    hipLaunchKernelGGL((k_lnl_prune_batch<L, PHYS, MIXED>), dim3(grid), dim3(block), 0, stream,
-                       b->d_stars, pb->d_stars, prune, items, n_items, counter, P, e, om, M0, s,
-                       ll, bound, n_full);
+    WorkSplit ws{0, std::min(2u, jk_item_parts(n_items, grid))};
+    const int64_t entries = n_items << ws.lg_parts;
+    for (; ws.first < entries; ws.first += JK_ITEM_LAUNCH)
+        hipLaunchKernelGGL((k_lnl_prune_batch<L, PHYS, MIXED>),
+                           dim3((unsigned)std::min(entries - ws.first, JK_ITEM_LAUNCH)),
+                           dim3(block), 0, stream, b->d_stars, pb->d_stars, prune, items, ws, P, e,
+                           om, M0, s, ll, bound, n_full);
 }
 
 hipError_t jk_launch_lnl_prune_batch(const jk_batch *b, const jk_batch *pb, const double *prune,
@@ -2286,7 +2323,7 @@ hipError_t jk_launch_lnl_prune_batch(const jk_batch *b, const jk_batch *pb, cons
                                      const double *P, const void *e, const void *om,
                                      const void *M0, const void *s, double *ll, float *bound,
                                      unsigned long long *n_full, int block, int grid,
-                                     unsigned *counter, hipStream_t stream)
+                                     hipStream_t stream)
 {
     if (n_items <= 0) return hipSuccess;
     const bool phys = b->jitter_mode == JK_JITTER_PHYSICAL;
@@ -2296,17 +2333,17 @@ hipError_t jk_launch_lnl_prune_batch(const jk_batch *b, const jk_batch *pb, cons
         if (precision == 1) {                                                                     \
             if (phys)                                                                             \
                 launch_prune_t<LL, true, true>(b, pb, pr, n_items, items, P, e, om, M0, s, ll,     \
-                                               bound, n_full, block, grid, counter, stream);      \
+                                               bound, n_full, block, grid, stream);      \
             else                                                                                  \
                 launch_prune_t<LL, false, true>(b, pb, pr, n_items, items, P, e, om, M0, s, ll,    \
-                                                bound, n_full, block, grid, counter, stream);     \
+                                                bound, n_full, block, grid, stream);     \
         } else {                                                                                  \
             if (phys)                                                                             \
                 launch_prune_t<LL, true, false>(b, pb, pr, n_items, items, P, e, om, M0, s, ll,    \
-                                                bound, n_full, block, grid, counter, stream);     \
+                                                bound, n_full, block, grid, stream);     \
             else                                                                                  \
                 launch_prune_t<LL, false, false>(b, pb, pr, n_items, items, P, e, om, M0, s, ll,   \
-                                                 bound, n_full, block, grid, counter, stream);    \
+                                                 bound, n_full, block, grid, stream);    \
         }                                                                                         \
         break;
     switch (b->L) {

@@ -5,7 +5,7 @@ Each request is one star run through ``iterative_rejection_sample``
 admitted while active slots and the HBM arena allow; each admitted star takes
 a slot of one device star table (``jk_batch_create_slots``) until it
 finishes.  Every step evaluates the next batch of rows of *every* active
-request in one persistent ``jk_lnl_batch`` launch (stars of different epoch
+request in one ``jk_lnl_batch`` launch (stars of different epoch
 counts side by side) writing straight into each request's region of one HBM
 lnL arena (mixed precision: with each row's error bound in a parallel
 arena), then re-evaluates in FP64 the new rows that the bound leaves within
@@ -425,7 +425,7 @@ class JokerServer:
     def _create_device_stars(self, r):
         """The device half of admission: the request's device star (and
         probe).  At the start of a step, when the device is idle: an upload
-        behind a running persistent launch would wait for it to end."""
+        behind a running likelihood launch would wait for it to end."""
         a, dd = r.arrays, r.data_prepared
         r.star = DeviceStar(a["t"], a["rv"], a["ivar"], a["trend"], a["mu"], a["lam"],
                             a["t_ref"], a["k_prior_mode"], a["sigma_K0"], a["P0"],
