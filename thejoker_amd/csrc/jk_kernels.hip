@@ -320,7 +320,7 @@ __device__ __forceinline__ void jk_kepler_markley_f32(float x, float e, float om
 
 // One prior row's orbit: what every epoch of it shares.
 struct RowOrbit {
-    double e, invP, nP, M0, M0t, s2, lam0, cwq, swsq, dmax;
+    double e, invP, nP, M0, M0t, s2, lam0, cw, ecw, swsq, dmax;
     // FP32 copies for the Kepler starter (e capped below 1 in FP32; 1 - e
     // rounded from its FP64 value, so it keeps its relative accuracy) and for
     // the mixed row's design value, which is combined in FP32.
@@ -373,12 +373,12 @@ __device__ __forceinline__ bool jk_row_orbit(const StarDev &st, int64_t r,
     o.a1f = JK_MARKLEY_A1N * __builtin_amdgcn_rcpf(1.0f + o.ef);
     double sw, cw;
     jk_sincos_tab_f64(omv, tab, sw, cw);
-    const double q2 = (1.0 - ev) * (1.0 + ev);
-    o.swsq = sw * sqrt(q2);
-    o.cwq = cw * q2;
+    o.swsq = sw * sqrt((1.0 - ev) * (1.0 + ev));
+    o.cw = cw;
+    o.ecw = ev * cw;
     o.cwf = (float)cw;
     o.swsqf = (float)o.swsq;
-    o.ecwf = (float)(ev * cw);
+    o.ecwf = (float)o.ecw;
     // The FP32 starter sees e rounded to FP32; within 1e-7 of 1 that can put
     // it outside the correction's reach, so such samples take the fallback.
     o.dmax = ev > 0.9999999 ? -1.0 : 1e-3;
@@ -433,13 +433,13 @@ __device__ __forceinline__ double jk_row_epoch(const RowOrbit &o, double dtk, do
         } else {
             bad |= !jk_kepler_markley_f64(x, o.e, o.ef, o.omef, o.a1f, o.dmax, tab, sE, cE);
         }
-        // m = [cos w (1-e^2) cos E - sin w sqrt(1-e^2) sin E] / (1 - e cos E)
+        // m = [cos w (cos E - e) - sin w sqrt(1-e^2) sin E] / (1 - e cos E) + e cos w
         // (one Newton step on the hardware reciprocal: relative 2e-15).
-        // cos f + e = (1-e^2) cos E / (1 - e cos E): one FP64 operation fewer
-        // than cos w (cos E - e) ... + e cos w, and no cancellation between
-        // the two terms in cos w
+        // cos f + e = (1-e^2) cos E / (1 - e cos E) saves one operation of
+        // about 100 but moves the rows of e -> 1 by as much as their rounding
+        // already does (up to 1e-8 of the lnL at 1 - e = 1e-6)
         const double den = jk_rcp1(fma(-o.e, cE, 1.0));
-        m = fma(o.cwq, cE, -o.swsq * sE) * den;
+        m = fma(fma(o.cw, cE - o.e, -o.swsq * sE), den, o.ecw);
     }
     return m;
 }
