@@ -85,3 +85,24 @@ def test_reject_dispatch_edges(gpu, n, kind):
     top = torch.as_tensor([ll.max()], dtype=torch.float64, device="cuda")
     idx, n_pass, _ = D.reject(d, state, 100, llmax=top)
     assert n_pass == len(want) and np.array_equal(idx, want[:100])
+
+
+@pytest.mark.parametrize("n_seg", [1, 4, 5])
+def test_descriptor_upload_edges(gpu, n_seg):
+    """Descriptors as kernel arguments (up to four segments) and by a copy:
+    two calls queued one after the other, each on other segments, give what
+    they give alone, segment by segment."""
+    g = np.random.default_rng(n_seg)
+    sizes = [700 + 131 * i for i in range(n_seg)]
+    off = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    ll = torch.as_tensor(g.normal(-20.0, 3.0, int(sum(sizes))), device="cuda")
+    ll2 = torch.as_tensor(g.normal(-5.0, 1.0, int(sum(sizes))), device="cuda")
+    states = [(int(g.integers(1 << 62)) << 60 | 5, int(g.integers(1 << 62)) | 1)
+              for _ in range(n_seg)]
+    for x in (ll, ll2):
+        idx, n_pass, mx = B.reject_batch(x, off, sizes, states, 50)
+        for i in range(n_seg):
+            one = B.reject_batch(x[off[i]:off[i] + sizes[i]].clone(), [0], [sizes[i]],
+                                 [states[i]], 50)
+            assert np.array_equal(idx[i], one[0][0]) and n_pass[i] == one[1][0]
+            assert mx[i] == one[2][0] == float(x[off[i]:off[i] + sizes[i]].max())

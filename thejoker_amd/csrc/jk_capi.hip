@@ -147,6 +147,30 @@ hipError_t scratch_get(hipStream_t st, size_t bytes, void **out, ScratchLease *l
     return hipSuccess;
 }
 
+// The descriptors of a segmented call on their way to the device, ordered on
+// the stream.  Up to JK_SEG_ARGS (one launch) go as kernel arguments and the
+// call returns without waiting; more go by a copy from the (pageable) host
+// array, which must outlive it: done() then waits for the stream.  One segment
+// of 2^22 rows settled, lnL included: 299 us by the copy, 276 by arguments; a
+// pruned rejection of 2^21 rows 364 and 302.  From about eight segments on the
+// copy is the faster (8: 114 against 124 us, 28: 147 against 159 with 28
+// descriptors per launch): the results' copy back is then larger and starts
+// sooner on an idle stream.  A call with host descriptors is refused under
+// capture (a replay could not read them again).
+struct SegUpload {
+    bool wait = false;
+
+    hipError_t put(SegDev *dst, const std::vector<SegDev> &h, const ScratchLease &lease,
+                   hipStream_t st)
+    {
+        if (lease.pooled) return hipErrorStreamCaptureUnsupported;
+        if (h.size() <= JK_SEG_ARGS) return jk_put_segs(dst, h.data(), (int)h.size(), st);
+        wait = true;
+        return hipMemcpyAsync(dst, h.data(), sizeof(SegDev) * h.size(), hipMemcpyHostToDevice, st);
+    }
+    hipError_t done(hipStream_t st) const { return wait ? hipStreamSynchronize(st) : hipSuccess; }
+};
+
 hipError_t scratch_put(hipStream_t st, void *ptr, ScratchLease &lease)
 {
     if (lease.pooled) return hipFreeAsync(ptr, st);
@@ -923,12 +947,12 @@ static int reject_batch_impl(const double *ll, int n_seg, const jk_segment *segs
     double *partials = (double *)(scratch + seg_pad);
     uint64_t *mask = (uint64_t *)(partials + (size_t)pb * n_seg);
     int64_t *bsum = (int64_t *)(mask + mask_words);
-    hipError_t err = hipMemcpyAsync(d_segs, h.data(), seg_bytes, hipMemcpyHostToDevice, st);
+    SegUpload up;
+    hipError_t err = up.put(d_segs, h, lease, st);
     if (err == hipSuccess)
         err = jk_launch_reject_batch(ll, n_seg, d_segs, max_n, max_nb, partials, pb, mask, bsum,
                                      idx_out, n_pass_out, llmax_out, st, zero_u_out);
-    // The host descriptor array must outlive the queued copy.
-    hipError_t err3 = hipStreamSynchronize(st);
+    hipError_t err3 = up.done(st);
     hipError_t err2 = scratch_put(st, scratch, lease);
     if (err != hipSuccess || err3 != hipSuccess) return JK_EHIP;
     return check_hip(err2);
@@ -1002,13 +1026,13 @@ int jk_polish_batch(const jk_batch *batch, int n_seg, const jk_polish_segment *s
     int64_t *bsum = (int64_t *)(mask + mask_words);
     int64_t *idx = bsum + bsum_n;
     int64_t *cum = idx + idx_n;
-    hipError_t err = hipMemcpyAsync(d_segs, h.data(), seg_bytes, hipMemcpyHostToDevice, st);
+    SegUpload up;
+    hipError_t err = up.put(d_segs, h, lease, st);
     if (err == hipSuccess)
         err = jk_launch_polish_batch(batch, n_seg, d_segs, max_n, max_nb, partials, pb, mask, bsum,
                                      idx, llmax, cum, P, e, omega, M0, s, rows, ll_inout, window,
                                      n_polished_out, st);
-    // The host descriptor array must outlive the queued copy.
-    hipError_t err3 = hipStreamSynchronize(st);
+    hipError_t err3 = up.done(st);
     hipError_t err2 = scratch_put(st, scratch, lease);
     if (err != hipSuccess || err3 != hipSuccess) return JK_EHIP;
     return check_hip(err2);
@@ -1061,13 +1085,13 @@ int jk_settle_batch(const jk_batch *batch, int n_seg, const jk_settle_segment *s
     int64_t *idx = (int64_t *)(key + n_seg);
     int64_t *cum = idx + idx_n;
     int64_t *count1 = cum + n_seg + 1;
-    hipError_t err = hipMemcpyAsync(d_segs, h.data(), seg_bytes, hipMemcpyHostToDevice, st);
+    SegUpload up;
+    hipError_t err = up.put(d_segs, h, lease, st);
     if (err == hipSuccess)
         err = jk_launch_settle_batch(batch, n_seg, d_segs, max_n, partials, pb, idx, key, cum,
                                      count1, P, e, omega, M0, s, rows, ll_inout, bound_inout,
                                      n_settled_out, st);
-    // The host descriptor array must outlive the queued copy.
-    hipError_t err3 = hipStreamSynchronize(st);
+    hipError_t err3 = up.done(st);
     hipError_t err2 = scratch_put(st, scratch, lease);
     if (err != hipSuccess || err3 != hipSuccess) return JK_EHIP;
     return check_hip(err2);
@@ -1139,16 +1163,16 @@ int jk_settle_reject_batch(const jk_batch *batch, int n_seg, const jk_settle_seg
     int64_t *idx = bsum + bsum_n;
     int64_t *cum = idx + idx_n;
     int64_t *count1 = cum + n_seg + 1;
-    hipError_t err = hipMemcpyAsync(d_settle, hs.data(), seg_bytes, hipMemcpyHostToDevice, st);
+    SegUpload up;
+    hipError_t err = up.put(d_settle, hs, lease, st);
     if (err == hipSuccess)
-        err = hipMemcpyAsync(d_reject, hr.data(), seg_bytes, hipMemcpyHostToDevice, st);
+        err = up.put(d_reject, hr, lease, st);
     if (err == hipSuccess)
         err = jk_launch_settle_reject_batch(batch, n_seg, d_settle, d_reject, max_n, max_nb,
                                             partials, pb, mask, bsum, idx, key, cum, count1, P, e, omega, M0, s, rows, ll_inout,
                                             bound_inout, idx_out, n_pass_out, llmax_out,
                                             n_settled_out, st);
-    // The host descriptor arrays must outlive the queued copies.
-    hipError_t err3 = hipStreamSynchronize(st);
+    hipError_t err3 = up.done(st);
     hipError_t err2 = scratch_put(st, scratch, lease);
     if (err != hipSuccess || err3 != hipSuccess) return JK_EHIP;
     return check_hip(err2);
@@ -1207,7 +1231,8 @@ static int settle_new_rows(int mode, const jk_batch *batch, int n_seg,
     int64_t *idx = (int64_t *)(partials + (size_t)pb * n_seg);
     int64_t *cum = idx + idx_n;
     int64_t *count1 = cum + n_seg + 1;
-    hipError_t err = hipMemcpyAsync(d_segs, h.data(), seg_bytes, hipMemcpyHostToDevice, st);
+    SegUpload up;
+    hipError_t err = up.put(d_segs, h, lease, st);
     if (err == hipSuccess && mode == SETTLE_LIVE)
         err = jk_launch_settle_live_batch(batch, n_seg, d_segs, max_n, partials, pb, idx, cum, P, e,
                                           omega, M0, s, rows, ll_inout, bound_inout, margin,
@@ -1219,8 +1244,7 @@ static int settle_new_rows(int mode, const jk_batch *batch, int n_seg,
         err = jk_launch_settle_pruned_batch(batch, n_seg, d_segs, max_n, partials, pb, idx, cum,
                                             count1, P, e, omega, M0, s, rows, ll_inout,
                                             bound_inout, window, margin, n_settled_out, st);
-    // The host descriptor array must outlive the queued copy.
-    hipError_t err3 = hipStreamSynchronize(st);
+    hipError_t err3 = up.done(st);
     hipError_t err2 = scratch_put(st, scratch, lease);
     if (err != hipSuccess || err3 != hipSuccess) return JK_EHIP;
     return check_hip(err2);

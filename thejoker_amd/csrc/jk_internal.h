@@ -49,6 +49,10 @@ struct PcgJump {
 // Host-side 128-bit helpers (same arithmetic as the device u128 functions).
 void jk_pcg_jump_coeffs(uint64_t k, u128 *A, u128 *D);
 
+// Most descriptors of one jk_put_segs launch.
+#define JK_SEG_ARGS 4
+hipError_t jk_put_segs(SegDev *dst, const SegDev *src, int n, hipStream_t stream);
+
 hipError_t jk_launch_lnl_f64(const jk_star *st, int64_t n, const double *P, const double *e,
                              const double *om, const double *M0, const double *s,
                              const int64_t *rows, double *ll, hipStream_t stream);

@@ -15,6 +15,7 @@
 //                          lanes per row).
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <type_traits>
 
 #include "jk_internal.h"
@@ -1991,6 +1992,31 @@ hipError_t jk_launch_polish(const jk_star *st, int64_t n, const double *P, const
         return hipErrorInvalidValue;
     }
 #undef JK_SCASE
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Up to JK_SEG_ARGS segment descriptors to the device as kernel arguments:
+// they are copied into the launch's argument buffer at the call, so the host
+// array need not outlive it and nothing waits.
+// ---------------------------------------------------------------------------
+struct SegArgs {
+    uint64_t w[JK_SEG_ARGS * sizeof(SegDev) / sizeof(uint64_t)];
+};
+
+__global__ __launch_bounds__(256) void k_put_segs(uint64_t *__restrict__ dst, const SegArgs a,
+                                                  int n_words)
+{
+    for (int i = threadIdx.x; i < n_words; i += 256) dst[i] = a.w[i];
+}
+
+hipError_t jk_put_segs(SegDev *dst, const SegDev *src, int n, hipStream_t stream)
+{
+    SegArgs a;
+    if (n > JK_SEG_ARGS) return hipErrorInvalidValue;
+    memcpy(a.w, src, sizeof(SegDev) * n);
+    hipLaunchKernelGGL(k_put_segs, dim3(1), dim3(256), 0, stream, (uint64_t *)dst, a,
+                       (int)(n * sizeof(SegDev) / sizeof(uint64_t)));
     return hipGetLastError();
 }
 
