@@ -2586,7 +2586,7 @@ hipError_t jk_launch_reject_batch(const double *ll, int n_seg, const SegDev *d_s
 // gathers its rows in LDS and claims room for up to JK_APPEND_CAP of them with
 // one atomic, its workgroup for the rest.  Flag words with a block-count and an ordered compaction pass
 // took two launches and a pass over the words more (2^21 rows: 7 + 6.5 + 6 us
-// for each of four lists; 8 us this way).
+// for each of four lists; 6 to 12 us this way).
 // ---------------------------------------------------------------------------
 #define JK_APPEND_CAP 512
 
