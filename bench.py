@@ -387,14 +387,13 @@ def leg_batched(args, torch, np, D, syn):
     items, off, total = B.work_items([n] * n_stars, shape.tile)
     items = items[B.heaviest_first(items, M)]
     d_items = B.upload_items(items)
-    ws = torch.zeros(64, dtype=torch.int32, device="cuda")
     llm = torch.empty(total, dtype=torch.float64, device="cuda")
     llf = torch.empty(total, dtype=torch.float64, device="cuda")
     bnd = torch.empty(total, dtype=torch.float32, device="cuda")
     run_m = lambda: B.lnl_batch(batch, cache, d_items, len(items), total, "mixed", shape,
-                                out=llm, workspace=ws, bound=bnd)
+                                out=llm, bound=bnd)
     run_f = lambda: B.lnl_batch(batch, cache, d_items, len(items), total, "f64", shape,
-                                out=llf, workspace=ws)
+                                out=llf)
     run_m()
     run_f()
     m_ms = timed(run_m, 3, torch)

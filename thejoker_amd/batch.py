@@ -556,18 +556,16 @@ def autotune(batch, cache, n_rows, precision="mixed", candidates=None, sample_st
     sub = min(sample_stars, len(batch))
     results = {}
     best, best_ms = None, np.inf
-    ws = torch.zeros(64, dtype=torch.int32, device=cache.P.device)
     for shape in candidates:
         items, _, total = work_items(n_rows[:sub], shape.tile)
         items = items[heaviest_first(items, batch.M)]
         d_items = upload_items(items, device)
         out = torch.empty(total, dtype=torch.float64, device=cache.P.device)
-        lnl_batch(batch, cache, d_items, len(items), total, precision, shape, out=out, workspace=ws)
+        lnl_batch(batch, cache, d_items, len(items), total, precision, shape, out=out)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         for _ in range(reps):
-            lnl_batch(batch, cache, d_items, len(items), total, precision, shape, out=out,
-                      workspace=ws)
+            lnl_batch(batch, cache, d_items, len(items), total, precision, shape, out=out)
         torch.cuda.synchronize()
         ms = (time.perf_counter() - t0) / reps * 1e3
         results[repr(shape)] = ms
@@ -779,7 +777,6 @@ class StepGraph:
         self.ll = torch.empty(total, dtype=torch.float64, device=dev)
         self.bound = (torch.empty(total, dtype=torch.float32, device=dev)
                       if precision == "mixed" else None)
-        self.ws = torch.zeros(64, dtype=torch.int32, device=dev)
         self.plan = SegPlan(batch, offsets, sizes, rng_states, max_keep, device=device)
         shape = shape or LaunchShape()
         if shape.grid <= 0:
@@ -788,7 +785,7 @@ class StepGraph:
 
         def body():
             lnl_batch(batch, cache, d_items, n_items, total, precision, shape, out=self.ll,
-                      workspace=self.ws, bound=self.bound)
+                      bound=self.bound)
             if precision == "mixed":
                 self.plan.settle_reject(cache, self.ll, self.bound)
             else:

@@ -306,7 +306,6 @@ class JokerServer:
         self._n_full = torch.zeros(self.max_active, dtype=torch.int64, device=cache.P.device)
         self.rows_probed = 0      # rows of requests whose star was probed
         self.rows_pruned = 0      # of those, the rows that kept their bound
-        self._ws = torch.zeros(64, dtype=torch.int32, device=cache.P.device)
         self._uploader = ItemUploader(device)
         self.profile = profile
         self.phase_s = dict.fromkeys(self.PHASES, 0.0)
@@ -690,12 +689,12 @@ class JokerServer:
         probed = []
         if thr is None:
             lnl_batch(self._table, self.cache, d_items, len(items), 0, self.precision, self.shape,
-                      out=self.arena, workspace=self._ws, bound=self.arena_b)
+                      out=self.arena, bound=self.arena_b)
         else:
             self._prune_dev.copy_(_torch().from_numpy(thr.reshape(-1)))
             lnl_prune_batch(self._table, self._probes, self._prune_dev, self.cache, d_items,
                             len(items), self.precision, self.shape, out=self.arena,
-                            bound=self.arena_b, workspace=self._ws, n_full=self._n_full)
+                            bound=self.arena_b, n_full=self._n_full)
             probed = [(r, r.slot, int(sizes[k])) for k, (r, _, _) in enumerate(plan)
                       if np.isfinite(thr[r.slot, 0])]
         lap("lnl_launch")
