@@ -106,3 +106,26 @@ def test_descriptor_upload_edges(gpu, n_seg):
                                  [states[i]], 50)
             assert np.array_equal(idx[i], one[0][0]) and n_pass[i] == one[1][0]
             assert mx[i] == one[2][0] == float(x[off[i]:off[i] + sizes[i]].max())
+
+
+def test_segment_maximum_edges(gpu):
+    """Segments whose maximum comes from one partial, from several, and from
+    more than a workgroup has threads, one with a NaN, side by side, against
+    numpy."""
+    g = np.random.default_rng(11)
+    sizes = [1, 4096, 4097, 300 * 4096 + 5, 64, 10000]
+    off = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    ll = -(g.random(int(sum(sizes))) * 5.0)
+    ll[off[5] + 9999] = np.nan
+    ll[off[3] + sizes[3] - 1] = 1.0          # the last row of the last partial
+    states, us = [], []
+    for i, n in enumerate(sizes):
+        rng = np.random.default_rng(100 + i)
+        states.append(D.pcg64_state(rng))
+        us.append(rng.uniform(size=n))
+    idx, n_pass, mx = B.reject_batch(torch.as_tensor(ll, device="cuda"), off, sizes, states, 500)
+    for i, n in enumerate(sizes):
+        x = ll[off[i]:off[i] + n]
+        want = np.where(np.exp(x - x.max()) > us[i])[0]
+        assert n_pass[i] == len(want) and np.array_equal(idx[i], want[:500])
+        assert np.array_equal(mx[i], x.max(), equal_nan=True)
