@@ -527,8 +527,9 @@ __device__ __forceinline__ double jk_row_finish(const StarDev &st, double lam0,
 // operations saved above, 2^20 x 37 at L = 5 134 -> 127 us) and the mixed
 // rows of many stars (64 x 2^18 rows 1935 -> 1895 us) take the records, the
 // mixed single-star row the arrays (2^22 x 50: 394 us, with records 415).
+// LONE: the row of a launch of at most one wave per SIMD (k_lnl).
 template <int L, bool PHYS, bool MIXED, bool SAFE = false, bool BOUND = false, bool ONE = false,
-          bool REC = !MIXED>
+          bool LONE = false, bool REC = !MIXED && !LONE>
 __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
                                              const double *__restrict__ P,
                                              const void *__restrict__ e_,
@@ -563,7 +564,7 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
     float dmx = 0.0f;      // largest 1 / (1 - e cos E) (BOUND only)
     // four epochs at a time where every fourth renormalises the product and the
     // registers allow it (2^24 rows x 16 epochs 936 -> 930 us), else two
-    constexpr int U = PHYS && !MIXED && ONE ? 4 : 2;
+    constexpr int U = LONE || (PHYS && !MIXED && ONE) ? 4 : 2;
 #pragma unroll U
     for (int k = 0; k < N; ++k) {
         const double *__restrict__ ep = st.ep + (size_t)k * (JK_EP_T + LT0);
@@ -845,6 +846,8 @@ __device__ __forceinline__ double jk_rows_split(const StarDev &st, int R, int sw
 #define JK_SPLIT_MAX_ROWS 49152
 #define JK_SPLIT_MIN_EPOCHS 10
 #define JK_SPLIT_RMIN 8
+// Rows that give every SIMD one wave.
+#define JK_LONE_MAX_ROWS 65536
 
 static int jk_split_rows(int64_t n, int N)
 {
@@ -971,17 +974,26 @@ __device__ __forceinline__ int64_t wave_incl_scan_i64(int64_t v, int lane)
 // (4 jk_dense_blocks(n) entries), so the rejection step need not read the
 // lnL array a second time to find the maximum.  With BOUND (mixed
 // precision), bound[i] receives the row's error bound (jk_lnl_row).
-template <int L, bool PHYS, bool MIXED, bool BOUND, bool ONE = false>
-__global__ __launch_bounds__(256) void k_lnl(const StarDev st, int64_t n,
-                                             const double *__restrict__ P,
-                                             const void *__restrict__ e_,
-                                             const void *__restrict__ om_,
-                                             const void *__restrict__ M0_,
-                                             const void *__restrict__ s_,
-                                             const int64_t *__restrict__ rows,
-                                             double *__restrict__ ll,
-                                             double *__restrict__ blockmax,
-                                             float *__restrict__ bound)
+//
+// LONE: the FP64 instance for launches of at most one wave per SIMD
+// (JK_LONE_MAX_ROWS).  Nothing else runs on the SIMD while such a wave waits,
+// so its time is its own chain of dependent operations, and what shortens that
+// is epochs in flight together: four at a time, scheduled for two waves per
+// SIMD at most (for more, the compiler keeps registers down by finishing one
+// epoch's table read before it starts the next), and the epochs from the
+// arrays, several to a scalar load.  60000 rows by the other instance and by
+// this one, us, for L = 2 and 3 without jitter, 2 and 3 with, 5 without, 6 with:
+// 16 epochs 7.7 -> 7.3, 8.7 -> 7.7, 8.6 -> 7.4, 7.8 -> 7.8, 9.5 -> 8.7, 9.6 -> 9.5;
+// 101 epochs 29.4 -> 25.8, 34.0 -> 27.8, 35.1 -> 28.2, 30.4 -> 30.2,
+// 38.1 -> 31.0, 39.2 -> 38.1.  With two waves per SIMD (131072 rows) it is from
+// 7 % faster (101 epochs, L = 3, no jitter) to 4 % slower (16 epochs, L = 5),
+// with three up to 12 % slower.
+template <int L, bool PHYS, bool MIXED, bool BOUND, bool ONE = false, bool LONE = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, LONE ? 2 : 8)))
+void k_lnl(const StarDev st, int64_t n, const double *__restrict__ P, const void *__restrict__ e_,
+           const void *__restrict__ om_, const void *__restrict__ M0_,
+           const void *__restrict__ s_, const int64_t *__restrict__ rows,
+           double *__restrict__ ll, double *__restrict__ blockmax, float *__restrict__ bound)
 {
     __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
     jk_stage_tab<MIXED>(s_tab);
@@ -996,7 +1008,8 @@ __global__ __launch_bounds__(256) void k_lnl(const StarDev st, int64_t n,
             v = jk_lnl_row<L, PHYS, MIXED, false, true, ONE>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
             bound[i] = b;
         } else {
-            v = jk_lnl_row<L, PHYS, MIXED, false, false, ONE>(st, r, P, e_, om_, M0_, s_, s_tab);
+            v = jk_lnl_row<L, PHYS, MIXED, false, false, ONE, LONE>(st, r, P, e_, om_, M0_, s_,
+                                                                    s_tab);
         }
         ll[i] = v;
         vmax = jk_nanmax(vmax, v);
@@ -1238,7 +1251,7 @@ static int64_t jk_dense_blocks(int64_t n)
     return b < 16384 ? (b < 1 ? 1 : b) : 16384;
 }
 
-// Entries of blockmax the launch over n rows of an N-epoch star writes.
+// Entries of blockmax the FP64 launch over n rows of an N-epoch star writes.
 static int64_t jk_lnl_partials(int64_t n, int N)
 {
     const int R = jk_split_rows(n, N);
@@ -1273,17 +1286,26 @@ static hipError_t launch_lnl_t(const jk_star *st, int64_t n, const double *P, co
             return hipGetLastError();
         }
     }
-    if constexpr (!MIXED && (L == 2 || L == 3)) {
-        // the constant offset as the first trend column (the usual v0)
-        if (st->dev.t0_one) {
-            hipLaunchKernelGGL((k_lnl<L, PHYS, false, false, true>), dim3((unsigned)blocks),
-                               dim3(256), 0, stream, st->dev, n, P, e, om, M0, s, rows, ll,
-                               blockmax, nullptr);
-            return hipGetLastError();
+    if constexpr (!MIXED) {
+        const bool lone = n <= JK_LONE_MAX_ROWS;
+        if constexpr (L == 2 || L == 3) {
+            // the constant offset as the first trend column (the usual v0)
+            if (st->dev.t0_one) {
+                hipLaunchKernelGGL((lone ? k_lnl<L, PHYS, false, false, true, true>
+                                         : k_lnl<L, PHYS, false, false, true>),
+                                   dim3((unsigned)blocks), dim3(256), 0, stream, st->dev, n, P, e,
+                                   om, M0, s, rows, ll, blockmax, nullptr);
+                return hipGetLastError();
+            }
         }
+        hipLaunchKernelGGL((lone ? k_lnl<L, PHYS, false, false, false, true>
+                                 : k_lnl<L, PHYS, false, false>),
+                           dim3((unsigned)blocks), dim3(256), 0, stream, st->dev, n, P, e, om, M0,
+                           s, rows, ll, blockmax, nullptr);
+    } else {
+        hipLaunchKernelGGL((k_lnl<L, PHYS, true, false>), dim3((unsigned)blocks), dim3(256), 0,
+                           stream, st->dev, n, P, e, om, M0, s, rows, ll, blockmax, nullptr);
     }
-    hipLaunchKernelGGL((k_lnl<L, PHYS, MIXED, false>), dim3((unsigned)blocks), dim3(256), 0,
-                       stream, st->dev, n, P, e, om, M0, s, rows, ll, blockmax, nullptr);
     return hipGetLastError();
 }
 
@@ -2090,8 +2112,8 @@ __device__ __forceinline__ double jk_lnl_row_sel(const StarDev &st, int64_t r,
         *bnd = 0.0f;
         return jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, tab);
     }
-    return jk_lnl_row<L, PHYS, true, false, true, false, true>(st, r, P, e_, om_, M0_, s_, tab,
-                                                               bnd);
+    return jk_lnl_row<L, PHYS, true, false, true, false, false, true>(st, r, P, e_, om_, M0_, s_,
+                                                                      tab, bnd);
 }
 
 // Slot `slot` of a star table evaluated in FP64 (exact != 0) or as the launch
@@ -2130,7 +2152,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_batch(const StarDe
         } else if constexpr (MIXED) {
             ll[w.out_offset + j] =
                 st.exact ? jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab)
-                         : jk_lnl_row<L, PHYS, true, false, false, false, true>(
+                         : jk_lnl_row<L, PHYS, true, false, false, false, false, true>(
                                st, r, P, e_, om_, M0_, s_, s_tab);
         } else {
             ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
