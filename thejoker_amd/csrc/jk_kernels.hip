@@ -837,21 +837,35 @@ __device__ __forceinline__ double jk_rows_split(const StarDev &st, int R, int sw
 }
 
 // Rows per workgroup of the split evaluation of n rows of N epochs, or 0 for
-// the launch with one row per lane: R = n / 512 up to 40, then n / 768 up to
-// 64.  Measured on one MI355X, N = 149, L = 3, against one row per lane
-// (about 50 us up to 65536 rows, the time of one wave per SIMD): 22 us at 2048
-// rows, 26 at 8192, 28 at 16384, 37 at 33001 (R = 64 there: 42; n / 1024:
-// 41); at 65536 rows the two are equal, so the line lies below.  Below
-// JK_SPLIT_MIN_EPOCHS there is little to spread (N = 6: no gain).
+// the launch with one row per lane.  R = n / 512 up to 40, then n / 768 up to
+// 64 (with R = 64 at 33001 rows x 149 epochs 42 us instead of 37, with n / 1024
+// 41).  The line between the two was measured on one MI355X from 4 to 200 epochs,
+// L = 2 (without and with jitter), 3 (both), 5 and 6, 1000 to 49152 rows: the
+// split's fixed cost (staging, barriers, the adding wave's last chunk) falls on
+// every workgroup, so the rows it pays for grow with the epochs; more rows
+// than that fill the SIMDs by themselves, the sooner in mixed precision, whose
+// solves are cheaper against the same FP64 sums.
+// FP64, one row per lane / split, us (L = 2 with jitter): N = 10: 2048 rows
+// 6.1 / 5.9, 8192 6.2 / 6.5; N = 17: 2048 7.7 / 6.5, 16384 7.6 / 7.7; N = 37:
+// 2048 12.3 / 8.5, 20480 12.5 / 10.9, 30000 12.4 / 12.8; N = 101: 2048 27.3 /
+// 14.6, 36864 27.6 / 24.8, 43008 27.7 / 30.3.  Mixed: N = 17: 2048 7.2 / 7.1,
+// 8192 7.3 / 8.3; N = 37: 2048 11.4 / 9.0, 20480 11.6 / 10.6, 30000 11.6 / 12.4;
+// N = 101: 2048 24.8 / 14.9, 49152 25.1 / 24.5.
 #define JK_SPLIT_MAX_ROWS 49152
-#define JK_SPLIT_MIN_EPOCHS 10
 #define JK_SPLIT_RMIN 8
 // Rows that give every SIMD one wave.
 #define JK_LONE_MAX_ROWS 65536
 
-static int jk_split_rows(int64_t n, int N)
+static int64_t jk_split_max_rows(int N, bool mixed)
 {
-    if (n > JK_SPLIT_MAX_ROWS || N < JK_SPLIT_MIN_EPOCHS) return 0;
+    if (!mixed) return N < 10 ? 0 : std::min<int64_t>(36864, 600 * ((int64_t)N - 3));
+    if (N < 30) return N < 17 ? 0 : 2048;
+    return std::min<int64_t>(JK_SPLIT_MAX_ROWS, std::max<int64_t>(20480, 490 * (int64_t)N));
+}
+
+static int jk_split_rows(int64_t n, int N, bool mixed)
+{
+    if (n > jk_split_max_rows(N, mixed)) return 0;
     int R = (int)((n + 511) / 512);
     if (R > 40) R = (int)((n + 767) / 768);
     return std::min(std::max(std::max(R, 192 / N), JK_SPLIT_RMIN), 64);
@@ -1254,7 +1268,7 @@ static int64_t jk_dense_blocks(int64_t n)
 // Entries of blockmax the FP64 launch over n rows of an N-epoch star writes.
 static int64_t jk_lnl_partials(int64_t n, int N)
 {
-    const int R = jk_split_rows(n, N);
+    const int R = jk_split_rows(n, N, false);
     return R ? (n + R - 1) / R : 4 * jk_dense_blocks(n);
 }
 
@@ -1264,7 +1278,7 @@ static hipError_t launch_lnl_t(const jk_star *st, int64_t n, const double *P, co
                                const int64_t *rows, double *ll, double *blockmax, float *bound,
                                hipStream_t stream)
 {
-    if (const int R = jk_split_rows(n, st->dev.n)) {
+    if (const int R = jk_split_rows(n, st->dev.n, MIXED)) {
         hipLaunchKernelGGL((k_lnl_split<L, PHYS, MIXED>), dim3((unsigned)((n + R - 1) / R)),
                            dim3(256), 0, stream, st->dev, n, R, P, e, om, M0, s, rows, ll,
                            blockmax, bound);
