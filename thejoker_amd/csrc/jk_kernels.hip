@@ -389,8 +389,9 @@ __device__ __forceinline__ bool jk_row_orbit(const StarDev &st, int64_t r,
 // The design value of an epoch at dt and, with PHYS, its weight from the
 // epoch's variance vk = sigma^2 + s^2.  MIXED: denb = 1 / (1 - e cos E) for
 // the error bound.  FP64 (not SAFE): bad is set where the row needs the
-// bracketed Newton iteration.
-template <bool PHYS, bool MIXED, bool SAFE>
+// bracketed Newton iteration.  FINE: the design value's reciprocal to an ulp
+// (two Newton steps on the hardware's) instead of a relative 2e-15.
+template <bool PHYS, bool MIXED, bool SAFE, bool FINE = false>
 __device__ __forceinline__ double jk_row_epoch(const RowOrbit &o, double dtk, double vk,
                                                const double2 *__restrict__ tab, double &w,
                                                float &denb, bool &bad)
@@ -439,7 +440,8 @@ __device__ __forceinline__ double jk_row_epoch(const RowOrbit &o, double dtk, do
         // cos f + e = (1-e^2) cos E / (1 - e cos E) saves one operation of
         // about 100 but moves the rows of e -> 1 by as much as their rounding
         // already does (up to 1e-8 of the lnL at 1 - e = 1e-6)
-        const double den = jk_rcp1(fma(-o.e, cE, 1.0));
+        const double f1 = fma(-o.e, cE, 1.0);
+        const double den = FINE ? jk_rcp2(f1) : jk_rcp1(f1);
         m = fma(fma(o.cw, cE - o.e, -o.swsq * sE), den, o.ecw);
     }
     return m;
@@ -887,7 +889,11 @@ static int jk_split_rows(int64_t n, int N, bool mixed)
 // products accumulate in registers (16 eigenvalues a tile) while the next
 // step's Kepler solves run on the vector units, so the N^2 multiply-adds per
 // row cost next to nothing, and the solves bound the kernel as they do the
-// diagonal one.  Against one lane per row (a serial dot product, one LDS read
+// diagonal one.  The weights and the design values' reciprocals are good to an
+// ulp (jk_rcp2), as they were with one lane per row: the solves hide the second
+// Newton step (2^18 x 40 69.0 us with one step, 69.1 with two; 524288 x 64 242
+// and 234).  The error of the lnL against 80-bit arithmetic, 60 stars of 4 to 64
+// epochs, is 0.74 of that form's in the mean.  Against one lane per row (a serial dot product, one LDS read
 // per multiply-add, 64 rows' columns in LDS): 2^18 rows x 40 epochs 182 ->
 // 75 us, 524288 x 64 1383 -> 245 us, 3000 x 64 84 -> 17 us, 2^18 x 5 30 ->
 // 27 us.
@@ -931,9 +937,10 @@ __device__ __forceinline__ void jk_cov_rotate(const StarDev &st, const RowOrbit 
             double w;
             float denb;
             bool b = false;
-            m = jk_row_epoch<false, false, false>(o, s_dt[k], 0.0, tab, w, denb, b);
+            m = jk_row_epoch<false, false, false, true>(o, s_dt[k], 0.0, tab, w, denb, b);
             if constexpr (SAFE) {
-                if (bad) m = jk_row_epoch<false, false, true>(o, s_dt[k], 0.0, tab, w, denb, b);
+                if (bad)
+                    m = jk_row_epoch<false, false, true, true>(o, s_dt[k], 0.0, tab, w, denb, b);
             } else {
                 bad |= b;
             }
@@ -1138,7 +1145,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev 
                 double w = s_ep[N + ei];
                 if constexpr (PHYS) {
                     const double vk = w + o.s2;
-                    w = jk_rcp1(vk);
+                    w = jk_rcp2(vk);
                     prod *= vk;      // at most four factors between renormalisations
                 }
                 const double wm = w * m;
