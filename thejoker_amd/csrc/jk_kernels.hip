@@ -891,8 +891,8 @@ static int jk_split_rows(int64_t n, int N, bool mixed)
 // row cost next to nothing, and the solves bound the kernel as they do the
 // diagonal one.  The weights and the design values' reciprocals are good to an
 // ulp (jk_rcp2), as they were with one lane per row: the solves hide the second
-// Newton step (2^18 x 40 69.0 us with one step, 69.1 with two; 524288 x 64 242
-// and 234).  The error of the lnL against 80-bit arithmetic, 60 stars of 4 to 64
+// Newton step (2^18 x 40 69.5 us with one step, 71.5 with two and the variances'
+// product renormalised at each factor; 524288 x 64 246 and 244).  The error of the lnL against 80-bit arithmetic, 60 stars of 4 to 64
 // epochs, is 0.74 of that form's in the mean.  Against one lane per row (a serial dot product, one LDS read
 // per multiply-add, 64 rows' columns in LDS): 2^18 rows x 40 epochs 182 ->
 // 75 us, 524288 x 64 1383 -> 245 us, 3000 x 64 84 -> 17 us, 2^18 x 5 30 ->
@@ -1146,7 +1146,11 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev 
                 if constexpr (PHYS) {
                     const double vk = w + o.s2;
                     w = jk_rcp2(vk);
-                    prod *= vk;      // at most four factors between renormalisations
+                    // renormalised at every factor: any finite variance keeps
+                    // its logarithm
+                    int ex;
+                    prod = frexp(prod * vk, &ex);
+                    pexp += ex;
                 }
                 const double wm = w * m;
                 Smm = fma(wm, m, Smm);
@@ -1166,11 +1170,6 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev 
                     }
                 }
                 if constexpr (PHYS) Srr = fma(w * rp, rp, Srr);
-            }
-            if constexpr (PHYS) {
-                int ex;
-                prod = frexp(prod, &ex);
-                pexp += ex;
             }
         }
         Smm = jk_cov_sum(Smm);
