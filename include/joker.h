@@ -9,7 +9,10 @@
  *     L x L system is singular, NaN for invalid rows).
  *   - Array arguments of the compute entry points are DEVICE pointers (HBM,
  *     e.g. torch tensors' data_ptr()).  `stream` is a hipStream_t passed as
- *     void* (NULL = the default stream).  Calls are asynchronous on `stream`.
+ *     void* (NULL = the default stream).  Calls are asynchronous on `stream`,
+ *     except jk_reject_batch, jk_reject_batch_zero_check, jk_polish_batch,
+ *     jk_settle_batch, jk_settle_reject_batch and jk_settle_live_batch, which
+ *     return with it synchronised.
  *   - Prior rows are structure-of-arrays columns P [day], e, omega [rad],
  *     M0 [rad], s [RV unit] -- the packed order of fast_likelihood.pyx:41 with
  *     the array-of-structs chunk split into columns.
@@ -385,7 +388,9 @@ int jk_lnl_prune_batch(const jk_batch *batch, const jk_batch *probes, const doub
 
 /* Segmented rejection step (jk_reject per segment, one launch sequence for
  * all): segs is a HOST array of n_seg descriptors; n_pass_out[i] and
- * llmax_out[i] (device) receive segment i's pass count and maximum. */
+ * llmax_out[i] receive segment i's pass count and maximum.  The outputs are
+ * device memory, or pinned host memory: the launches only write them, and the
+ * call returns with the stream synchronised. */
 int jk_reject_batch(const double *ll, int n_seg, const jk_segment *segs, int64_t *idx_out,
                     int64_t *n_pass_out, double *llmax_out, void *stream);
 
@@ -455,8 +460,9 @@ int jk_settle_batch(const jk_batch *batch, int n_seg, const jk_settle_segment *s
  * pass decides every row the bound leaves no doubt about and flags the
  * others, which are re-evaluated in FP64 and decided from their own uniform.
  * Same accepted set, n_pass and maximum as the two calls; n_settled_out[i]
- * counts segment i's re-evaluated rows.  segs is a HOST array.  No reference
- * counterpart. */
+ * counts segment i's re-evaluated rows.  segs is a HOST array; the outputs
+ * may be pinned host memory, and the call returns with the stream
+ * synchronised, as in jk_reject_batch.  No reference counterpart. */
 int jk_settle_reject_batch(const jk_batch *batch, int n_seg, const jk_settle_segment *segs,
                            int64_t max_keep, const double *P, const double *e,
                            const double *omega, const double *M0, const double *s,

@@ -287,9 +287,9 @@ def reject_batch(ll, offsets, sizes, rng_states, max_keep, stream_offsets=None, 
         segs["inc_hi"][i], segs["inc_lo"][i] = _split(int(inc))
     if stream_offsets is not None:
         segs["stream_offset"] = stream_offsets
-    # one device block [n_pass (n_seg), max (n_seg), zero (n_seg), idx...],
-    # one copy back
-    res = torch.empty(3 * n_seg + max(int(mk.sum()), 1), dtype=torch.int64, device=ll.device)
+    # one pinned host block [n_pass (n_seg), max (n_seg), zero (n_seg), idx...]
+    # that the launches write; the call waits for them
+    res = torch.empty(3 * n_seg + max(int(mk.sum()), 1), dtype=torch.int64, pin_memory=True)
     p = res.data_ptr()
     args = [_dptr(ll), n_seg, segs.ctypes.data_as(ctypes.c_void_p),
             ctypes.c_void_p(p + 24 * n_seg), ctypes.c_void_p(p), ctypes.c_void_p(p + 8 * n_seg)]
@@ -298,7 +298,7 @@ def reject_batch(ll, offsets, sizes, rng_states, max_keep, stream_offsets=None, 
                                                   _stream(device)), "jk_reject_batch_zero_check")
     else:
         _lib.check(lib.jk_reject_batch(*args, _stream(device)), "jk_reject_batch")
-    h = to_host(res)
+    h = res.numpy()
     n_pass = h[:n_seg].copy()
     mx = h[n_seg:2 * n_seg].view(np.float64).copy()
     idx_h = h[3 * n_seg:]
@@ -385,8 +385,9 @@ def settle_reject_batch(batch, cache, ll, bound, offsets, sizes, rng_states, max
         segs["stream_offset"] = stream_offsets
     keep = np.minimum(sizes, int(max_keep))
     keep_off = np.concatenate([[0], np.cumsum(keep)[:-1]]).astype(np.int64)
-    # one device block [n_pass | llmax | n_settled | kept indices], one copy back
-    res = torch.empty(3 * n_seg + max(int(keep.sum()), 1), dtype=torch.int64, device=ll.device)
+    # one pinned host block [n_pass | llmax | n_settled | kept indices] that
+    # the launches write; the call waits for them
+    res = torch.empty(3 * n_seg + max(int(keep.sum()), 1), dtype=torch.int64, pin_memory=True)
     p = res.data_ptr()
     _lib.check(lib.jk_settle_reject_batch(
         batch.handle, n_seg, segs.ctypes.data_as(ctypes.c_void_p), int(max_keep), _dptr(cache.P),
@@ -394,7 +395,7 @@ def settle_reject_batch(batch, cache, ll, bound, offsets, sizes, rng_states, max
         _dptr(ll), _dptr(bound), ctypes.c_void_p(p + 24 * n_seg), ctypes.c_void_p(p),
         ctypes.c_void_p(p + 8 * n_seg), ctypes.c_void_p(p + 16 * n_seg), _stream(device)),
         "jk_settle_reject_batch")
-    h = to_host(res)
+    h = res.numpy()
     n_pass = h[:n_seg].copy()
     mx = h[n_seg:2 * n_seg].view(np.float64).copy()
     settled = h[2 * n_seg:3 * n_seg].copy()

@@ -148,27 +148,39 @@ hipError_t scratch_get(hipStream_t st, size_t bytes, void **out, ScratchLease *l
 }
 
 // The descriptors of a segmented call on their way to the device, ordered on
-// the stream.  Up to JK_SEG_ARGS (one launch) go as kernel arguments and the
-// call returns without waiting; more go by a copy from the (pageable) host
-// array, which must outlive it: done() then waits for the stream.  One segment
-// of 2^22 rows settled, lnL included: 299 us by the copy, 276 by arguments; a
-// pruned rejection of 2^21 rows 364 and 302.  From about eight segments on the
-// copy is the faster (8: 114 against 124 us, 28: 147 against 159 with 28
-// descriptors per launch): the results' copy back is then larger and starts
-// sooner on an idle stream.  A call with host descriptors is refused under
-// capture (a replay could not read them again).
+// the stream.  Up to JK_SEG_ARGS (one launch) go as kernel arguments, more by a
+// copy from the (pageable) host array, which must outlive it.  Such a copy
+// also holds the call's launches back until the work before it on the stream is
+// done, where those behind an argument launch queue up meanwhile.  With the
+// results copied back after the call, one segment of 2^22 rows settled, lnL
+// included, took 299 us by the copy and 276 by arguments, a pruned rejection of
+// 2^21 rows 364 and 302, but 8 segments 114 and 124, and 28 147 and 159 (28
+// descriptors per launch).
+// done(): the wait at the end.  jk_reject_batch, its zero check, jk_polish_batch,
+// jk_settle_batch, jk_settle_reject_batch and jk_settle_live_batch promise
+// that the stream is idle when they return, whatever the number of segments;
+// the others (promised = false) wait for the copy only.  The promise costs 25 us
+// where a copy of the results follows it and nothing where the launches write
+// them to the pinned block the caller reads (the two calls above: 309 and 327 us
+// with the copy, 273 and 296 without).
+// A call with host descriptors is refused under capture (a replay could not
+// read them again).
 struct SegUpload {
-    bool wait = false;
+    bool copied = false, refused = false;
 
     hipError_t put(SegDev *dst, const std::vector<SegDev> &h, const ScratchLease &lease,
                    hipStream_t st)
     {
-        if (lease.pooled) return hipErrorStreamCaptureUnsupported;
+        refused = lease.pooled;
+        if (refused) return hipErrorStreamCaptureUnsupported;
         if (h.size() <= JK_SEG_ARGS) return jk_put_segs(dst, h.data(), (int)h.size(), st);
-        wait = true;
+        copied = true;
         return hipMemcpyAsync(dst, h.data(), sizeof(SegDev) * h.size(), hipMemcpyHostToDevice, st);
     }
-    hipError_t done(hipStream_t st) const { return wait ? hipStreamSynchronize(st) : hipSuccess; }
+    hipError_t done(hipStream_t st, bool promised = true) const
+    {
+        return copied || (promised && !refused) ? hipStreamSynchronize(st) : hipSuccess;
+    }
 };
 
 hipError_t scratch_put(hipStream_t st, void *ptr, ScratchLease &lease)
@@ -1148,28 +1160,31 @@ int jk_settle_reject_batch(const jk_batch *batch, int n_seg, const jk_settle_seg
     hipStream_t st = (hipStream_t)stream;
     const size_t seg_bytes = sizeof(SegDev) * n_seg;
     const size_t seg_pad = ((seg_bytes + 255) / 256) * 256;
-    const size_t bytes = 2 * seg_pad + sizeof(double) * (2 * (size_t)pb * n_seg) +
+    const size_t bytes = 2 * seg_pad + sizeof(double) * (2 * (size_t)pb * n_seg + n_seg) +
                          sizeof(uint64_t) * (mask_words + n_seg) +
-                         sizeof(int64_t) * (bsum_n + idx_n + 2 * (size_t)n_seg + 1);
+                         sizeof(int64_t) * (bsum_n + idx_n + 3 * (size_t)n_seg + 1);
     char *scratch = nullptr;
     ScratchLease lease;
     if (scratch_get(st, bytes, (void **)&scratch, &lease) != hipSuccess) return JK_ENOMEM;
     SegDev *d_settle = (SegDev *)scratch;
     SegDev *d_reject = (SegDev *)(scratch + seg_pad);
     double *partials = (double *)(scratch + 2 * seg_pad);
-    unsigned long long *key = (unsigned long long *)(partials + 2 * (size_t)pb * n_seg);
+    double *llmax = partials + 2 * (size_t)pb * n_seg;
+    unsigned long long *key = (unsigned long long *)(llmax + n_seg);
     uint64_t *mask = (uint64_t *)(key + n_seg);
     int64_t *bsum = (int64_t *)(mask + mask_words);
     int64_t *idx = bsum + bsum_n;
     int64_t *cum = idx + idx_n;
     int64_t *count1 = cum + n_seg + 1;
+    int64_t *count2 = count1 + n_seg;
     SegUpload up;
     hipError_t err = up.put(d_settle, hs, lease, st);
     if (err == hipSuccess)
         err = up.put(d_reject, hr, lease, st);
     if (err == hipSuccess)
         err = jk_launch_settle_reject_batch(batch, n_seg, d_settle, d_reject, max_n, max_nb,
-                                            partials, pb, mask, bsum, idx, key, cum, count1, P, e, omega, M0, s, rows, ll_inout,
+                                            partials, pb, mask, bsum, idx, key, cum, count1,
+                                            count2, llmax, P, e, omega, M0, s, rows, ll_inout,
                                             bound_inout, idx_out, n_pass_out, llmax_out,
                                             n_settled_out, st);
     hipError_t err3 = up.done(st);
@@ -1244,7 +1259,7 @@ static int settle_new_rows(int mode, const jk_batch *batch, int n_seg,
         err = jk_launch_settle_pruned_batch(batch, n_seg, d_segs, max_n, partials, pb, idx, cum,
                                             count1, P, e, omega, M0, s, rows, ll_inout,
                                             bound_inout, window, margin, n_settled_out, st);
-    hipError_t err3 = up.done(st);
+    hipError_t err3 = up.done(st, mode == SETTLE_LIVE);
     hipError_t err2 = scratch_put(st, scratch, lease);
     if (err != hipSuccess || err3 != hipSuccess) return JK_EHIP;
     return check_hip(err2);
@@ -1297,10 +1312,10 @@ struct jk_seg_plan {
     hipEvent_t staged;                         // the last staging copy has been read
     char *mem;                                 // device: descriptors + scratch
     SegDev *d_settle, *d_reject;
-    double *partials;
+    double *partials, *llmax;
     unsigned long long *key;
     uint64_t *mask;
-    int64_t *bsum, *idx, *cum, *count1;
+    int64_t *bsum, *idx, *cum, *count1, *count2;
 };
 
 static void plan_fill_streams(jk_seg_plan *p, const uint64_t *streams)
@@ -1390,9 +1405,9 @@ int jk_seg_plan_create(const jk_batch *batch, int n_seg, const jk_settle_segment
     const size_t seg_bytes = sizeof(SegDev) * n_seg;
     const size_t seg_pad = ((seg_bytes + 255) / 256) * 256;
     const size_t bytes = 2 * seg_pad +
-                         sizeof(double) * (2 * (size_t)pb * n_seg) +
+                         sizeof(double) * (2 * (size_t)pb * n_seg + n_seg) +
                          sizeof(uint64_t) * (mask_words + n_seg) +
-                         sizeof(int64_t) * (bsum_n + idx_n + 2 * (size_t)n_seg + 1);
+                         sizeof(int64_t) * (bsum_n + idx_n + 3 * (size_t)n_seg + 1);
     if (hipMalloc((void **)&p->mem, bytes) != hipSuccess ||
         hipHostMalloc((void **)&p->pinned, 2 * seg_bytes, hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&p->staged, hipEventDisableTiming) != hipSuccess) {
@@ -1402,12 +1417,14 @@ int jk_seg_plan_create(const jk_batch *batch, int n_seg, const jk_settle_segment
     p->d_settle = (SegDev *)p->mem;
     p->d_reject = (SegDev *)(p->mem + seg_pad);
     p->partials = (double *)(p->mem + 2 * seg_pad);
-    p->key = (unsigned long long *)(p->partials + 2 * (size_t)pb * n_seg);
+    p->llmax = p->partials + 2 * (size_t)pb * n_seg;
+    p->key = (unsigned long long *)(p->llmax + n_seg);
     p->mask = (uint64_t *)(p->key + n_seg);
     p->bsum = (int64_t *)(p->mask + mask_words);
     p->idx = p->bsum + bsum_n;
     p->cum = p->idx + idx_n;
     p->count1 = p->cum + n_seg + 1;
+    p->count2 = p->count1 + n_seg;
     if (hipMemcpy(p->d_settle, p->h_settle.data(), seg_bytes, hipMemcpyHostToDevice) !=
             hipSuccess ||
         hipMemcpy(p->d_reject, p->h_reject.data(), seg_bytes, hipMemcpyHostToDevice) !=
@@ -1467,8 +1484,8 @@ int jk_seg_plan_settle_reject(const jk_seg_plan *p, const double *P, const doubl
     if (current_device_inited() < 0) return JK_ENODEV;
     return check_hip(jk_launch_settle_reject_batch(
         p->batch, p->n_seg, p->d_settle, p->d_reject, p->max_n, p->max_nb, p->partials, p->pb,
-        p->mask, p->bsum, p->idx, p->key, p->cum, p->count1, P, e, omega, M0, s, rows, ll_inout,
-        bound_inout, idx_out, n_pass_out, llmax_out, n_settled_out, (hipStream_t)stream));
+        p->mask, p->bsum, p->idx, p->key, p->cum, p->count1, p->count2, p->llmax, P, e, omega, M0,
+        s, rows, ll_inout, bound_inout, idx_out, n_pass_out, llmax_out, n_settled_out, (hipStream_t)stream));
 }
 
 int jk_seg_plan_reject(const jk_seg_plan *p, const double *ll, int64_t *idx_out,

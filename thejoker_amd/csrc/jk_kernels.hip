@@ -2510,17 +2510,24 @@ __global__ __launch_bounds__(256) void k_seg_flags(const double *__restrict__ ll
     }
 }
 
-// With add_from, add_to[segment] += add_from[segment] as well.
+// With n_settled_out, the segment's results that later launches of a settling
+// sequence no longer change are written too: the rows of both its lists and the
+// settled maximum.
 __global__ __launch_bounds__(256) void k_seg_bsum(const SegDev *__restrict__ segs,
                                                   const uint64_t *__restrict__ mask,
                                                   int64_t *__restrict__ bsum,
-                                                  const int64_t *__restrict__ add_from = nullptr,
-                                                  int64_t *__restrict__ add_to = nullptr)
+                                                  const int64_t *__restrict__ count1 = nullptr,
+                                                  const int64_t *__restrict__ count2 = nullptr,
+                                                  const double *__restrict__ llmax = nullptr,
+                                                  int64_t *__restrict__ n_settled_out = nullptr,
+                                                  double *__restrict__ llmax_out = nullptr)
 {
     __shared__ int64_t red[4];
     const SegDev sg = segs[blockIdx.y];
-    if (add_from && blockIdx.x == 0 && threadIdx.x == 0)
-        add_to[blockIdx.y] += add_from[blockIdx.y];
+    if (n_settled_out && blockIdx.x == 0 && threadIdx.x == 0) {
+        n_settled_out[blockIdx.y] = count1[blockIdx.y] + count2[blockIdx.y];
+        llmax_out[blockIdx.y] = llmax[blockIdx.y];
+    }
     if ((int64_t)blockIdx.x >= sg.nb) return;
     const int64_t nwords = (sg.n + 63) / 64;
     const int64_t w0 = (int64_t)blockIdx.x * JK_WORDS_PER_BLOCK;
@@ -2620,7 +2627,7 @@ hipError_t jk_launch_reject_batch(const double *ll, int n_seg, const SegDev *d_s
     hipLaunchKernelGGL(k_seg_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, d_segs, partials,
                        pb, llmax_out, AT, DT, mask, zero_u);
     hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum, nullptr, nullptr);
+                       mask, bsum, nullptr, nullptr, nullptr, nullptr, nullptr);
     hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
                        mask, bsum, idx_out, n_pass_out);
     return hipGetLastError();
@@ -2946,7 +2953,7 @@ hipError_t jk_launch_polish_batch(const jk_batch *b, int n_seg, const SegDev *d_
     hipLaunchKernelGGL(k_seg_window_flags, dim3(fb, n_seg), dim3(256), 0, stream, ll, d_segs, llmax,
                        window, mask);
     hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
-                       mask, bsum, nullptr, nullptr);
+                       mask, bsum, nullptr, nullptr, nullptr, nullptr, nullptr);
     hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_segs,
                        mask, bsum, idx, n_polished);
     return launch_seg_scatter(b, n_seg, d_segs, n_polished, cum, idx, P, e, om, M0, s, rows, ll,
@@ -3291,22 +3298,24 @@ __global__ __launch_bounds__(256) void k_seg_patch(const SegDev *__restrict__ se
     }
 }
 
+// The outputs are written once and never read: they may be in host memory.
 hipError_t jk_launch_settle_reject_batch(const jk_batch *b, int n_seg, const SegDev *d_settle,
                                          const SegDev *d_reject, int64_t max_n, int64_t max_nb,
                                          double *partials, int pb, uint64_t *mask, int64_t *bsum,
                                          int64_t *idx, unsigned long long *key, int64_t *cum,
-                                         int64_t *count1, const double *P, const double *e,
-                                         const double *om, const double *M0, const double *s,
-                                         const int64_t *rows, double *ll, float *bound,
-                                         int64_t *idx_out, int64_t *n_pass_out, double *llmax_out,
-                                         int64_t *n_settled, hipStream_t stream)
+                                         int64_t *count1, int64_t *count2, double *llmax,
+                                         const double *P, const double *e, const double *om,
+                                         const double *M0, const double *s, const int64_t *rows,
+                                         double *ll, float *bound, int64_t *idx_out,
+                                         int64_t *n_pass_out, double *llmax_out,
+                                         int64_t *n_settled_out, hipStream_t stream)
 {
     if (n_seg <= 0) return hipSuccess;
     const int fb = jk_seg_flag_blocks(max_n);
     double *partials2 = partials + (size_t)pb * n_seg;
     // 1. the rows that could hold the FP64 maximum, settled
     hipLaunchKernelGGL(k_seg_lo_partial, dim3(pb, n_seg), dim3(256), 0, stream, ll, bound,
-                       d_settle, partials, partials2, pb, count1, n_settled, key);
+                       d_settle, partials, partials2, pb, count1, count2, key);
     hipLaunchKernelGGL(k_seg_shell_list, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound,
                        d_settle, partials, pb, count1, idx);
     hipError_t err = launch_seg_scatter(b, n_seg, d_settle, count1, cum, idx, P, e, om, M0, s,
@@ -3317,16 +3326,16 @@ hipError_t jk_launch_settle_reject_batch(const jk_batch *b, int n_seg, const Seg
     u128 AT, DT;
     jk_pcg_jump_coeffs((uint64_t)fb * 256, &AT, &DT);
     hipLaunchKernelGGL(k_seg_decide, dim3(fb, n_seg), dim3(256), 0, stream, ll, bound, d_settle,
-                       partials2, pb, key, AT, DT, llmax_out, mask, n_settled, idx);
+                       partials2, pb, key, AT, DT, llmax, mask, count2, idx);
     // 3. the open rows in FP64, then their decisions
-    err = launch_seg_scatter(b, n_seg, d_settle, n_settled, cum, idx, P, e, om, M0, s, rows, ll,
+    err = launch_seg_scatter(b, n_seg, d_settle, count2, cum, idx, P, e, om, M0, s, rows, ll,
                              bound, stream);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(k_seg_patch, dim3(4, n_seg), dim3(256), 0, stream, d_settle, n_settled,
-                       idx, ll, llmax_out, mask);
+    hipLaunchKernelGGL(k_seg_patch, dim3(4, n_seg), dim3(256), 0, stream, d_settle, count2, idx,
+                       ll, llmax, mask);
     // 4. the ordered compaction of the accepted rows
     hipLaunchKernelGGL(k_seg_bsum, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream, d_reject,
-                       mask, bsum, count1, n_settled);
+                       mask, bsum, count1, count2, llmax, n_settled_out, llmax_out);
     hipLaunchKernelGGL(k_seg_compact, dim3((unsigned)max_nb, n_seg), dim3(256), 0, stream,
                        d_reject, mask, bsum, idx_out, n_pass_out);
     return hipGetLastError();
