@@ -77,3 +77,33 @@ def test_same_bits_on_both_sides(cache, N, L, ones, mode):
     _, _, n_pass, mx = D.lnl_reject(star, cache, state, 64,
                                     rows=torch.as_tensor(fine, device="cuda"))
     assert mx == want[fine].max() and n_pass >= 1
+
+
+@pytest.mark.parametrize("N,L", [(3, 2), (8, 2), (9, 3), (12, 2), (30, 5), (55, 4), (56, 5),
+                                 (87, 2), (88, 3)])
+@pytest.mark.parametrize("slots", [False, True])
+def test_scatter_line(cache, N, L, slots):
+    """FP64 re-evaluations on both sides of the line where a row's epochs are
+    spread over lanes (4 (N - 8) waves of 64, 320 or 192 at most): the rows' own values,
+    bounds 0 and counts, for tables of stars and of slots."""
+    star = _star(N, L, "physical", True)
+    table = B.StarBatch([star])
+    items, off, total = B.work_items([ROWS], 4096)
+    d_items = B.upload_items(items)
+    want = B.lnl_batch(table, cache, d_items, len(items), total, "f64").cpu().numpy()
+    if slots:
+        table = B.StarBatch.slots(2, L, "physical")
+        table.set(1, star)
+    waves = min(max(4 * (N - 8), 0), 320 if L <= 3 else 192)
+    g = np.random.default_rng(N)
+    for n in sorted({1, max(64 * waves, 1), 64 * waves + 1}):
+        at = np.sort(g.permutation(ROWS)[:n])
+        b = np.zeros(ROWS, dtype=np.float32)
+        b[at] = 1.0
+        ll = torch.full((ROWS,), -1e9, dtype=torch.float64, device="cuda")
+        bound = torch.as_tensor(b, device="cuda")
+        cnt = B.settle_tol_batch(table, cache, ll, bound, [0], [ROWS], stars=[int(slots)], tol=1e-3)
+        got = ll.cpu().numpy()
+        assert int(cnt[0]) == n and (bound.cpu().numpy() == 0).all()
+        assert np.array_equal(got[at], want[at], equal_nan=True)
+        assert (np.delete(got, at) == -1e9).all()

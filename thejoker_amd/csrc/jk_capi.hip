@@ -740,10 +740,12 @@ int jk_batch_create(const jk_star *const *stars, int n_stars, jk_batch **out)
     const int L = stars[0] ? stars[0]->dev.L : 0;
     const int jm = stars[0] ? stars[0]->dev.jitter_mode : 0;
     size_t n_epoch_doubles = 0;
+    int max_epochs = 0;
     for (int i = 0; i < n_stars; ++i) {
         if (!stars[i] || stars[i]->dev.L != L || stars[i]->dev.jitter_mode != jm) return JK_EINVAL;
         if (stars[i]->dev.Qt) return JK_EINVAL;   // full covariance: single-star calls only
         n_epoch_doubles += JK_EPOCH_DOUBLES(stars[i]->dev.n, L - 1);
+        max_epochs = std::max(max_epochs, stars[i]->dev.n);
     }
     jk_batch *b = new (std::nothrow) jk_batch;
     if (!b) return JK_ENOMEM;
@@ -752,6 +754,7 @@ int jk_batch_create(const jk_star *const *stars, int n_stars, jk_batch **out)
     b->L = L;
     b->jitter_mode = jm;
     b->device = dev;
+    b->max_epochs = max_epochs;
     if (hipMalloc((void **)&b->d_stars, sizeof(StarDev) * n_stars) != hipSuccess ||
         hipMalloc(&b->d_epochs, sizeof(double) * n_epoch_doubles) != hipSuccess) {
         (void)hipFree(b->d_stars);
@@ -835,6 +838,10 @@ int jk_batch_set_star(jk_batch *b, int slot, const jk_star *star, void *stream)
     if (star->dev.Qt) return JK_EINVAL;   // full covariance: single-star calls only
     if (star->device != b->device) return JK_EINVAL;
     if (current_device_inited() < 0) return JK_ENODEV;
+    // only chooses between launches that give the same values: a call of another
+    // thread may read it before or after
+    if (star->dev.n > __atomic_load_n(&b->max_epochs, __ATOMIC_RELAXED))
+        __atomic_store_n(&b->max_epochs, star->dev.n, __ATOMIC_RELAXED);
     return check_hip(hipMemcpyAsync(b->d_stars + slot, &star->dev, sizeof(StarDev),
                                     hipMemcpyHostToDevice, (hipStream_t)stream));
 }

@@ -27,6 +27,7 @@ struct jk_batch {
     int jitter_mode;
     int device;
     void *d_epochs;     // epoch arrays of all stars (StarDev pointers point here)
+    int max_epochs;     // most epochs of a star the table holds (slots: has held)
 };
 
 // Internal segment descriptor of the segmented rejection step.

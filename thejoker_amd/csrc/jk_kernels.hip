@@ -2795,13 +2795,28 @@ __device__ __forceinline__ int jk_seg_of(const int64_t *__restrict__ cum, int n_
     return lo;
 }
 
-// Scatters of at most this many padded waves (49152 positions, as the dense
-// launch's line) take the split evaluation, 16 rows to a workgroup or as many
-// more as it takes to fill the grid once.  The FP64 re-evaluations around a
-// maximum are a few hundred rows: 100 epochs 36 -> 18 us, 16 epochs 10.6 ->
-// 8.6 us (8 or 32 rows to a workgroup: the same within 1 us).
-#define JK_SPLIT_SCATTER_WAVES 768
-#define JK_SPLIT_SCATTER_LGR 4
+// Most padded waves of a scatter that take the split evaluation, 16 rows to a
+// workgroup (with 8 or 32 the same within 1 us), for a table of L parameters
+// whose longest star has N epochs: what the split saves grows with the epochs
+// that one lane would walk alone, what it costs with the rows, and with more
+// workgroups than the compute units hold at once (the LDS of one grows with L)
+// it falls behind.  The FP64 re-evaluations around a maximum are a few hundred
+// rows.  One lane per row minus the split, us, L = 2 with jitter: N = 5: 4000
+// rows -2; N = 12: 300 2.8, 4000 -0.7; N = 24: 2000 5.7, 12000 -1.7; N = 40: 6000
+// 7.7, 16000 -0.8; N = 100: 1000 29, 12000 22, 16000 16, 20000 2, 30000 -4; N = 200: 20000 24.
+// L = 6: N = 12: 300 2.7, 4000 -2; N = 24: 2000 6.2, 8000 -3; N = 100: 8000 27,
+// 12000 22, 16000 -3, 30000 -52.
+// (16 as a constant also leaves the one-lane half its own registers: with the
+// rows per workgroup chosen on the device, <3, true> spilled two and <2, false>
+// took 121 VGPRs instead of 97.)
+#define JK_SPLIT_SCATTER_R 16
+static int jk_split_scatter_waves(int N, int L)
+{
+    return std::min(std::max(4 * (N - 8), 0), L <= 3 ? 320 : 192);
+}
+
+// Workgroups of the scatter: at least 4 for each wave of the split.
+#define JK_SCATTER_GRID 2048
 
 // FP64 re-evaluation of every segment's selected entries as one flat list
 // spread over the whole grid: wavefront w takes padded positions
@@ -2810,7 +2825,7 @@ __device__ __forceinline__ int jk_seg_of(const int64_t *__restrict__ cum, int n_
 template <int L, bool PHYS>
 __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_seg_scatter_f64(const StarDev *__restrict__ stars,
                                                          const SegDev *__restrict__ segs,
-                                                         int n_seg,
+                                                         int n_seg, int split_waves,
                                                          const int64_t *__restrict__ count,
                                                          const int64_t *__restrict__ cum_in,
                                                          const int64_t *__restrict__ idx,
@@ -2834,32 +2849,28 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_seg_scatter_f64(const 
         cum = s_cum;
     }
     const int64_t total_waves = cum[n_seg] >> 6;
-    if (total_waves <= JK_SPLIT_SCATTER_WAVES) {
+    if (total_waves <= split_waves) {
         // Few rows: each 64 positions over 64 / R workgroups, a row's epochs
         // over many lanes (jk_rows_split; the same bits).
-        int lgR = JK_SPLIT_SCATTER_LGR;
-        while (lgR < 6 && (total_waves << (6 - lgR)) > gridDim.x) ++lgR;
-        const int R = 1 << lgR, sw = jk_split_wave(blockIdx.x), sl = jk_split_lane(sw),
+        constexpr int R = JK_SPLIT_SCATTER_R;
+        const int sw = jk_split_wave(blockIdx.x), sl = jk_split_lane(sw),
                   row = jk_split_row(sl, R);
-        const int64_t units = total_waves << (6 - lgR);
-        if ((int64_t)blockIdx.x >= units) return;
+        const int64_t j0 = (int64_t)blockIdx.x * R;
+        if (j0 >= total_waves * 64) return;
         jk_stage_tab<false>(s_tab);
-        for (int64_t w = blockIdx.x; w < units; w += gridDim.x) {
-            const int64_t j0 = w << lgR;
-            const int sidx = __builtin_amdgcn_readfirstlane(jk_seg_of(cum, n_seg, j0));
-            const SegDev &sg = segs[sidx];
-            const int64_t local = j0 - cum[sidx] + row;
-            const bool some = row < R && local < count[sidx];
-            const int64_t p = some ? idx[sg.idx_off + local] : 0, q = sg.row0 + p;
-            const double v = jk_rows_split<L, PHYS, false>(
-                stars[sg.star], R, sw, some ? (rows ? rows[q] : q) : -1, P, e_, om_, M0_, s_, s_tab,
-                sh, nullptr);
-            if (some && sl < R) {
-                ll[sg.off + p] = v;
-                if (bound) bound[sg.off + p] = 0.0f;
-            }
-            if (key && sl < 64) jk_wave_max_key(v, some && sl < R, key + sidx);
+        const int sidx = __builtin_amdgcn_readfirstlane(jk_seg_of(cum, n_seg, j0));
+        const SegDev &sg = segs[sidx];
+        const int64_t local = j0 - cum[sidx] + row;
+        const bool some = row < R && local < count[sidx];
+        const int64_t p = some ? idx[sg.idx_off + local] : 0, q = sg.row0 + p;
+        const double v = jk_rows_split<L, PHYS, false>(
+            stars[sg.star], R, sw, some ? (rows ? rows[q] : q) : -1, P, e_, om_, M0_, s_, s_tab,
+            sh, nullptr);
+        if (some && sl < R) {
+            ll[sg.off + p] = v;
+            if (bound) bound[sg.off + p] = 0.0f;
         }
+        if (key && sl < 64) jk_wave_max_key(v, some && sl < R, key + sidx);
         return;
     }
     jk_stage_tab<false>(s_tab);
@@ -2887,13 +2898,16 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_seg_scatter_f64(const 
 template <int L, bool PHYS>
 static void launch_seg_scatter_t(const jk_batch *b, int n_seg, const SegDev *d_segs,
                                  const int64_t *count, const int64_t *cum, const int64_t *idx,
-                                 unsigned long long *key, int gx, const double *P, const void *e,
+                                 unsigned long long *key, const double *P, const void *e,
                                  const void *om, const void *M0, const void *s,
                                  const int64_t *rows, double *ll, float *bound,
                                  hipStream_t stream)
 {
-    hipLaunchKernelGGL((k_seg_scatter_f64<L, PHYS>), dim3(gx), dim3(256), 0, stream, b->d_stars,
-                       d_segs, n_seg, count, cum, idx, key, P, e, om, M0, s, rows, ll, bound);
+    hipLaunchKernelGGL((k_seg_scatter_f64<L, PHYS>), dim3(JK_SCATTER_GRID), dim3(256), 0, stream,
+                       b->d_stars, d_segs, n_seg,
+                       jk_split_scatter_waves(
+                           __atomic_load_n(&b->max_epochs, __ATOMIC_RELAXED), L),
+                       count, cum, idx, key, P, e, om, M0, s, rows, ll, bound);
 }
 
 // FP64 re-evaluation of every segment's list idx (counts in count) as one flat
@@ -2910,16 +2924,15 @@ static hipError_t launch_seg_scatter(const jk_batch *b, int n_seg, const SegDev 
         hipLaunchKernelGGL(k_seg_count_scan, dim3(1), dim3(256), 0, stream, count, n_seg, cum);
     else
         cum = nullptr;
-    const int gx = 2048;
     const bool phys = b->jitter_mode == JK_JITTER_PHYSICAL;
 #define JK_SCASE2(LL)                                                                             \
     case LL:                                                                                      \
         if (phys)                                                                                 \
-            launch_seg_scatter_t<LL, true>(b, n_seg, d_segs, count, cum, idx, key, gx, P, e, om,   \
-                                           M0, s, rows, ll, bound, stream);                       \
+            launch_seg_scatter_t<LL, true>(b, n_seg, d_segs, count, cum, idx, key, P, e, om, M0,   \
+                                           s, rows, ll, bound, stream);                           \
         else                                                                                      \
-            launch_seg_scatter_t<LL, false>(b, n_seg, d_segs, count, cum, idx, key, gx, P, e, om,  \
-                                            M0, s, rows, ll, bound, stream);                      \
+            launch_seg_scatter_t<LL, false>(b, n_seg, d_segs, count, cum, idx, key, P, e, om, M0,  \
+                                            s, rows, ll, bound, stream);                          \
         break;
     switch (b->L) {
         JK_SCASE2(1)
