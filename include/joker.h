@@ -347,8 +347,9 @@ int jk_batch_set_exact(jk_batch *batch, int slot, int exact, void *stream);
  * precision 0: FP64; 1: mixed (as jk_lnl_mixed).  The columns are the FP64
  * ones in both cases.  bound_out (mixed only, optional): per-row error bounds as in
  * jk_lnl_mixed, at the same offsets as ll_out.  block: threads per workgroup
- * (64, 128 or 256); grid: workgroups taken to fill the device (0 = 8 per
- * compute unit): items are split while that leaves at most twice as many.
+ * (64, 128 or 256); grid: the most workgroups the launch may have (each then
+ * takes every grid-th item or part), or 0: one per item or part.  Items are
+ * split while that leaves at most twice grid (0: twice 8 per compute unit).
  * workspace: not used (may be NULL); the call allocates nothing. */
 int jk_lnl_batch(const jk_batch *batch, int precision, int64_t n_items,
                  const jk_work_item *items, const double *P, const void *e, const void *omega,

@@ -6,8 +6,8 @@ of linear parameters is gathered into a device star table (``jk_batch``) and
 evaluated by one launch over (star, row tile) items
 (``jk_lnl_batch``); the rejection step of every star runs as one segmented
 launch sequence (``jk_reject_batch``), each star with its own numpy PCG64
-stream.  :func:`autotune` picks the launch shape (threads per workgroup,
-workgroups, rows per work item) by timing candidates on the actual workload.
+stream.  :func:`autotune` picks the launch shape (threads per workgroup, rows
+per work item) by timing candidates on the actual workload.
 """
 import ctypes
 import time
@@ -64,8 +64,8 @@ SEGMENT_DTYPE = np.dtype([("offset", "<i8"), ("n", "<i8"), ("max_keep", "<i8"),
 
 
 class LaunchShape:
-    """Threads per workgroup, workgroups taken to fill the device (0 = 8 per
-    CU; few items are split to reach them), rows per work item."""
+    """Threads per workgroup, most workgroups of a launch (0 = one per work
+    item; few items are split to fill the device), rows per work item."""
 
     def __init__(self, block=256, grid=0, tile=2048):
         self.block, self.grid, self.tile = int(block), int(grid), int(tile)
@@ -218,7 +218,7 @@ def lnl_batch(batch, cache, d_items, n_items, n_out, precision="mixed", shape=No
               rows=None, workspace=None, bound=None):
     """lnL of every work item into a device float64 tensor of n_out entries;
     with `bound` (mixed only, a device float32 tensor indexed like `out`) each
-    row's bound on |lnL(mixed) - lnL(FP64)| as well."""
+    row's bound on |lnL(mixed) - lnL(FP64)| as well.  `workspace` is not used."""
     torch = _torch()
     lib = _lib.ensure_device(cache.device)
     shape = shape or LaunchShape()
@@ -247,7 +247,8 @@ def lnl_prune_batch(batch, probes, prune, cache, d_items, n_items, precision="mi
     by bound -1.  `bound` is required in mixed precision; in f64 it is
     optional and receives only the marks (0: an FP64 value, -1: an upper
     bound).  n_full: optional device int64 tensor with an entry per table
-    slot, accumulating each star's rows evaluated in full."""
+    slot, accumulating each star's rows evaluated in full.  `workspace` is not
+    used."""
     lib = _lib.ensure_device(cache.device)
     shape = shape or LaunchShape()
     if precision not in ("f64", "mixed"):
@@ -550,10 +551,7 @@ def autotune(batch, cache, n_rows, precision="mixed", candidates=None, sample_st
     torch = _torch()
     n_rows = np.asarray(n_rows, dtype=np.int64)
     if candidates is None:
-        props = torch.cuda.get_device_properties(device)
-        cus = props.multi_processor_count
-        candidates = [LaunchShape(b, g * cus, t) for b in (256, 128) for g in (4, 8, 16)
-                      for t in (1024, 4096)]
+        candidates = [LaunchShape(b, 0, t) for b in (256, 128) for t in (1024, 2048, 4096)]
     sub = min(sample_stars, len(batch))
     results = {}
     best, best_ms = None, np.inf
@@ -780,9 +778,6 @@ class StepGraph:
                       if precision == "mixed" else None)
         self.plan = SegPlan(batch, offsets, sizes, rng_states, max_keep, device=device)
         shape = shape or LaunchShape()
-        if shape.grid <= 0:
-            props = torch.cuda.get_device_properties(device)
-            shape = LaunchShape(shape.block, 8 * props.multi_processor_count, shape.tile)
 
         def body():
             lnl_batch(batch, cache, d_items, n_items, total, precision, shape, out=self.ll,

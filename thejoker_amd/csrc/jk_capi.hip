@@ -884,7 +884,7 @@ int jk_lnl_batch(const jk_batch *batch, int precision, int64_t n_items, const jk
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             return JK_EHIP;
-        grid = 8 * cus;
+        grid = -8 * cus;      // no cap
     }
     return check_hip(jk_launch_lnl_batch(batch, precision, n_items, items, P, e, omega, M0, s, rows,
                                          ll_out, bound_out, block, grid, (hipStream_t)stream));
@@ -912,7 +912,7 @@ int jk_lnl_prune_batch(const jk_batch *batch, const jk_batch *probes, const doub
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             return JK_EHIP;
-        grid = 8 * cus;
+        grid = -8 * cus;      // no cap
     }
     return check_hip(jk_launch_lnl_prune_batch(batch, probes, prune, precision, n_items, items, P,
                                                e, omega, M0, s, ll_out, bound_out,

@@ -15,8 +15,8 @@
 //                          lanes per row).
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
-#include <type_traits>
 
 #include "jk_internal.h"
 
@@ -2072,10 +2072,12 @@ hipError_t jk_put_segs(SegDev *dst, const SegDev *src, int n, hipStream_t stream
 // much for the fetches that found the queue empty) and a launch to clear the
 // counter, more than staging the tables again costs.
 // ---------------------------------------------------------------------------
-// Entries [first, first + gridDim.x) of a launch: each work item as 1 <<
-// lg_parts parts.
+// Entries [first, end) of a launch, each work item as 1 << lg_parts parts: one
+// workgroup per entry, or (CAPPED) the caller's most workgroups, each taking
+// every gridDim.x-th entry.  An instance of its own, since the loop over the
+// entries costs the other registers (L = 4 with jitter, FP64: 126 -> 163 VGPRs).
 struct WorkSplit {
-    int64_t first;
+    int64_t first, end;
     unsigned lg_parts;
 };
 
@@ -2106,12 +2108,22 @@ __device__ __forceinline__ void jk_split_item(const WorkSplit &ws, int64_t q, in
 // gathered to fill waves, and there are fewer in a smaller part (2^21 rows of
 // 100 epochs, the whole call with its rejection: 345 us whole, 337 in two,
 // 335 in four, 340 in eight).
+// grid < 0: -grid workgroups fill the device; grid > 0: the caller's cap, which
+// is then what items are split for.
 #define JK_ITEM_LAUNCH ((int64_t)1 << 23)   // entries per launch (x 256 threads < 2^32)
 static unsigned jk_item_parts(int64_t n_items, int grid)
 {
     unsigned lg = 0;
-    while (lg < 3 && (n_items << (lg + 1)) <= 2 * (int64_t)grid) ++lg;
+    while (lg < 3 && (n_items << (lg + 1)) <= 2 * std::abs((int64_t)grid)) ++lg;
     return lg;
+}
+
+// The end of the launch that starts at ws.first, and its workgroups (cap: 0 for
+// none).
+static unsigned jk_item_launch(int64_t entries, int cap, WorkSplit &ws)
+{
+    ws.end = cap ? entries : std::min(entries, ws.first + JK_ITEM_LAUNCH);
+    return (unsigned)std::min(cap ? cap : ws.end - ws.first, JK_ITEM_LAUNCH);
 }
 
 // One row of a mixed-precision batched launch: in FP64 with error bound 0
@@ -2141,7 +2153,7 @@ __device__ __forceinline__ double jk_lnl_row_sel(const StarDev &st, int64_t r,
 // reads no host memory after it returns.
 __global__ void k_set_exact(StarDev *stars, int slot, int exact) { stars[slot].exact = exact; }
 
-template <int L, bool PHYS, bool MIXED, bool BOUND>
+template <int L, bool PHYS, bool MIXED, bool BOUND, bool CAPPED>
 __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_batch(const StarDev *__restrict__ stars,
                                                    const jk_work_item *__restrict__ items,
                                                    WorkSplit ws,
@@ -2155,28 +2167,33 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_batch(const StarDe
                                                    float *__restrict__ bound)
 {
     __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
-    const int64_t q0 = ws.first + blockIdx.x;
-    const jk_work_item w = items[q0 >> ws.lg_parts];
-    int lo, hi;
-    jk_split_item(ws, q0, w.n_rows, lo, hi);
-    if (lo >= hi) return;
-    jk_stage_tab<MIXED>(s_tab);
-    const StarDev &st = stars[w.star];
-    for (int j = lo + threadIdx.x; j < hi; j += blockDim.x) {
-        const int64_t q = w.row_begin + j;
-        const int64_t r = rows ? rows[q] : q;
-        if constexpr (BOUND) {
-            float b;
-            ll[w.out_offset + j] = jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
-            bound[w.out_offset + j] = b;
-        } else if constexpr (MIXED) {
-            ll[w.out_offset + j] =
-                st.exact ? jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab)
-                         : jk_lnl_row<L, PHYS, true, false, false, false, false, true>(
-                               st, r, P, e_, om_, M0_, s_, s_tab);
-        } else {
-            ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
+    if (CAPPED) jk_stage_tab<MIXED>(s_tab);
+    for (int64_t q0 = ws.first + blockIdx.x; q0 < ws.end; q0 += gridDim.x) {
+        const jk_work_item w = items[q0 >> ws.lg_parts];
+        int lo, hi;
+        jk_split_item(ws, q0, w.n_rows, lo, hi);
+        if (!CAPPED) {
+            if (lo >= hi) return;
+            jk_stage_tab<MIXED>(s_tab);
         }
+        const StarDev &st = stars[w.star];
+        for (int j = lo + threadIdx.x; j < hi; j += blockDim.x) {
+            const int64_t q = w.row_begin + j;
+            const int64_t r = rows ? rows[q] : q;
+            if constexpr (BOUND) {
+                float b;
+                ll[w.out_offset + j] = jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
+                bound[w.out_offset + j] = b;
+            } else if constexpr (MIXED) {
+                ll[w.out_offset + j] =
+                    st.exact ? jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab)
+                             : jk_lnl_row<L, PHYS, true, false, false, false, false, true>(
+                                   st, r, P, e_, om_, M0_, s_, s_tab);
+            } else {
+                ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
+            }
+        }
+        if (!CAPPED) return;
     }
 }
 
@@ -2192,16 +2209,21 @@ static void launch_batch_t(const jk_batch *b, int64_t n_items, const jk_work_ite
                            const void *s, const int64_t *rows, double *ll, float *bound,
                            int block, int grid, hipStream_t stream)
 {
-    WorkSplit ws{0, jk_item_parts(n_items, grid)};
+    WorkSplit ws{0, 0, jk_item_parts(n_items, grid)};
     const int64_t entries = n_items << ws.lg_parts;
-    for (; ws.first < entries; ws.first += JK_ITEM_LAUNCH) {
-        const dim3 blocks((unsigned)std::min(entries - ws.first, JK_ITEM_LAUNCH));
+    const bool capped = grid > 0 && entries > grid;
+    for (; ws.first < entries; ws.first = ws.end) {
+        const dim3 blocks(jk_item_launch(entries, capped ? grid : 0, ws));
         if (MIXED && bound)
-            hipLaunchKernelGGL((k_lnl_batch<L, PHYS, MIXED, MIXED>), blocks, dim3(block), 0, stream,
-                               b->d_stars, items, ws, P, e, om, M0, s, rows, ll, bound);
+            hipLaunchKernelGGL((capped ? k_lnl_batch<L, PHYS, MIXED, MIXED, true>
+                                       : k_lnl_batch<L, PHYS, MIXED, MIXED, false>),
+                               blocks, dim3(block), 0, stream, b->d_stars, items, ws, P, e, om, M0,
+                               s, rows, ll, bound);
         else
-            hipLaunchKernelGGL((k_lnl_batch<L, PHYS, MIXED, false>), blocks, dim3(block), 0, stream,
-                               b->d_stars, items, ws, P, e, om, M0, s, rows, ll, nullptr);
+            hipLaunchKernelGGL((capped ? k_lnl_batch<L, PHYS, MIXED, false, true>
+                                       : k_lnl_batch<L, PHYS, MIXED, false, false>),
+                               blocks, dim3(block), 0, stream, b->d_stars, items, ws, P, e, om, M0,
+                               s, rows, ll, nullptr);
     }
 }
 
@@ -2271,7 +2293,7 @@ hipError_t jk_launch_lnl_batch(const jk_batch *b, int precision, int64_t n_items
 // ---------------------------------------------------------------------------
 #define JK_PRUNE_LIST 2048   // survivors held in LDS before their evaluation
 
-template <int L, bool PHYS, bool MIXED>
+template <int L, bool PHYS, bool MIXED, bool CAPPED>
 __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const StarDev *__restrict__ stars,
                                                          const StarDev *__restrict__ probes,
                                                          const double2 *__restrict__ prune,
@@ -2289,85 +2311,91 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const 
     __shared__ int s_n;
     __shared__ int s_list[JK_PRUNE_LIST];
     __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
-    const int64_t q0 = ws.first + blockIdx.x;
-    const jk_work_item w = items[q0 >> ws.lg_parts];
-    int lo, hi;
-    jk_split_item(ws, q0, w.n_rows, lo, hi);
-    if (lo >= hi) return;
-    jk_stage_tab<MIXED>(s_tab);
-    const StarDev &st = stars[w.star];
-    const double2 pr = prune[w.star];
-    if (!(pr.x > -INFINITY)) {
-        for (int j = lo + (int)threadIdx.x; j < hi; j += blockDim.x) {
-            const int64_t r = w.row_begin + j;
-            if constexpr (MIXED) {
-                float b;
-                ll[w.out_offset + j] =
-                    jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
-                bound[w.out_offset + j] = b;
-            } else {
-                ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
-                if (bound) bound[w.out_offset + j] = 0.0f;
-            }
+    if (CAPPED) jk_stage_tab<MIXED>(s_tab);
+    for (int64_t q0 = ws.first + blockIdx.x; q0 < ws.end; q0 += gridDim.x) {
+        const jk_work_item w = items[q0 >> ws.lg_parts];
+        int lo, hi;
+        jk_split_item(ws, q0, w.n_rows, lo, hi);
+        if (!CAPPED) {
+            if (lo >= hi) return;
+            jk_stage_tab<MIXED>(s_tab);
         }
-        if (n_full && threadIdx.x == 0)
-            atomicAdd(n_full + w.star, (unsigned long long)(hi - lo));
-        return;
-    }
-    const StarDev &pb = probes[w.star];
-    unsigned n_surv = 0;
-    if (threadIdx.x == 0) s_n = 0;
-    __syncthreads();
-    for (int base = lo; base < hi; base += blockDim.x) {
-        const int j = base + (int)threadIdx.x;
-        if (j < hi) {
-            const int64_t r = w.row_begin + j;
-            double v;
-            if constexpr (MIXED) {
-                float b;
-                v = jk_lnl_row<L, PHYS, true, false, true>(pb, r, P, e_, om_, M0_, s_, s_tab, &b);
-                v += (double)b + pr.y;
-            } else {
-                v = jk_lnl_row<L, PHYS, false>(pb, r, P, e_, om_, M0_, s_, s_tab);
-                // FP64 rounding of both evaluations, far below this slack
-                v += pr.y + 1e-9 * (1.0 + fabs(v));
-            }
-            if (isfinite(v) && v < pr.x) {
-                ll[w.out_offset + j] = v;
-                if (bound) bound[w.out_offset + j] = JK_BOUND_UPPER;
-            } else {
-                s_list[atomicAdd(&s_n, 1)] = j;
-            }
-        }
-        __syncthreads();
-        // Survivors gather over chunks and are evaluated once another
-        // chunk might overflow the list, or at the item's end: the full
-        // evaluations then run on whole waves.
-        const int ns = s_n;
-        __syncthreads();   // every thread holds ns before the next append
-        if (ns > JK_PRUNE_LIST - (int)blockDim.x || base + (int)blockDim.x >= hi) {
-            n_surv += (unsigned)ns;
-            for (int k = threadIdx.x; k < ns; k += blockDim.x) {
-                const int jj = s_list[k];
-                const int64_t r = w.row_begin + jj;
+        const StarDev &st = stars[w.star];
+        const double2 pr = prune[w.star];
+        if (!(pr.x > -INFINITY)) {
+            for (int j = lo + (int)threadIdx.x; j < hi; j += blockDim.x) {
+                const int64_t r = w.row_begin + j;
                 if constexpr (MIXED) {
                     float b;
-                    ll[w.out_offset + jj] =
+                    ll[w.out_offset + j] =
                         jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
-                    bound[w.out_offset + jj] = b;
+                    bound[w.out_offset + j] = b;
                 } else {
-                    ll[w.out_offset + jj] =
-                        jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
-                    if (bound) bound[w.out_offset + jj] = 0.0f;
+                    ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
+                    if (bound) bound[w.out_offset + j] = 0.0f;
                 }
             }
-            __syncthreads();   // every read of s_list before it is reset
-            if (threadIdx.x == 0) s_n = 0;
-            __syncthreads();
+            if (n_full && threadIdx.x == 0)
+                atomicAdd(n_full + w.star, (unsigned long long)(hi - lo));
+            if (CAPPED) continue;
+            return;
         }
+        const StarDev &pb = probes[w.star];
+        unsigned n_surv = 0;
+        if (threadIdx.x == 0) s_n = 0;
+        __syncthreads();
+        for (int base = lo; base < hi; base += blockDim.x) {
+            const int j = base + (int)threadIdx.x;
+            if (j < hi) {
+                const int64_t r = w.row_begin + j;
+                double v;
+                if constexpr (MIXED) {
+                    float b;
+                    v = jk_lnl_row<L, PHYS, true, false, true>(pb, r, P, e_, om_, M0_, s_, s_tab, &b);
+                    v += (double)b + pr.y;
+                } else {
+                    v = jk_lnl_row<L, PHYS, false>(pb, r, P, e_, om_, M0_, s_, s_tab);
+                    // FP64 rounding of both evaluations, far below this slack
+                    v += pr.y + 1e-9 * (1.0 + fabs(v));
+                }
+                if (isfinite(v) && v < pr.x) {
+                    ll[w.out_offset + j] = v;
+                    if (bound) bound[w.out_offset + j] = JK_BOUND_UPPER;
+                } else {
+                    s_list[atomicAdd(&s_n, 1)] = j;
+                }
+            }
+            __syncthreads();
+            // Survivors gather over chunks and are evaluated once another
+            // chunk might overflow the list, or at the item's end: the full
+            // evaluations then run on whole waves.
+            const int ns = s_n;
+            __syncthreads();   // every thread holds ns before the next append
+            if (ns > JK_PRUNE_LIST - (int)blockDim.x || base + (int)blockDim.x >= hi) {
+                n_surv += (unsigned)ns;
+                for (int k = threadIdx.x; k < ns; k += blockDim.x) {
+                    const int jj = s_list[k];
+                    const int64_t r = w.row_begin + jj;
+                    if constexpr (MIXED) {
+                        float b;
+                        ll[w.out_offset + jj] =
+                            jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
+                        bound[w.out_offset + jj] = b;
+                    } else {
+                        ll[w.out_offset + jj] =
+                            jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
+                        if (bound) bound[w.out_offset + jj] = 0.0f;
+                    }
+                }
+                __syncthreads();   // every read of s_list before it is reset
+                if (threadIdx.x == 0) s_n = 0;
+                __syncthreads();
+            }
+        }
+        if (n_full && threadIdx.x == 0 && n_surv)
+            atomicAdd(n_full + w.star, (unsigned long long)n_surv);
+        if (!CAPPED) return;
     }
-    if (n_full && threadIdx.x == 0 && n_surv)
-        atomicAdd(n_full + w.star, (unsigned long long)n_surv);
 }
 
 template <int L, bool PHYS, bool MIXED>
@@ -2377,13 +2405,16 @@ static void launch_prune_t(const jk_batch *b, const jk_batch *pb, const double2 
                            double *ll, float *bound, unsigned long long *n_full, int block,
                            int grid, hipStream_t stream)
 {
-    WorkSplit ws{0, std::min(2u, jk_item_parts(n_items, grid))};
+    WorkSplit ws{0, 0, std::min(2u, jk_item_parts(n_items, grid))};
     const int64_t entries = n_items << ws.lg_parts;
-    for (; ws.first < entries; ws.first += JK_ITEM_LAUNCH)
-        hipLaunchKernelGGL((k_lnl_prune_batch<L, PHYS, MIXED>),
-                           dim3((unsigned)std::min(entries - ws.first, JK_ITEM_LAUNCH)),
-                           dim3(block), 0, stream, b->d_stars, pb->d_stars, prune, items, ws, P, e,
-                           om, M0, s, ll, bound, n_full);
+    const bool capped = grid > 0 && entries > grid;
+    for (; ws.first < entries; ws.first = ws.end) {
+        const dim3 blocks(jk_item_launch(entries, capped ? grid : 0, ws));
+        hipLaunchKernelGGL((capped ? k_lnl_prune_batch<L, PHYS, MIXED, true>
+                                   : k_lnl_prune_batch<L, PHYS, MIXED, false>),
+                           blocks, dim3(block), 0, stream, b->d_stars, pb->d_stars, prune, items,
+                           ws, P, e, om, M0, s, ll, bound, n_full);
+    }
 }
 
 hipError_t jk_launch_lnl_prune_batch(const jk_batch *b, const jk_batch *pb, const double *prune,
