@@ -5,6 +5,8 @@
 //                          lane per prior sample; the star's epoch arrays are
 //                          wave-uniform and read through scalar loads.
 //  k_lnl_split             the same for few rows, a row's epochs over many lanes.
+//  k_lnl_cov               the same for a full covariance, rotated on the matrix
+//                          cores.
 //  k_max_partial / final   NaN-propagating max (np.max).
 //  k_reject_words / rows   numpy-PCG64 uniforms generated in registers for the
 //                          rows that can pass, exp(ll - max) > u, one 64-bit
@@ -59,8 +61,9 @@ __device__ double2 g_log_tab[JK_LOG_TAB_N];
 
 // Minimum waves per SIMD asked of the row kernels that evaluate many stars
 // or scattered rows: 4 (at most 128 VGPRs) for L <= 3, where the allocator
-// otherwise settled some variants at 129-132 VGPRs and 3 waves without
-// spilling at 128; none for larger L, which would spill.
+// otherwise settled some variants at 129-132 VGPRs and 3 waves (at 128 none of
+// them spills, but for two VGPRs of the capped pruned launch at L = 3 in mixed
+// precision with jitter); none for larger L, which would spill.
 #define JK_ROW_WAVES(L) ((L) <= 3 ? 4 : 1)
 
 // F32: with the FP32 grid of the mixed-precision row.
@@ -524,9 +527,9 @@ __device__ __forceinline__ double jk_row_finish(const StarDev &st, double lam0,
 // With REC the epoch loop reads the epochs' records (StarDev::ep: one base
 // address, so few scalar registers and one or two scalar loads per epoch),
 // else the separate arrays.  Same values either way; which is faster is the
-// register allocator's doing: the FP64 rows (their separate arrays spilled
-// scalars into vector lanes: 2^24 rows x 16 epochs 957 -> 927 us with the
-// operations saved above, 2^20 x 37 at L = 5 134 -> 127 us) and the mixed
+// register allocator's doing: the FP64 rows (2^24 rows x 16 epochs 957 -> 927 us
+// with the operations saved above; 2^20 x 37 at L = 5 134 -> 127 us, where scalars
+// spilled into vector lanes went from 72 to 30) and the mixed
 // rows of many stars (64 x 2^18 rows 1935 -> 1895 us) take the records, the
 // mixed single-star row the arrays (2^22 x 50: 394 us, with records 415).
 // LONE: the row of a launch of at most one wave per SIMD (k_lnl).
@@ -1237,7 +1240,7 @@ static hipError_t launch_lnl_cov(const jk_star *st, int64_t n, const double *P, 
 #undef JK_CCASE
 }
 
-// Scatter launch over a device-resident index list: for j < *count,// Scatter launch over a device-resident index list: for j < *count,
+// Scatter launch over a device-resident index list: for j < *count,
 // i = idx[j], ll[i] = lnL(row rows[i] or i).  Grid-stride, so the host does
 // not need the count.
 template <int L, bool PHYS>
@@ -3010,7 +3013,7 @@ hipError_t jk_launch_polish_batch(const jk_batch *b, int n_seg, const SegDev *d_
 // |lnL(mixed) - lnL(FP64)| (0 for rows already FP64):
 //   1. lo = max(ll - B) is a lower bound on the FP64 maximum; a row with
 //      ll + B >= lo could be the maximum: re-evaluate it in FP64 (B := 0).
-//      So is a row with ll + B >= lo - 40 and B > 1e-3 (k_seg_shell_flags).
+//      So is a row with ll + B >= lo - 40 and B > 1e-3 (k_seg_shell_list).
 //      A NaN anywhere makes lo NaN and every unsettled row is re-evaluated.
 //   2. mx = max(ll) is then the FP64 maximum.
 //   3. u = the row's numpy uniform (the stream the rejection step draws); a
