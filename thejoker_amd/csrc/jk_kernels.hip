@@ -65,6 +65,15 @@ __device__ double2 g_log_tab[JK_LOG_TAB_N];
 // them spills, but for two VGPRs of the capped pruned launch at L = 3 in mixed
 // precision with jitter); none for larger L, which would spill.
 #define JK_ROW_WAVES(L) ((L) <= 3 ? 4 : 1)
+// The pruned launch with jitter asks for them at L = 4 too (171 VGPRs and 2
+// waves in FP64 otherwise: 2^20 rows x 60 epochs 158 -> 96 us; mixed 106 -> 83,
+// with three VGPRs spilled), and in mixed precision for 3 at L = 6, with one
+// epoch at a time: 1024 and 2048 items of 2048 rows, 24 to 150 epochs, with and
+// without survivors, 0.97 to 1.14 times as fast as a persistent grid was; two
+// epochs at a time on 2 waves 0.87 to 1.04, on 3 waves 0.87 to 1.12.
+#define JK_PRUNE_WAVES(L, PHYS, MIXED)                                                            \
+    ((L) <= 3 || ((PHYS) && (L) == 4) ? 4 : ((PHYS) && (MIXED) && (L) == 6 ? 3 : 1))
+#define JK_PRUNE_UNROLL(L, PHYS) ((PHYS) && (L) == 6 ? 1 : 2)
 
 // F32: with the FP32 grid of the mixed-precision row.
 template <bool F32>
@@ -533,8 +542,12 @@ __device__ __forceinline__ double jk_row_finish(const StarDev &st, double lam0,
 // rows of many stars (64 x 2^18 rows 1935 -> 1895 us) take the records, the
 // mixed single-star row the arrays (2^22 x 50: 394 us, with records 415).
 // LONE: the row of a launch of at most one wave per SIMD (k_lnl).
+// U: epochs per turn of the loop, four where every fourth renormalises the
+// product and the registers allow it (2^24 rows x 16 epochs 936 -> 930 us), else
+// two.
 template <int L, bool PHYS, bool MIXED, bool SAFE = false, bool BOUND = false, bool ONE = false,
-          bool LONE = false, bool REC = !MIXED && !LONE>
+          bool LONE = false, bool REC = !MIXED && !LONE,
+          int U = LONE || (PHYS && !MIXED && ONE) ? 4 : 2>
 __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
                                              const double *__restrict__ P,
                                              const void *__restrict__ e_,
@@ -567,9 +580,6 @@ __device__ __forceinline__ double jk_lnl_row(const StarDev &st, int64_t r,
     bool bad = false;
     double Sw = 0.0;       // sum w (BOUND only; with ONE it is Stt[0])
     float dmx = 0.0f;      // largest 1 / (1 - e cos E) (BOUND only)
-    // four epochs at a time where every fourth renormalises the product and the
-    // registers allow it (2^24 rows x 16 epochs 936 -> 930 us), else two
-    constexpr int U = LONE || (PHYS && !MIXED && ONE) ? 4 : 2;
 #pragma unroll U
     for (int k = 0; k < N; ++k) {
         const double *__restrict__ ep = st.ep + (size_t)k * (JK_EP_T + LT0);
@@ -2107,10 +2117,7 @@ __device__ __forceinline__ void jk_split_item(const WorkSplit &ws, int64_t q, in
 // epochs, L = 2) 67 -> 27 us, 500 82 -> 37, 2400 155 -> 132; mixed, 3 to 64
 // epochs, L = 3: 40 items 210 -> 28, 600 268 -> 122, 8192 1425 -> 1411.  More
 // parts than that cost more than they level out: 2400 FP64 items in 8 parts
-// 240 us.  A pruned launch takes at most four: an item's survivors are
-// gathered to fill waves, and there are fewer in a smaller part (2^21 rows of
-// 100 epochs, the whole call with its rejection: 345 us whole, 337 in two,
-// 335 in four, 340 in eight).
+// 240 us.  A capped launch splits for the cap.
 // grid < 0: -grid workgroups fill the device; grid > 0: the caller's cap, which
 // is then what items are split for.
 #define JK_ITEM_LAUNCH ((int64_t)1 << 23)   // entries per launch (x 256 threads < 2^32)
@@ -2119,6 +2126,21 @@ static unsigned jk_item_parts(int64_t n_items, int grid)
     unsigned lg = 0;
     while (lg < 3 && (n_items << (lg + 1)) <= 2 * std::abs((int64_t)grid)) ++lg;
     return lg;
+}
+
+// Parts per item of a pruned launch: two or four where that leaves at most a
+// quarter of grid (512 entries).  An item's survivors are gathered to fill
+// waves, and a part has fewer of them: each part ends on waves of a few lanes
+// that walk all the star's epochs.  Against a persistent grid of whole items,
+// live thresholds (the star's maximum - 40), 2048 rows per item, L = 2 to 5, 24 to
+// 150 epochs, FP64, geometric mean (worst), for whole items, two parts, four:
+// 1024 items 1.14 (0.92), 0.97 (0.66), 0.76 (0.47); 512 1.54 (1.18), 1.44
+// (0.93), 1.12 (0.73); 256 1.91, 2.10 (1.49), 1.80 (1.09); 128 1.88, 2.51, 2.62.
+// With no survivors parts only help: 1024 items 1.21, 1.26, 1.25; 512
+// 1.66, 1.87, 1.90.
+static unsigned jk_prune_parts(int64_t n_items, int grid)
+{
+    return std::min(2u, jk_item_parts(n_items, grid / 8));
 }
 
 // The end of the launch that starts at ws.first, and its workgroups (cap: 0 for
@@ -2134,7 +2156,7 @@ static unsigned jk_item_launch(int64_t entries, int cap, WorkSplit &ws)
 // whose rows nearly all land within the settling margin of its maximum, so
 // that mixed values would be re-evaluated anyway), else in mixed precision
 // with its bound.  The branch is uniform over a work item.
-template <int L, bool PHYS>
+template <int L, bool PHYS, int U = 2>
 __device__ __forceinline__ double jk_lnl_row_sel(const StarDev &st, int64_t r,
                                                  const double *__restrict__ P,
                                                  const void *__restrict__ e_,
@@ -2147,8 +2169,8 @@ __device__ __forceinline__ double jk_lnl_row_sel(const StarDev &st, int64_t r,
         *bnd = 0.0f;
         return jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, tab);
     }
-    return jk_lnl_row<L, PHYS, true, false, true, false, false, true>(st, r, P, e_, om_, M0_, s_,
-                                                                      tab, bnd);
+    return jk_lnl_row<L, PHYS, true, false, true, false, false, true, U>(st, r, P, e_, om_, M0_,
+                                                                         s_, tab, bnd);
 }
 
 // Slot `slot` of a star table evaluated in FP64 (exact != 0) or as the launch
@@ -2297,7 +2319,8 @@ hipError_t jk_launch_lnl_batch(const jk_batch *b, int precision, int64_t n_items
 #define JK_PRUNE_LIST 2048   // survivors held in LDS before their evaluation
 
 template <int L, bool PHYS, bool MIXED, bool CAPPED>
-__global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const StarDev *__restrict__ stars,
+__global__ __launch_bounds__(256, JK_PRUNE_WAVES(L, PHYS, MIXED))
+                                                    void k_lnl_prune_batch(const StarDev *__restrict__ stars,
                                                          const StarDev *__restrict__ probes,
                                                          const double2 *__restrict__ prune,
                                                          const jk_work_item *__restrict__ items,
@@ -2311,6 +2334,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const 
                                                          float *__restrict__ bound,
                                                          unsigned long long *__restrict__ n_full)
 {
+    constexpr int U = JK_PRUNE_UNROLL(L, PHYS);   // of the mixed rows
     __shared__ int s_n;
     __shared__ int s_list[JK_PRUNE_LIST];
     __shared__ double2 s_tab[MIXED ? JK_TAB_LDS : JK_TAB_LDS64];
@@ -2331,7 +2355,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const 
                 if constexpr (MIXED) {
                     float b;
                     ll[w.out_offset + j] =
-                        jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
+                        jk_lnl_row_sel<L, PHYS, U>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
                     bound[w.out_offset + j] = b;
                 } else {
                     ll[w.out_offset + j] = jk_lnl_row<L, PHYS, false>(st, r, P, e_, om_, M0_, s_, s_tab);
@@ -2354,7 +2378,8 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const 
                 double v;
                 if constexpr (MIXED) {
                     float b;
-                    v = jk_lnl_row<L, PHYS, true, false, true>(pb, r, P, e_, om_, M0_, s_, s_tab, &b);
+                    v = jk_lnl_row<L, PHYS, true, false, true, false, false, true, U>(
+                        pb, r, P, e_, om_, M0_, s_, s_tab, &b);
                     v += (double)b + pr.y;
                 } else {
                     v = jk_lnl_row<L, PHYS, false>(pb, r, P, e_, om_, M0_, s_, s_tab);
@@ -2382,7 +2407,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_prune_batch(const 
                     if constexpr (MIXED) {
                         float b;
                         ll[w.out_offset + jj] =
-                            jk_lnl_row_sel<L, PHYS>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
+                            jk_lnl_row_sel<L, PHYS, U>(st, r, P, e_, om_, M0_, s_, s_tab, &b);
                         bound[w.out_offset + jj] = b;
                     } else {
                         ll[w.out_offset + jj] =
@@ -2408,7 +2433,7 @@ static void launch_prune_t(const jk_batch *b, const jk_batch *pb, const double2 
                            double *ll, float *bound, unsigned long long *n_full, int block,
                            int grid, hipStream_t stream)
 {
-    WorkSplit ws{0, 0, std::min(2u, jk_item_parts(n_items, grid))};
+    WorkSplit ws{0, 0, jk_prune_parts(n_items, grid)};
     const int64_t entries = n_items << ws.lg_parts;
     const bool capped = grid > 0 && entries > grid;
     for (; ws.first < entries; ws.first = ws.end) {
