@@ -6,7 +6,7 @@
 //                          wave-uniform and read through scalar loads.
 //  k_lnl_split             the same for few rows, a row's epochs over many lanes.
 //  k_lnl_cov               the same for a full covariance, rotated on the matrix
-//                          cores.
+//                          cores; k_lnl_cov_lane for few epochs and many rows.
 //  k_max_partial / final   NaN-propagating max (np.max).
 //  k_reject_words / rows   numpy-PCG64 uniforms generated in registers for the
 //                          rows that can pass, exp(ll - max) > u, one 64-bit
@@ -1091,10 +1091,121 @@ __global__ __launch_bounds__(256) void k_lnl_split(const StarDev st, int64_t n, 
     }
 }
 
+// A full-covariance row's sums over the eigenvalues.  ep: r', sigma^2 (PHYS) or
+// ivar and T, N values each.
+template <int L, bool PHYS>
+struct CovSums {
+    static constexpr int LT = L > 1 ? L - 1 : 1;
+    double Smm = 0.0, Smr = 0.0, Srr = 0.0, prod = 1.0;
+    double Smt[LT] = {}, Str[LT] = {}, Stt[LT * LT] = {};
+    int pexp = 0;
+
+    // eigenvalue i, with rotated design value m
+    __device__ __forceinline__ void add(double m, int i, int N, const double *ep, double s2)
+    {
+        const double rp = ep[i];
+        double w = ep[N + i];
+        if constexpr (PHYS) {
+            const double vk = w + s2;
+            w = jk_rcp2(vk);
+            // renormalised at every factor: any finite variance keeps
+            // its logarithm
+            int ex;
+            prod = frexp(prod * vk, &ex);
+            pexp += ex;
+        }
+        const double wm = w * m;
+        Smm = fma(wm, m, Smm);
+        Smr = fma(wm, rp, Smr);
+        if constexpr (L > 1) {
+#pragma unroll
+            for (int j = 0; j < L - 1; ++j) {
+                const double Tj = ep[(j + 2) * N + i];
+                Smt[j] = fma(wm, Tj, Smt[j]);
+                if constexpr (PHYS) {
+                    const double wT = w * Tj;
+                    Str[j] = fma(wT, rp, Str[j]);
+#pragma unroll
+                    for (int q = 0; q <= j; ++q)
+                        Stt[j * LT + q] = fma(wT, ep[(q + 2) * N + i], Stt[j * LT + q]);
+                }
+            }
+        }
+        if constexpr (PHYS) Srr = fma(w * rp, rp, Srr);
+    }
+
+    // with another part of the row's sums: plus() of the parts of a row's four
+    // lanes, ((0, 1), (2, 3)), gives the bits of sum4()
+    __device__ __forceinline__ void plus(const CovSums &b)
+    {
+        Smm += b.Smm;
+        Smr += b.Smr;
+#pragma unroll
+        for (int j = 0; j < L - 1; ++j) Smt[j] += b.Smt[j];
+        if constexpr (PHYS) {
+            Srr += b.Srr;
+#pragma unroll
+            for (int j = 0; j < L - 1; ++j) {
+                Str[j] += b.Str[j];
+#pragma unroll
+                for (int q = 0; q <= j; ++q) Stt[j * LT + q] += b.Stt[j * LT + q];
+            }
+            prod *= b.prod;
+            pexp += b.pexp;
+        }
+    }
+
+    // over the four lanes of a row (jk_cov_sum)
+    __device__ __forceinline__ void sum4()
+    {
+        Smm = jk_cov_sum(Smm);
+        Smr = jk_cov_sum(Smr);
+#pragma unroll
+        for (int j = 0; j < L - 1; ++j) Smt[j] = jk_cov_sum(Smt[j]);
+        if constexpr (PHYS) {
+            Srr = jk_cov_sum(Srr);
+#pragma unroll
+            for (int j = 0; j < L - 1; ++j) {
+                Str[j] = jk_cov_sum(Str[j]);
+#pragma unroll
+                for (int q = 0; q <= j; ++q) Stt[j * LT + q] = jk_cov_sum(Stt[j * LT + q]);
+            }
+            // mantissas in [1/2, 1): four of them stay far inside the range
+            prod *= __shfl_xor(prod, 16, 64);
+            prod *= __shfl_xor(prod, 32, 64);
+            pexp += __shfl_xor(pexp, 16, 64);
+            pexp += __shfl_xor(pexp, 32, 64);
+        }
+    }
+
+    __device__ __forceinline__ double finish(const StarDev &st, const RowOrbit &o,
+                                             const double2 *__restrict__ tab) const
+    {
+        return jk_row_finish<L, PHYS, false>(st, o.lam0, Smm, Smr, Srr, Smt, Str, Stt, prod, pexp,
+                                             0.0, 0.0f, tab, nullptr);
+    }
+};
+
+// r', sigma^2 (PHYS) or ivar and T per eigenvalue, and dt per epoch, to LDS
+// (256 threads).
+template <int L, bool PHYS>
+__device__ __forceinline__ void jk_cov_stage_ep(const StarDev &st, double *s_ep)
+{
+    const int N = st.n;
+    for (int q = threadIdx.x; q < N * (L + 2); q += 256) {
+        const int v = q / N, i = q - v * N;
+        s_ep[q] = v == 0 ? st.rp[i]
+                         : (v == 1 ? (PHYS ? st.sig2[i] : st.ivar[i])
+                                   : (v == L + 1 ? st.dt[i] : st.T[(size_t)(v - 2) * N + i]));
+    }
+}
+
 // Full-covariance stars, FP64: 16 rows per wave (jk_cov_rotate), the
 // workgroups striding over the rows so that each stages Q and the tables once.
+// For L >= 7 two waves per SIMD are asked for (else 253 VGPRs and more, and one
+// wave: 62689 rows x 8 epochs, L = 8 22.7 -> 15.9 us).
 template <int L, bool PHYS>
-__global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev st, int64_t n,
+__global__ __launch_bounds__(256, L >= 7 ? 2 : JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev st, int64_t n,
                                                  const double *__restrict__ P,
                                                  const void *__restrict__ e_,
                                                  const void *__restrict__ om_,
@@ -1111,12 +1222,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev 
         const int k = q / pitch, i = q - k * pitch;
         s_q[q] = k < N && i < N ? st.Qt[(size_t)i * N + k] : 0.0;
     }
-    for (int q = threadIdx.x; q < N * (L + 2); q += 256) {
-        const int v = q / N, i = q - v * N;
-        s_ep[q] = v == 0 ? st.rp[i]
-                         : (v == 1 ? (PHYS ? st.sig2[i] : st.ivar[i])
-                                   : (v == L + 1 ? st.dt[i] : st.T[(size_t)(v - 2) * N + i]));
-    }
+    jk_cov_stage_ep<L, PHYS>(st, s_ep);
     const double *s_dt = s_ep + (L + 1) * N;
     jk_stage_tab<false>(s_tab);
     const int lane = threadIdx.x & 63, kq = lane >> 4;
@@ -1136,17 +1242,7 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev 
             jk_cov_rotate<true>(st, o, valid, s_tab, s_q, s_dt, acc, bad);
         }
         // moments in the eigenbasis, a quarter of the eigenvalues per lane
-        constexpr int LT = L > 1 ? L - 1 : 1;
-        double Smm = 0.0, Smr = 0.0, Srr = 0.0, prod = 1.0;
-        double Smt[LT], Str[LT], Stt[LT * LT];
-        int pexp = 0;
-#pragma unroll
-        for (int j = 0; j < LT; ++j) {
-            Smt[j] = 0.0;
-            Str[j] = 0.0;
-#pragma unroll
-            for (int q = 0; q < LT; ++q) Stt[j * LT + q] = 0.0;
-        }
+        CovSums<L, PHYS> q;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             if (16 * t >= N) break;
@@ -1154,60 +1250,114 @@ __global__ __launch_bounds__(256, JK_ROW_WAVES(L)) void k_lnl_cov(const StarDev 
             for (int r = 0; r < 4; ++r) {
                 const int ei = 16 * t + 4 * r + kq;
                 if (ei >= N) continue;
-                const double m = acc[t][r], rp = s_ep[ei];
-                double w = s_ep[N + ei];
-                if constexpr (PHYS) {
-                    const double vk = w + o.s2;
-                    w = jk_rcp2(vk);
-                    // renormalised at every factor: any finite variance keeps
-                    // its logarithm
-                    int ex;
-                    prod = frexp(prod * vk, &ex);
-                    pexp += ex;
-                }
-                const double wm = w * m;
-                Smm = fma(wm, m, Smm);
-                Smr = fma(wm, rp, Smr);
-                if constexpr (L > 1) {
-#pragma unroll
-                    for (int j = 0; j < L - 1; ++j) {
-                        const double Tj = s_ep[(j + 2) * N + ei];
-                        Smt[j] = fma(wm, Tj, Smt[j]);
-                        if constexpr (PHYS) {
-                            const double wT = w * Tj;
-                            Str[j] = fma(wT, rp, Str[j]);
-#pragma unroll
-                            for (int q = 0; q <= j; ++q)
-                                Stt[j * LT + q] = fma(wT, s_ep[(q + 2) * N + ei], Stt[j * LT + q]);
-                        }
-                    }
-                }
-                if constexpr (PHYS) Srr = fma(w * rp, rp, Srr);
+                q.add(acc[t][r], ei, N, s_ep, o.s2);
             }
         }
-        Smm = jk_cov_sum(Smm);
-        Smr = jk_cov_sum(Smr);
-#pragma unroll
-        for (int j = 0; j < L - 1; ++j) Smt[j] = jk_cov_sum(Smt[j]);
-        if constexpr (PHYS) {
-            Srr = jk_cov_sum(Srr);
-#pragma unroll
-            for (int j = 0; j < L - 1; ++j) {
-                Str[j] = jk_cov_sum(Str[j]);
-#pragma unroll
-                for (int q = 0; q <= j; ++q) Stt[j * LT + q] = jk_cov_sum(Stt[j * LT + q]);
-            }
-            // mantissas in [1/2, 1): four of them stay far inside the range
-            prod *= __shfl_xor(prod, 16, 64);
-            prod *= __shfl_xor(prod, 32, 64);
-            pexp += __shfl_xor(pexp, 16, 64);
-            pexp += __shfl_xor(pexp, 32, 64);
-        }
-        if (kq == 0 && i < n)
-            ll[i] = valid ? jk_row_finish<L, PHYS, false>(st, o.lam0, Smm, Smr, Srr, Smt, Str, Stt,
-                                                          prod, pexp, 0.0, 0.0f, s_tab, nullptr)
-                          : __builtin_nan("");
+        q.sum4();
+        if (kq == 0 && i < n) ll[i] = valid ? q.finish(st, o, s_tab) : __builtin_nan("");
     }
+}
+
+// The rotated design values of one lane's row of N <= NL epochs, eigenvalue i
+// in acc[i].  SAFE: with the bracketed Newton iteration; else returns whether
+// the row needs it.
+template <int NL, bool SAFE>
+__device__ __forceinline__ bool jk_cov_rotate_lane(const StarDev &st, const RowOrbit &o,
+                                                   const double2 *__restrict__ tab,
+                                                   const double *s_q, const double *s_dt,
+                                                   double acc[NL])
+{
+    const int N = st.n;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < NL; ++i) acc[i] = 0.0;
+    for (int k = 0; k < N; ++k) {
+        double w;
+        float denb;
+        const double m = jk_row_epoch<false, false, SAFE, true>(o, s_dt[k], 0.0, tab, w, denb, bad);
+        const double *q = s_q + k * NL;
+#pragma unroll
+        for (int i0 = 0; i0 < NL; i0 += 8) {
+            if (i0 >= N) break;
+#pragma unroll
+            for (int i = i0; i < i0 + 8; ++i) acc[i] = fma(q[i], m, acc[i]);
+        }
+    }
+    return bad;
+}
+
+// Full-covariance stars of few epochs, N <= NL (jk_cov_lane), one lane per row:
+// the rotation is N multiply-adds per epoch, its operands read by all lanes
+// alike from LDS, in the order in which the matrix cores add (each rounded like
+// an fma), and the sums go by the parts that the tile form's lanes hold.  A row's
+// lnL is the same bits in either form.  Bound by the latency of one row's
+// chain of solves up to a wave per SIMD (65536 rows), then by the vector units,
+// with jitter and L >= 5 at one wave per SIMD for the parts' registers (two
+// waves asked for spill them: 131072 x 8, L = 6 18 -> 22 us).
+template <int L, bool PHYS, int NL>
+__global__ __launch_bounds__(256) void k_lnl_cov_lane(const StarDev st, int64_t n,
+                                                      const double *__restrict__ P,
+                                                      const void *__restrict__ e_,
+                                                      const void *__restrict__ om_,
+                                                      const void *__restrict__ M0_,
+                                                      const void *__restrict__ s_,
+                                                      const int64_t *__restrict__ rows,
+                                                      double *__restrict__ ll)
+{
+    __shared__ double2 s_tab[JK_TAB_LDS64];
+    __shared__ double s_q[NL * NL];    // epoch-major, zero-padded
+    __shared__ double s_ep[NL * (L + 2)];
+    const int N = st.n;
+    for (int q = threadIdx.x; q < N * NL; q += 256) {
+        const int k = q / NL, i = q % NL;
+        s_q[q] = i < N ? st.Qt[(size_t)i * N + k] : 0.0;
+    }
+    jk_cov_stage_ep<L, PHYS>(st, s_ep);
+    const double *s_dt = s_ep + (L + 1) * N;
+    jk_stage_tab<false>(s_tab);
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        RowOrbit o;
+        if (!jk_row_orbit<PHYS>(st, rows ? rows[i] : i, P, e_, om_, M0_, s_, s_tab, o)) {
+            ll[i] = __builtin_nan("");
+            continue;
+        }
+        double acc[NL];
+        if (jk_cov_rotate_lane<NL, false>(st, o, s_tab, s_q, s_dt, acc))
+            jk_cov_rotate_lane<NL, true>(st, o, s_tab, s_q, s_dt, acc);
+        CovSums<L, PHYS> half, sum;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            CovSums<L, PHYS> q;
+#pragma unroll
+            for (int j = g; j < NL; j += 4)
+                if (j < N) q.add(acc[j], j, N, s_ep, o.s2);
+            if (g & 1)
+                half.plus(q);
+            else
+                half = q;
+            if (g == 1) sum = half;
+            if (g == 3) sum.plus(half);
+        }
+        ll[i] = sum.finish(st, o, s_tab);
+    }
+}
+
+// Whether a launch takes one lane per row.  The tile form pays the orbit on
+// four lanes per row and the finish on one lane of four, which few epochs do
+// not outweigh once its waves (a row to every 4 lanes) fill the device, the
+// sooner the larger L.  us, tile form -> this: 62689 rows, 4 epochs, L = 2 7.6 ->
+// 6.6, L = 4 11.7 -> 6.8, L = 6 15.4 -> 7.9; 16 epochs, L = 4 15.4 -> 12.5, L = 6 19.9
+// -> 15.5; 131072 rows, 16 epochs, L = 2 15.8 -> 14.3, L = 6 32.4 -> 28.5.
+// Below the lines the tile form is ahead: 16384 rows, 16 epochs, L = 2 6.9 ->
+// 11.0; 32768, 12 epochs, L = 5 8.6 -> 10.4; 62689, 16 epochs, L = 2 10.2 -> 11.7.  Up
+// to 24 epochs for L >= 6 alone (131072 x 20 at L = 6 38.4 -> 35.0, L = 8 without
+// jitter 52.0 -> 21.5): there the tile form's registers leave one or two waves
+// per SIMD.
+static bool jk_cov_lane(int64_t n, int N, int L)
+{
+    if (N <= 8) return n > (L <= 3 ? 49152 : (L <= 5 ? 36864 : 16384));
+    if (N <= 16) return n > (L <= 3 ? 65536 : (L <= 5 ? 53248 : 32768));
+    return N <= 24 && L >= 6 && n > 53248;
 }
 
 template <int L, bool PHYS>
@@ -1215,6 +1365,15 @@ static hipError_t launch_lnl_cov_t(const jk_star *st, int64_t n, const double *P
                                    const void *om, const void *M0, const void *s,
                                    const int64_t *rows, double *ll, hipStream_t stream)
 {
+    if (jk_cov_lane(n, st->dev.n, L)) {
+        const int64_t blocks = std::min<int64_t>((n + 255) / 256, 1024);
+        auto kernel = k_lnl_cov_lane<L, PHYS, 16>;
+        if constexpr (L >= 6)
+            if (st->dev.n > 16) kernel = k_lnl_cov_lane<L, PHYS, 24>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, stream, st->dev, n, P, e,
+                           om, M0, s, rows, ll);
+        return hipGetLastError();
+    }
     // four workgroups per compute unit, then a stride: staging Q and the tables
     // costs as much as a few rows (2^18 rows x 40: 78 us with 4096 workgroups,
     // 75 with 1024; 100000 x 64: 75 and 66)
